@@ -441,7 +441,9 @@ int mdffgpu_profile_only(mdffgpu_ctx* ctx, int32_t kernel);
  * the Python autotuner): K slices of the field apply (1, 2 or 4) and atoms
  * per structure-factor split of the sums with charges (a multiple of 128;
  * the dipole-only sums of the SCF and final calls size their splits to fill
- * the device in one round).  MDFFGPU_ERR_UNSUPPORTED on an FP64 context.
+ * the device in one round).  The grid sums, which every context takes whose
+ * kmax they support, have no such shape: there the arguments are checked
+ * only.  MDFFGPU_ERR_UNSUPPORTED on an FP64 context.
  * No counterpart in the reference. */
 int mdffgpu_set_mixed_tuning(mdffgpu_ctx* ctx, int32_t apply_slices, int32_t split_atoms);
 int mdffgpu_profile_read(const mdffgpu_ctx* ctx, int32_t kernel,

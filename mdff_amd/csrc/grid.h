@@ -1,0 +1,69 @@
+// grid.h -- reciprocal-space Ewald sums through a uniform grid: the sums over
+// every k vector of the half-space mesh, evaluated as a non-uniform Fourier
+// transform (spread the moments onto a grid, transform, multiply by the
+// Ewald factors, transform back, interpolate) instead of one term per
+// (atom, k).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <vector>
+
+#include "common.h"
+
+struct mdffgpu_ctx;
+
+namespace mdff {
+namespace grid {
+
+// One configuration: its cell and Ewald alpha and its atoms in the caller's
+// arrays.
+struct Seg {
+  Cell cell;
+  double alpha;
+  int off, n;
+};
+
+struct Plan;
+
+// Whether a plan exists for these kmax (grid extents within the kernels'
+// limits).
+bool supported(const int kmax[3]);
+
+// Plan for configurations that share kmax; fp64: grid and kernel tables in
+// double (support 16), else in float (support 10; transforms in double).
+// Null when device memory runs out.
+Plan* create(hipStream_t st, const std::vector<Seg>& segs, const int kmax[3], bool fp64);
+void destroy(Plan* p);
+
+// New cells (and alpha) of the configurations; the binning has to be redone.
+void set_cells(Plan* p, hipStream_t st, const std::vector<Seg>& segs);
+
+// Bins of the current positions (fractional coordinates s4, one per atom).
+// Atoms of a species with its bit in `active` come first in their own bins:
+// the calls over the active atoms alone read those.  Until the next call no
+// atom may move by more than drift (a length).  Waits for the stream; false
+// when device memory runs out.
+bool bin(Plan* p, hipStream_t st, const double4* s4, const int* typ, const int* cfg,
+         unsigned active, double drift);
+bool binned(const Plan* p);
+void unbin(Plan* p);
+
+// Kernel values and tile lists at the current positions: once per
+// evaluation.  ctx (here and below) brackets the launches for its
+// instrumentation, or null.
+void prepare(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double4* s4);
+
+// The reciprocal sums of one Ewald call with charges q (chg) and dipoles mu
+// (dip; SoA of stride n): U_a = sum_k A_k n_a Im(S conj e^{ikr}) and, with
+// second, V_ab = sum_k A_k n_a n_b Re(..) over the half-space mesh into
+// out[row * n + atom], rows U1 U2 U3 V11 V22 V33 V12 V13 V23.  src_active:
+// only the active atoms carry moments; dst_active: rows of the active atoms
+// only.  With pout (one configuration), block partials of the energy and
+// stress sums go to pout[row * nblocks + block] (7 rows); returns nblocks.
+int sums(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double4* s4, const double* q,
+         const double* mu, bool chg, bool dip,
+         bool second, bool src_active, bool dst_active, double* out, double* pout);
+
+}  // namespace grid
+}  // namespace mdff

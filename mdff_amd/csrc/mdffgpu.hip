@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/mdffgpu.h"
+#include "grid.h"
 #include "kernels.h"
 #include "mixed.h"
 #include "tables.h"
@@ -184,6 +185,9 @@ struct mdffgpu_ctx {
   hipStream_t st = nullptr;
   int linduced = 0, ldip_static = 0;
   mixed::MixedState* mx = nullptr;
+  // reciprocal space through the uniform grid (grid.hip), or null: the
+  // direct sums
+  grid::Plan* gp = nullptr;
   // kernel instrumentation: HIP events around each launch of the own stream
   int prof = 0;
   long long evals = 0;  // engforce evaluations run (positions may change between)
@@ -202,7 +206,8 @@ const char* const kKernelNames[K_COUNT] = {
     "k_scf_resid", "k_extrap", "k_reduce_rows", "k_add", "k_pairs_t2", "k_dd_field",
     "mx_shortrange", "mx_es_dir",
     "mx_phase", "mx_rho", "mx_rho_reduce", "mx_apply", "mx_combine", "mx_weights", "mx_gprep",
-    "batch", "adjoint", "k_efg_es_dir", "k_efg_ds", "k_efg_combine", "md", "k_es_quad", "k_wfc"};
+    "batch", "adjoint", "k_efg_es_dir", "k_efg_ds", "k_efg_combine", "md", "k_es_quad", "k_wfc",
+    "grid_prepare", "grid_spread", "grid_transform", "grid_gather"};
 
 ProfScope::ProfScope(mdffgpu_ctx* ctx, int kid) : c(ctx), id(kid), a(nullptr), b(nullptr) {
   if (!c || !c->prof || (c->prof_only != -1 && c->prof_only != kid)) return;
@@ -397,6 +402,32 @@ void build_kmesh(mdffgpu_ctx* c) {
   dalloc(c, &c->d_apart, (size_t)c->app_split * 9 * n);
   // rows a partial call leaves alone hold finite values
   HCK(c, hipMemsetAsync(c->d_apart, 0, (size_t)c->app_split * 9 * n * sizeof(double), c->st));
+}
+
+// Grid plan of the reciprocal sums in the precision they run in.
+bool grid_fp64(const mdffgpu_ctx* c) {
+  return c->P.precision != MDFFGPU_PREC_MIXED ||
+         (c->P.mixed_fp64_parts & MDFFGPU_MIXED_FP64_KSPACE) != 0;
+}
+
+std::vector<grid::Seg> grid_segs(const mdffgpu_ctx* c) {
+  grid::Seg s;
+  s.cell = c->cell;
+  s.alpha = c->P.alphaES;
+  s.off = 0;
+  s.n = c->n;
+  return {s};
+}
+
+// Whether the reciprocal sums go through the grid.  The direct sums stay
+// where there are quadrupoles (their second-order terms are not spread), in
+// the allocation-free context (its scratch is fixed) and for kmax beyond the
+// plan's extents.  There is no lower limit of size: whole evaluations with 45
+// atoms at kmax 5 take 1.12 ms with either in FP64 (launches and
+// synchronisations; 20 SCF iterations) and 0.61 against 0.67 ms in mixed
+// precision, 300 atoms at kmax 10 1.21 against 3.00 and 0.69 against 0.89 ms.
+bool grid_rule(const mdffgpu_ctx* c) {
+  return c->P.lcoulomb && c->nchunk > 0 && !c->noalloc && !c->lquad && grid::supported(c->kmax);
 }
 
 void build_tables(mdffgpu_ctx* c) {
@@ -810,7 +841,16 @@ void es_call(mdffgpu_ctx* c, int mode, const double* q, const double* mu, int ta
   // does the combine (no surface term)
   int fused_parts = 0;
   c->cg_npap = gb;
-  if (mxk && c->nchunk > 0) {
+  if (c->gp) {
+    // the induced dipoles sit on the active (polarizable) atoms, where alone
+    // the static and SCF calls' field is read
+    const int nb = grid::sums(c->gp, c, st, c->d_s4, q, mu, chg, dip, efgv, mode == ES_IND,
+                              mode != ES_FINAL, c->d_apart,
+                              mode == ES_FINAL ? c->d_part : nullptr);
+    check_launch(c, "grid sums");
+    if (mode == ES_FINAL) reduce(c, 7, nb, SC_REC);
+    nsplit_apply = 1;
+  } else if (mxk && c->nchunk > 0) {
     const bool fuse = (mode == ES_IND) && c->cg_Ap && !P.lsurf;
     fused_parts = mixed::kspace(c->mx, mode, q, mu, chg, dip, efgv, c->d_apart, wt_ready,
                                 fuse ? &ca : nullptr);
@@ -1137,7 +1177,7 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
     g.p4 = pk ? reinterpret_cast<float4*>(c->d_mu4) : nullptr;
     // with the mixed reciprocal space, k_cg_dir also writes the FP32
     // structure-factor weights of the direction
-    if (mixed_prec && !(P.mixed_fp64_parts & MDFFGPU_MIXED_FP64_KSPACE) && c->mx &&
+    if (mixed_prec && !(P.mixed_fp64_parts & MDFFGPU_MIXED_FP64_KSPACE) && c->mx && !c->gp &&
         c->nchunk > 0) {
       g.wt = mixed::dipole_weights(c->mx, &g.wt_npad);
       g.wscale = mixed::DIP_WEIGHT_SCALE;
@@ -1573,6 +1613,14 @@ void update_floor(mdffgpu_ctx* c) {
     c->mx_floor = std::min(c->mx_floor, c->scf_best);
 }
 
+// Bins of the grid at the current positions, good for displacements up to
+// drift.
+void grid_bin(mdffgpu_ctx* c, double drift) {
+  if (!grid::bin(c->gp, c->st, c->d_s4, c->d_typ, nullptr, c->polmask, drift))
+    fail(c, MDFFGPU_ERR_ALLOC, "bins of the reciprocal-space grid");
+  check_launch(c, "grid bins");
+}
+
 // engforce_driver on the device buffers of ctx; d_pos and d_force are
 // loaded by the caller.
 // Verlet list of the current positions: rebuilt when invalid or when the
@@ -1582,7 +1630,7 @@ void update_list(mdffgpu_ctx* c) {
   const int n = c->n;
   const int gb = nblk(n);
   hipStream_t st = c->st;
-  bool rebuild = !c->list_valid;
+  bool rebuild = !c->list_valid || (c->gp && !grid::binned(c->gp));
   if (c->list_cut > 0.0 && !rebuild) {
     // Verlet skin (vnlistcheck, src/tools.f90:446-535): the list holds every
     // pair within cutoff + skin at the last build, so it stays complete
@@ -1652,6 +1700,9 @@ void update_list(mdffgpu_ctx* c) {
       if (*c->h_ovf <= c->maxnb) break;
       set_list_capacity(c, (int)(*c->h_ovf * 1.2) + 16);
     }
+    // the grid's bins follow the list: no atom moves by more than skin/2
+    // while it is valid
+    if (c->gp) grid_bin(c, 0.5 * P.skindiff);
   }
 }
 
@@ -1669,6 +1720,7 @@ void run(mdffgpu_ctx* c, int itime, mdffgpu_energies* en) {
   }
   check_launch(c, "k_prepare");
   update_list(c);
+  if (c->gp) grid::prepare(c->gp, c, st, c->d_s4);
   if (P.lcoulomb && c->linduced) build_t2(c);
   const bool sr = P.lnmlj || P.lbmhft || P.lbmhftd || P.lmorse;
   const bool mxs = (P.precision == MDFFGPU_PREC_MIXED) &&
@@ -1881,6 +1933,7 @@ void efg_frame(mdffgpu_ctx* c, const mdffgpu_efg_opts& o, mdffgpu_energies* en) 
     c->P.calc_mode = 0;
     try {
       update_list(c);
+      if (c->gp) grid::prepare(c->gp, c, st, c->d_s4);
       build_t2(c);
       int n_es = 0;
       scf(c, 0, &en->n_scf, &en->rmsd, &n_es, &en->scf_tol);
@@ -1953,7 +2006,18 @@ void efg_frame(mdffgpu_ctx* c, const mdffgpu_efg_opts& o, mdffgpu_energies* en) 
     ca.ndir = js;
     // reciprocal space: charge_density_k (src/efg.f90:2888-2930) and the
     // EFG of every k (:1507-1556), on the FP64 structure-factor kernels
-    if (c->nchunk > 0) {
+    if (c->gp && grid_fp64(c)) {
+      if (!c->linduced) {
+        // no list of this frame: bins of its positions alone
+        grid_bin(c, 0.0);
+        grid::prepare(c->gp, c, st, c->d_s4);
+        grid::unbin(c->gp);
+      }
+      grid::sums(c->gp, c, st, c->d_s4, q, mu, true, dip, true, false, false, c->d_apart, nullptr);
+      check_launch(c, "grid sums");
+      ca.rec = c->d_apart;
+      ca.nrec = 1;
+    } else if (c->nchunk > 0) {
       RhoArgs ra;
       ra.n = n;
       ra.nchunk = c->nchunk;
@@ -2146,7 +2210,11 @@ void create_impl(const mdffgpu_params* params, const int32_t* itype, const doubl
     if (c->P.lcoulomb) build_kmesh(c);
     size_t need = 12 * (size_t)std::max(nblk(c->kpad), nblk(c->n * LPA)) + 4096;
     ensure_part(c, need);
-    if (c->P.precision == MDFFGPU_PREC_MIXED) {
+    if (grid_rule(c)) {
+      c->gp = grid::create(c->st, grid_segs(c), c->kmax, grid_fp64(c));
+      if (!c->gp) fail(c, MDFFGPU_ERR_ALLOC, "reciprocal-space grid");
+    }
+    if (c->P.precision == MDFFGPU_PREC_MIXED && !c->gp) {
       c->mx = mixed::create(c);
       if (!c->mx) fail(c, MDFFGPU_ERR_UNSUPPORTED, "mixed-precision path unavailable");
       mx_active(c);
@@ -2410,6 +2478,7 @@ void mdffgpu_destroy(mdffgpu_ctx* c) {
     return;
   }
   if (c->mx) mixed::destroy(c->mx);
+  grid::destroy(c->gp);
   double* dp[] = {c->d_rref, c->d_pos, c->d_s, c->d_q, c->d_qzero, c->d_dip, c->d_mu, c->d_muind,
                   c->d_mup, c->d_Estat, c->d_E, c->d_efdir, c->d_efgdir, c->d_fdir,
                   c->d_force, c->d_ef, c->d_efg, c->d_apart, c->d_Ak, c->d_kcoe, c->d_kvec,
@@ -2447,6 +2516,11 @@ int mdffgpu_set_cell(mdffgpu_ctx* c, const double* A) {
     if (c->list_cut > 0.0) set_list_capacity(c, std::max(c->maxnb, initial_capacity(c)));
     if (c->P.lcoulomb) build_kmesh(c);
     if (c->mx) mixed::on_cell(c->mx);
+    if (c->gp) {
+      grid::set_cells(c->gp, c->st, grid_segs(c));
+      // a later call may run on the caller's stream
+      HCK(c, hipStreamSynchronize(c->st));
+    }
     return MDFFGPU_OK;
   } catch (Fail& f) {
     return f.code;
@@ -2957,7 +3031,9 @@ const char* mdffgpu_last_error(const mdffgpu_ctx* c) {
 
 int mdffgpu_set_mixed_tuning(mdffgpu_ctx* c, int32_t apply_slices, int32_t split_atoms) {
   if (!c) return MDFFGPU_ERR_ARG;
-  if (!c->mx) return MDFFGPU_ERR_UNSUPPORTED;
+  if (c->P.precision != MDFFGPU_PREC_MIXED) return MDFFGPU_ERR_UNSUPPORTED;
+  // the grid sums have no such launch shape
+  if (!c->mx) return mixed::valid_tuning(apply_slices, split_atoms) ? MDFFGPU_OK : MDFFGPU_ERR_ARG;
   if (hipStreamSynchronize(c->st) != hipSuccess) return MDFFGPU_ERR_DEVICE;
   return mixed::set_tuning(c->mx, apply_slices, split_atoms) ? MDFFGPU_OK : MDFFGPU_ERR_ARG;
 }

@@ -92,6 +92,7 @@ float* dipole_weights(MixedState* m, int* npad);
 MixedState* create_batch(int N, const int kmax[3], const std::vector<MxSeg>& segs);
 // Launch shape: K slices of the apply GEMM (1, 2 or 4) and atoms per
 // structure-factor split (a multiple of 128); false if rejected.
+bool valid_tuning(int app_slices, int split_atoms);
 bool set_tuning(MixedState* m, int app_slices, int split_atoms);
 // Reciprocal-space field (and, with force, force) of every atom of the
 // batch for sources (q, mu): Erec = -2 (4 pi/V) sum_k k t_k,

@@ -1754,9 +1754,13 @@ MixedState* create_batch(int N, const int kmax[3], const std::vector<MxSeg>& seg
   return m;
 }
 
+bool valid_tuning(int app_slices, int split_atoms) {
+  return (app_slices == 1 || app_slices == 2 || app_slices == 4) && split_atoms >= 128 &&
+         split_atoms % 128 == 0;
+}
+
 bool set_tuning(MixedState* m, int app_slices, int split_atoms) {
-  if (app_slices != 1 && app_slices != 2 && app_slices != 4) return false;
-  if (split_atoms < 128 || split_atoms % 128 != 0) return false;
+  if (!valid_tuning(app_slices, split_atoms)) return false;
   if (app_slices > m->x_slices) {
     m->x_slices = app_slices;
     m->X_cap = (size_t)m->x_slices * m->npad * APP_NCT_E * 16;

@@ -1,0 +1,74 @@
+"""Reciprocal sums through the uniform grid (grid.hip) against the oracle,
+which sums every k vector: kmax from 1 (a grid of one tile, as wide as the
+kernel) over odd and unequal values to a padded last tile, atoms on the cell
+faces and outside the cell, a cluster (every atom in a few bins), and atoms
+moved within the list's skin since their bins were made.
+
+Tolerances: the FP64 bar of the parity tests (1e-10 of the largest value);
+in mixed precision 4e-6 of the RMS, about eight times the FP32 error of the
+whole evaluation.
+"""
+import copy
+
+import numpy as np
+import pytest
+
+from helpers import compare_engforce
+from test_gpu_geometry import skewed_silica
+
+from mdff_amd import configs as C
+from mdff_amd import params as P
+
+pytestmark = pytest.mark.gpu
+
+KMAX = [(1, 1, 1), (2, 5, 1), (7, 3, 12), (17, 4, 9), (4, 16, 15)]
+
+
+def _edge_positions(s):
+    """The melt with atoms on the faces, just inside and outside the cell."""
+    r = s.r.copy()
+    frac = r @ np.linalg.inv(s.A).T
+    frac -= (frac[0, 0], frac[1, 1], frac[2, 2])
+    frac[1, 1] = 1.0
+    frac[2, 2] = -1e-17
+    frac[4] += (1.0, -2.0, 3.0)
+    return frac @ s.A.T
+
+
+@pytest.mark.parametrize("kmax", KMAX)
+@pytest.mark.parametrize("precision", [P.PREC_FP64, P.PREC_MIXED])
+def test_grid_sums_match_oracle(oracle_lib, kmax, precision):
+    from mdff_amd.field import ForceField
+    s = skewed_silica(24, 48, seed=5, kmax=kmax, rc=4.5)
+    r = _edge_positions(s)
+    p = copy.deepcopy(s.params)
+    p.precision = precision
+    print(f"kmax {kmax} precision {precision}", flush=True)
+    ff = ForceField(p, s.itype, s.A)
+    orc = oracle_lib.Oracle(s.params, s.itype, s.A)
+    step = 0.05 * np.random.default_rng(1).uniform(-1, 1, r.shape)
+    for k in range(3):
+        # the second and third frame stay within the skin of the first
+        g = ff.engforce(r + k * step, itime=k + 1)
+        o = orc.engforce(r + k * step, itime=k + 1)
+        if precision == P.PREC_FP64:
+            compare_engforce(g, o)
+            continue
+        for key in ("f", "mu", "ef", "efg"):
+            err = np.linalg.norm(g[key] - o[key]) / np.linalg.norm(o[key])
+            assert err < 4e-6, (key, err)
+    assert ff.list_info()["builds"] == 1
+    ff.close()
+
+
+def test_grid_clustered_atoms(oracle_lib):
+    """All atoms in one corner of a large cell: a few bins hold everything."""
+    from mdff_amd.field import ForceField
+    s = C.silica(20, 40, seed=8, rc=4.0, kmax=9, pim=False, efg=True)
+    A = 4.0 * s.A
+    p = copy.deepcopy(s.params)
+    p.cutlongrange = p.cutshortrange = 4.0
+    ff = ForceField(p, s.itype, A)
+    g = ff.engforce(s.r, itime=1)
+    ff.close()
+    compare_engforce(g, oracle_lib.Oracle(p, s.itype, A).engforce(s.r, itime=1))
