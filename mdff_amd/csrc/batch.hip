@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "../../include/mdffgpu.h"
+#include "grid.h"
 #include "kernels.h"
 #include "mixed.h"
 #include "rtypes.h"
@@ -320,6 +321,41 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_b_combine(
 }
 
 // ---------------------------------------------------------------------------
+// Reciprocal field and force of atom i from its U, V sums (grid.h) with its
+// configuration's lattice:
+//   Erec = -2 (4 pi/V) (2 pi) B U,
+//   Frec = q Erec + 2 (4 pi/V) (2 pi)^2 B V B^T mu.
+__global__ __launch_bounds__(MDFF_BLOCK) void k_b_grid_fields(
+    int N, const int* __restrict__ cfg, const BatchCfg* __restrict__ bc,
+    const double* __restrict__ ap, const double* __restrict__ q, const double* __restrict__ mu,
+    int force, double* __restrict__ Erec, double* __restrict__ Frec) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= N) return;
+  const BatchCfg& b = bc[cfg[i]];
+  const double* B = b.cell.B;
+  const double tpi = 2.0 * MDFF_PI;
+  const double fe = -2.0 * b.fpi_V * tpi;
+  const size_t n = N;
+  const double U[3] = {ap[i], ap[i + n], ap[i + 2 * n]};
+  double er[3];
+  for (int r = 0; r < 3; ++r) {
+    er[r] = fe * (B[r] * U[0] + B[r + 3] * U[1] + B[r + 6] * U[2]);
+    Erec[i + r * n] = er[r];
+  }
+  if (!force) return;
+  double V[6];
+  for (int c = 0; c < 6; ++c) V[c] = ap[i + (3 + c) * n];
+  const double Vm[3][3] = {{V[0], V[3], V[4]}, {V[3], V[1], V[5]}, {V[4], V[5], V[2]}};
+  const double fg = 2.0 * b.fpi_V * tpi * tpi;
+  // B^T mu first, then V, then B
+  double m[3], w[3];
+  for (int y = 0; y < 3; ++y)
+    m[y] = B[3 * y] * mu[i] + B[3 * y + 1] * mu[i + n] + B[3 * y + 2] * mu[i + 2 * n];
+  for (int x = 0; x < 3; ++x) w[x] = Vm[x][0] * m[0] + Vm[x][1] * m[1] + Vm[x][2] * m[2];
+  for (int r = 0; r < 3; ++r)
+    Frec[i + r * n] = q[i] * er[r] + fg * (B[r] * w[0] + B[r + 3] * w[1] + B[r + 6] * w[2]);
+}
+
 // small vector kernels (graph-safe replacements of memset / memcpy)
 __global__ __launch_bounds__(MDFF_BLOCK) void k_b_fill(size_t n, double v, double* __restrict__ x) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -655,6 +691,10 @@ struct mdffgpu_batch {
   // common kmax); positions' version for its phase tables
   mdff::mixed::MixedState* mx = nullptr;
   bool mx_tried = false;
+  // reciprocal sums through the uniform grid (configurations with a common
+  // kmax), its U, V sums per atom
+  mdff::grid::Plan* gp = nullptr;
+  double* d_apart = nullptr;
   long long epoch = 0;
   int pol_type[MDFF_NT];
   double pol_alpha[MDFF_NT];
@@ -863,6 +903,39 @@ mdff::mixed::MixedState* mx_state(mdffgpu_batch* b) {
   return b->mx;
 }
 
+bool common_kmax(const mdffgpu_batch* b) {
+  for (const BatchCfg& x : b->bc_h)
+    for (int a = 0; a < 3; ++a)
+      if (x.kmax[a] != b->bc_h[0].kmax[a]) return false;
+  return true;
+}
+
+// Grid plan of an FP64 batch whose configurations share kmax, binned at the
+// current positions (set_positions: never inside a graph capture).  Loss and
+// gradient, per-k kernels against the grid: 12 configurations (5,400 atoms,
+// kmax 8) 51.2 -> 10.4 ms, 64 (58,000 atoms) 119 -> 55 ms, 2 (400 atoms, kmax
+// 5) 13.4 -> 4.8 ms.
+void grid_state(mdffgpu_batch* b) {
+  if (!b->P.lcoulomb || b->mixed || !common_kmax(b)) return;
+  if (!b->gp) {
+    std::vector<grid::Seg> segs(b->bc_h.size());
+    for (size_t c = 0; c < segs.size(); ++c) {
+      segs[c].cell = b->bc_h[c].cell;
+      segs[c].alpha = b->bc_h[c].alpha;
+      segs[c].off = b->bc_h[c].off;
+      segs[c].n = b->bc_h[c].n;
+    }
+    b->gp = grid::create(b->st, segs, b->bc_h[0].kmax, !b->mixed);
+    if (!b->gp) bfail(b, MDFFGPU_ERR_ALLOC, "reciprocal-space grid");
+    balloc(b, &b->d_apart, 9 * (size_t)b->N);
+    BCK(b, hipMemsetAsync(b->d_apart, 0, 9 * (size_t)b->N * sizeof(double), b->st));
+  }
+  if (!grid::bin(b->gp, b->st, b->d_s4, b->d_typ, b->d_cfg, b->polmask, 0.0))
+    bfail(b, MDFFGPU_ERR_ALLOC, "bins of the reciprocal-space grid");
+  grid::prepare(b->gp, nullptr, b->st, b->d_s4);
+  launch_check(b, "batch grid bins");
+}
+
 // One multipole_ES call over the batch with sources (q, mu):
 //   STATIC  out = static field (charges only)
 //   IND     out = S + dipole field of mu (the SCF field operator)
@@ -919,7 +992,14 @@ void es_call(mdffgpu_batch* b, int mode, const double* q, const double* mu, cons
   launch_check(b, "batch real space");
   const int chg = (mode != ES_IND) ? 1 : 0;
   const int dip = (mode != ES_STATIC && b->pim) ? 1 : 0;
-  if (sizeof(R) == sizeof(float) && mx_state(b)) {
+  if (b->gp) {
+    // the induced dipoles sit on the polarizable atoms, where alone the
+    // static and SCF calls' field is read
+    grid::sums(b->gp, nullptr, b->st, b->d_s4, q, mu, chg, dip, mode == ES_FINAL, mode == ES_IND,
+               mode != ES_FINAL, b->d_apart, nullptr);
+    k_b_grid_fields<<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, b->d_cfg, b->d_bc, b->d_apart, q, mu,
+                                                       mode == ES_FINAL, b->d_rec, b->d_frec);
+  } else if (sizeof(R) == sizeof(float) && mx_state(b)) {
     mdff::mixed::kspace_batch(b->mx, b->st, b->d_s, b->epoch, b->d_cfg, q, mu, chg, dip,
                               mode == ES_FINAL, b->d_rec, b->d_frec);
   } else {
@@ -1421,7 +1501,8 @@ void set_positions_impl(mdffgpu_batch* b, const double* d_pos) {
   }
   b->positions_set = true;
   ++b->epoch;
-  if (b->mixed) mx_state(b);  // allocates: never first inside a graph capture
+  grid_state(b);
+  if (b->mixed && !b->gp) mx_state(b);  // allocates: never first inside a graph capture
   if (b->gexec) {
     (void)hipGraphExecDestroy(b->gexec);
     b->gexec = nullptr;
@@ -1481,6 +1562,7 @@ void mdffgpu_batch_destroy(mdffgpu_batch* b) {
   if (!b) return;
   if (b->st) (void)hipStreamSynchronize(b->st);
   if (b->mx) mdff::mixed::destroy(b->mx);
+  mdff::grid::destroy(b->gp);
   if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
   for (void* p : b->allocs) (void)hipFree(p);
   if (b->h_out) (void)hipHostFree(b->h_out);

@@ -72,3 +72,26 @@ def test_grid_clustered_atoms(oracle_lib):
     g = ff.engforce(s.r, itime=1)
     ff.close()
     compare_engforce(g, oracle_lib.Oracle(p, s.itype, A).engforce(s.r, itime=1))
+
+
+def test_grid_batch_matches_oracle(oracle_lib):
+    """FP64 batch with a common, unequal-axes kmax (one plan over uneven
+    configurations) against the oracle, configuration by configuration, and
+    with different kmax (the per-k kernels)."""
+    import torch
+    from mdff_amd.batch import Batch
+    systems = [C.silica(n, 2 * n, seed=30 + n, rc=4.5, kmax=4, pim=True, scf_tol=1e-12,
+                        pot_seed=3) for n in (16, 21, 40)]
+    for kmaxes in ([(3, 5, 4)] * 3, [(3, 5, 4), (4, 4, 4), (3, 5, 4)]):
+        for s, k in zip(systems, kmaxes):
+            s.params.kES[:] = list(k)
+        b = Batch.from_systems(systems, precision=P.PREC_FP64)
+        b.set_positions(torch.tensor(np.concatenate([s.r for s in systems]).T.copy(),
+                                     device="cuda"))
+        f, _ = b.forces(0)
+        f = f.cpu().numpy()
+        for c, s in enumerate(systems):
+            o = oracle_lib.Oracle(s.params, s.itype, s.A).engforce(s.r, itime=1)
+            g = f[:, b.offsets[c]:b.offsets[c + 1]].T
+            assert np.abs(g - o["f"]).max() <= 1e-10 * np.abs(o["f"]).max(), (kmaxes[c], c)
+        b.close()
