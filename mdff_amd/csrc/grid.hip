@@ -291,21 +291,6 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_bin(int n, Ext e, const dou
   atomicAdd(&cnt[k + 1], 1);  // k_cell_scan turns these into bin starts
 }
 
-// Atoms of a bin in index order: the rank of an entry is the number of
-// smaller indexes in its bin.
-__global__ __launch_bounds__(MDFF_BLOCK) void k_grid_order(int n, const int* __restrict__ key,
-                                                           const int* __restrict__ start,
-                                                           const int* __restrict__ in,
-                                                           int* __restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int a = in[t];
-  const int b = start[key[a]], e = start[key[a] + 1];
-  int r = b;
-  for (int k = b; k < e; ++k) r += in[k] < a;
-  out[r] = a;
-}
-
 // Bins a tile's candidates may sit in, along one axis: atoms whose support
 // starts within W - 1 points before the tile or in it, give or take margin.
 struct BinRange {
@@ -1264,7 +1249,7 @@ bool bin(Plan* p, hipStream_t st, const double4* s4, const int* typ, const int* 
     k_grid_bin<W32><<<gn, MDFF_BLOCK, 0, st>>>(n, e, s4, typ, cfg, active, p->d_key, p->d_start);
   k_cell_scan<<<1, 1024, 0, st>>>(nb, p->d_start, p->d_cur);
   k_cell_fill<<<gn, MDFF_BLOCK, 0, st>>>(n, p->d_key, p->d_cur, p->d_perm0);
-  k_grid_order<<<gn, MDFF_BLOCK, 0, st>>>(n, p->d_key, p->d_start, p->d_perm0, p->d_perm);
+  k_cell_order<<<gn, MDFF_BLOCK, 0, st>>>(n, p->d_key, p->d_start, p->d_perm0, p->d_perm, nullptr);
   const int gt = (e.nseg * e.ntile + MDFF_BLOCK - 1) / MDFF_BLOCK;
   if (p->fp64)
     k_grid_cap<W64><<<gt, MDFF_BLOCK, 0, st>>>(e, mg, p->d_start, p->d_cap);

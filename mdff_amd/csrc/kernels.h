@@ -232,7 +232,8 @@ __global__ void k_cell_bin(int n, const double4* s4, int nc0, int nc1, int nc2, 
                            int* cnt);
 __global__ void k_cell_scan(int m, int* cnt, int* cur);
 __global__ void k_cell_fill(int n, const int* cellof, int* cur, int* perm);
-__global__ void k_cell_order(int m, const int* cnt, int* perm, int* rank);
+__global__ void k_cell_order(int n, const int* cellof, const int* cnt, const int* in, int* perm,
+                             int* rank);
 __global__ void k_pol_rows(int n, const int* perm, const int* typ, unsigned polmask, int* rows);
 __global__ void k_nlist_cells(NlCellArgs a);
 __global__ void k_perm_gather(int n, int inner, int planes, const int* idx, const double* src,

@@ -1397,8 +1397,10 @@ void cell_sort(mdffgpu_ctx* c) {
   k_cell_bin<<<nblk(n), MDFF_BLOCK, 0, st>>>(n, c->d_s4, c->gnc[0], c->gnc[1], c->gnc[2],
                                              c->d_cellof, c->d_cstart);
   k_cell_scan<<<1, 1024, 0, st>>>(ncell, c->d_cstart, c->d_ccur);
-  k_cell_fill<<<nblk(n), MDFF_BLOCK, 0, st>>>(n, c->d_cellof, c->d_ccur, c->d_perm);
-  k_cell_order<<<nblk(ncell), MDFF_BLOCK, 0, st>>>(ncell, c->d_cstart, c->d_perm, c->d_rank);
+  // unordered cells in the rows buffer, which k_pol_rows fills afterwards
+  k_cell_fill<<<nblk(n), MDFF_BLOCK, 0, st>>>(n, c->d_cellof, c->d_ccur, c->d_polrows);
+  k_cell_order<<<nblk(n), MDFF_BLOCK, 0, st>>>(n, c->d_cellof, c->d_cstart, c->d_polrows,
+                                               c->d_perm, c->d_rank);
   if (c->linduced && scf_field_fp32(c))
     k_pol_rows<<<1, 1024, 0, st>>>(n, c->d_perm, c->d_typ, c->polmask, c->d_polrows);
   check_launch(c, "cell sort");

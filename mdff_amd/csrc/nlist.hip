@@ -85,23 +85,24 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_cell_fill(int n, const int* __re
   perm[atomicAdd(&cur[cellof[i]], 1)] = i;
 }
 
-// Atoms of each cell in index order; rank[perm[r]] = r.
-__global__ __launch_bounds__(MDFF_BLOCK) void k_cell_order(int m, const int* __restrict__ cnt,
+// Atoms of each cell in index order: the slot of an atom is its cell's first
+// plus the number of smaller indexes among its cell's entries of `in` (filled
+// by k_cell_fill).  rank[perm[r]] = r, unless rank is null.  One thread per
+// entry: at 16,384 atoms in cells of 54, 5 us against 717 us for one thread
+// per cell with an insertion sort in memory.
+__global__ __launch_bounds__(MDFF_BLOCK) void k_cell_order(int n, const int* __restrict__ cellof,
+                                                           const int* __restrict__ cnt,
+                                                           const int* __restrict__ in,
                                                            int* __restrict__ perm,
                                                            int* __restrict__ rank) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= m) return;
-  const int b = cnt[c], e = cnt[c + 1];
-  for (int r = b + 1; r < e; ++r) {
-    const int v = perm[r];
-    int q = r - 1;
-    while (q >= b && perm[q] > v) {
-      perm[q + 1] = perm[q];
-      --q;
-    }
-    perm[q + 1] = v;
-  }
-  for (int r = b; r < e; ++r) rank[perm[r]] = r;
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int a = in[t];
+  const int b = cnt[cellof[a]], e = cnt[cellof[a] + 1];
+  int r = b;
+  for (int k = b; k < e; ++k) r += in[k] < a;
+  perm[r] = a;
+  if (rank) rank[a] = r;
 }
 
 // Ranks r whose atom perm[r] has a species with its bit in polmask, in rank
