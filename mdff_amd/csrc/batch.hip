@@ -995,7 +995,7 @@ void es_call(mdffgpu_batch* b, int mode, const double* q, const double* mu, cons
   if (b->gp) {
     // the induced dipoles sit on the polarizable atoms, where alone the
     // static and SCF calls' field is read
-    grid::sums(b->gp, nullptr, b->st, b->d_s4, q, mu, chg, dip, mode == ES_FINAL, mode == ES_IND,
+    grid::sums(b->gp, nullptr, b->st, q, mu, chg, dip, mode == ES_FINAL, mode == ES_IND,
                mode != ES_FINAL, b->d_apart, nullptr);
     k_b_grid_fields<<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, b->d_cfg, b->d_bc, b->d_apart, q, mu,
                                                        mode == ES_FINAL, b->d_rec, b->d_frec);

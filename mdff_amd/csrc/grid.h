@@ -14,6 +14,7 @@
 struct mdffgpu_ctx;
 
 namespace mdff {
+struct CombineArgs;
 namespace grid {
 
 // One configuration: its cell and Ewald alpha and its atoms in the caller's
@@ -61,9 +62,12 @@ void prepare(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double4* s4);
 // only the active atoms carry moments; dst_active: rows of the active atoms
 // only.  With pout (one configuration), block partials of the energy and
 // stress sums go to pout[row * nblocks + block] (7 rows); returns nblocks.
-int sums(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double4* s4, const double* q,
-         const double* mu, bool chg, bool dip,
-         bool second, bool src_active, bool dst_active, double* out, double* pout);
+// With ind (an SCF call of one configuration, no surface term) the combine of
+// k_combine64<ES_IND> is done here instead of writing out; returns the number
+// of block partials per row of ind->rpart.
+int sums(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q, const double* mu, bool chg,
+         bool dip, bool second, bool src_active, bool dst_active, double* out, double* pout,
+         const CombineArgs* ind = nullptr);
 
 }  // namespace grid
 }  // namespace mdff

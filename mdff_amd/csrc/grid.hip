@@ -67,7 +67,9 @@ struct Mat;
 template <>
 struct Mat<double> {
   typedef v4d acc;
-  static constexpr int W = W64, DEG = DEG64;
+  // ZV: z per lane of the interpolation; PADZ: padding of the potential's
+  // rows, at least W - 1
+  static constexpr int W = W64, DEG = DEG64, ZV = 1, PADZ = 20;
   static __device__ __forceinline__ v4d mma(double a, double b, v4d c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
@@ -77,7 +79,7 @@ struct Mat<double> {
 template <>
 struct Mat<float> {
   typedef v4f acc;
-  static constexpr int W = W32, DEG = DEG32;
+  static constexpr int W = W32, DEG = DEG32, ZV = 2, PADZ = 12;
   static __device__ __forceinline__ v4f mma(float a, float b, v4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
@@ -123,6 +125,8 @@ struct Plan {
   double* d_D = nullptr;     // Ewald factors / phi^^2, [seg][n1][n2][n3]
   void* d_tab = nullptr;     // [atom][axis][phi, phi'][W]
   void* d_tab2 = nullptr;    // [atom][axis][W], phi''
+  int4* d_l0 = nullptr;      // first points of the supports
+  void* d_P = nullptr;       // potentials, [seg][x][y][M3 + PADZ]
   // bins: two classes (active atoms, the others) of nseg x ntile bins
   int *d_key = nullptr, *d_start = nullptr, *d_cur = nullptr, *d_perm0 = nullptr,
       *d_perm = nullptr, *d_cap = nullptr;
@@ -439,14 +443,15 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_lists(
 }
 
 // Kernel values of every atom: tab[atom][axis][phi, phi'][W] and
-// tab2[atom][axis][phi''][W].  One thread per (atom, axis, point); the
+// tab2[atom][axis][phi''][W], and the first points l0[atom] of its support.  One thread per (atom, axis, point); the
 // coefficients in LDS with the piece fastest, so that the lanes of an atom
 // read consecutive words.
 template <typename R>
 __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_tab(int n, Ext e, const double4* __restrict__ s4,
                                                          const R* __restrict__ poly,
                                                          R* __restrict__ tab,
-                                                         R* __restrict__ tab2) {
+                                                         R* __restrict__ tab2,
+                                                         int* __restrict__ l0) {
   constexpr int W = Mat<R>::W, D = Mat<R>::DEG + 1;
   __shared__ R pc[9 * D * W];
   for (int k = threadIdx.x; k < 9 * D * W; k += MDFF_BLOCK) pc[k] = poly[k];
@@ -459,7 +464,8 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_tab(int n, Ext e, const dou
     const int i = (int)(g / (3 * W));
     const double* sp = reinterpret_cast<const double*>(s4 + i);
     double ud;
-    (void)support<W>(sp[ax], e.M[ax], ud);
+    const int l = support<W>(sp[ax], e.M[ax], ud);
+    if (a == 0) l0[4 * (size_t)i + ax] = l;
     const R u = (R)ud;
     const R* c = pc + (size_t)ax * 3 * D * W + (W - 1 - a);
     R f0 = 0, f1 = 0, f2 = 0;
@@ -527,64 +533,69 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_spread(
             x0 = tile / (e.nt[2] * e.nt[1]) * TX;
   const Cell& cell = segs[seg].cell;
   const int al = t >> 3, pp = t & 7;  // 8 threads expand an atom
-  // this thread's share of a chunk, in registers; the list entry of the
-  // chunk after the one being loaded, so that the loads that depend on it
-  // issue at once
-  R vx[2][2], vy[2], vz[2];
-  int2 en = al < m ? lst[al] : make_int2(-1, 0);
+  // this thread's share of a chunk as loaded, every load unconditional (a
+  // masked one is waited for at the end of its branch), masked and multiplied
+  // when it goes to LDS; the list entry a chunk further ahead, so that the
+  // loads that depend on it issue at once
+  R tx[2][2], ty[2], tz[2];
+  double m0 = 0.0, m1 = 0.0, m2 = 0.0, qi = 0.0;
+  int2 cur, nxt = lst[min(al, max(m - 1, 0))];
+  auto dist = [](int d, int M) { return d < 0 ? d + M : d; };
   auto load = [&](int c0) {
-    const int2 cur = en;
-    en = c0 + SCH + al < m ? lst[c0 + SCH + al] : make_int2(-1, 0);
-    for (int k = 0; k < 2; ++k) vx[k][0] = vx[k][1] = R(0);
-    vy[0] = vy[1] = vz[0] = vz[1] = R(0);
+    cur = nxt;
+    nxt = lst[min(c0 + SCH + al, max(m - 1, 0))];
     const int i = cur.x;
-    if (i < 0) return;
     const R* T = tab + (size_t)i * 6 * W;
-    R mg[3] = {R(0), R(0), R(0)};
-    if (DIP) {
-      const double m0 = mu[i], m1 = mu[i + n], m2 = mu[i + 2 * (size_t)n];
-      for (int a = 0; a < 3; ++a)
-        mg[a] = (R)(e.M[a] * (cell.B[3 * a] * m0 + cell.B[3 * a + 1] * m1 + cell.B[3 * a + 2] * m2));
-    }
-    const R qi = CHG ? (R)q[i] : R(0);
     const int ox = (cur.y & 255) - 64, oy = (cur.y >> 8 & 255) - 64, oz = (cur.y >> 16 & 255) - 64;
+    if (DIP) {
+      m0 = mu[i];
+      m1 = mu[i + n];
+      m2 = mu[i + 2 * (size_t)n];
+    }
+    if (CHG) qi = q[i];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      int d = pp + 8 * k - ox;
-      d += d < 0 ? e.M[0] : 0;
-      if (d < W) {
-        vx[k][1] = T[d];
-        if (DIP) vx[k][0] = mg[0] * T[W + d];
-      }
+      const int d = min(dist(pp + 8 * k - ox, e.M[0]), W - 1);
+      tx[k][1] = T[d];
+      if (DIP) tx[k][0] = T[W + d];
     }
-    int d = pp - oy;
-    d += d < 0 ? e.M[1] : 0;
-    if (d < W) {
-      const R f = T[2 * W + d];
-      vy[0] = f;
-      vy[1] = CHG ? qi * f : R(0);
-      if (DIP) vy[1] += mg[1] * T[3 * W + d];
-    }
-    d = pp - oz;
-    d += d < 0 ? e.M[2] : 0;
-    if (d < W) {
-      vz[0] = T[4 * W + d];
-      if (DIP) vz[1] = mg[2] * T[5 * W + d];
+    const int dy = min(dist(pp - oy, e.M[1]), W - 1), dz = min(dist(pp - oz, e.M[2]), W - 1);
+    ty[0] = T[2 * W + dy];
+    tz[0] = T[4 * W + dz];
+    if (DIP) {
+      ty[1] = T[3 * W + dy];
+      tz[1] = T[5 * W + dz];
     }
   };
   acc_t acc = {0, 0, 0, 0};
   const int row = lane & 15, kk = lane >> 4;
   const int yy = 2 * wv + (row >> 3), zz = row & 7;
-  load(0);
+  if (m > 0) load(0);
   for (int c0 = 0; c0 < m; c0 += SCH) {
-    for (int k = 0; k < 2; ++k) {
-      if (DIP) lx[al][0][pp + 8 * k] = vx[k][0];
-      lx[al][1][pp + 8 * k] = vx[k][1];
+    {
+      const int ox = (cur.y & 255) - 64, oy = (cur.y >> 8 & 255) - 64,
+                oz = (cur.y >> 16 & 255) - 64;
+      const bool in = c0 + al < m;
+      R mg[3] = {R(0), R(0), R(0)};
+      if (DIP)
+        for (int a = 0; a < 3; ++a)
+          mg[a] = (R)(e.M[a] *
+                      (cell.B[3 * a] * m0 + cell.B[3 * a + 1] * m1 + cell.B[3 * a + 2] * m2));
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const R on = in && dist(pp + 8 * k - ox, e.M[0]) < W ? R(1) : R(0);
+        if (DIP) lx[al][0][pp + 8 * k] = on * mg[0] * tx[k][0];
+        lx[al][1][pp + 8 * k] = on * tx[k][1];
+      }
+      const R ony = dist(pp - oy, e.M[1]) < W ? R(1) : R(0);
+      const R onz = dist(pp - oz, e.M[2]) < W ? R(1) : R(0);
+      R y1 = CHG ? (R)qi * ty[0] : R(0);
+      if (DIP) y1 += mg[1] * ty[1];
+      ly[al][pp] = {ony * ty[0], ony * y1};
+      lz[al][pp] = {onz * tz[0], DIP ? onz * mg[2] * tz[1] : R(0)};
     }
-    ly[al][pp] = {vy[0], vy[1]};
-    lz[al][pp] = {vz[0], vz[1]};
     __syncthreads();
-    load(c0 + SCH);
+    if (c0 + SCH < m) load(c0 + SCH);
     const int left = min(SCH, m - c0);
     if (DIP) {
       // lane's K slot: atom 2 s + (kk >> 1), term kk & 1
@@ -856,7 +867,7 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_mid(Ext e, Tw tw, const dou
 // with c = 1 for n3 = 0, else 2 (the other half space).
 template <typename R>
 __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_inv(Ext e, Tw tw, const double2* __restrict__ T,
-                                                         R* __restrict__ G) {
+                                                         R* __restrict__ P) {
   extern __shared__ double sh[];
   const int KZ = e.np[2], KS = KZ + 1;
   double* Wr = sh;                // [2][16][KS]
@@ -904,7 +915,8 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_inv(Ext e, Tw tw, const dou
     }
   }
   __syncthreads();
-  R* g = G + (size_t)seg * e.ng + (size_t)x * M2 * M3;
+  const int P3 = M3 + Mat<R>::PADZ;
+  R* g = P + ((size_t)seg * e.M[0] + x) * M2 * P3;
   const int nz = (M3 / 2 + 15) / 16;
   for (int j = wv; j < 2 * nz; j += 4) {
     const int m = j & 1, zt = j >> 1;
@@ -933,8 +945,12 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_inv(Ext e, Tw tw, const dou
       int y = yt * 16 + Mat<double>::row(lane, i);
       if (y >= M2 / 2 || z >= M3 / 2) continue;
       if (m) y = M2 - 1 - y;
-      g[(size_t)y * M3 + z] = (R)(C[i] + S[i]);
-      g[(size_t)y * M3 + M3 - 1 - z] = (R)(C[i] - S[i]);
+      R* o = g + (size_t)y * P3;
+      const R lo = (R)(C[i] + S[i]), hi = (R)(C[i] - S[i]);
+      o[z] = lo;
+      o[M3 - 1 - z] = hi;
+      if (z < Mat<R>::PADZ) o[M3 + z] = lo;
+      if (M3 - 1 - z < Mat<R>::PADZ) o[2 * M3 - 1 - z] = hi;
     }
   }
 }
@@ -963,86 +979,230 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_factors(Ext e, const Seg* _
 // ---------------------------------------------------------------------------
 // interpolation
 
-// A wave takes an atom, its lanes the W x W (y, z) columns of the support,
-// each summing its column over x against phi_x, phi'_x (phi''_x).  The grid
-// is read where it lies: consecutive waves take atoms in bin order, which
-// share most of their support in the caches.  16,384 atoms on 96^3 points:
-// 18 us at W = 10, 41 us at W = 16; with a tile's region staged in LDS first
-// 24 and 79 us (the staging is latency, and one workgroup per CU at W = 16).
-template <typename R, bool SECOND>
+// Sum over the wave, uniform: DPP adds within rows, then across them.
+template <int CTRL>
+__device__ __forceinline__ float dpp0(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp0(double x) {
+  return __hiloint2double(
+      __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true),
+      __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane63(float x) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
+__device__ __forceinline__ double lane63(double x) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
+                          __builtin_amdgcn_readlane(__double2loint(x), 63));
+}
+template <typename R>
+__device__ __forceinline__ R wave_total(R x) {
+  x += dpp0<0x111>(x);  // row_shr 1, 2, 4, 8
+  x += dpp0<0x112>(x);
+  x += dpp0<0x114>(x);
+  x += dpp0<0x118>(x);
+  x += dpp0<0x142>(x);  // row_bcast 15, 31
+  x += dpp0<0x143>(x);
+  return lane63(x);
+}
+
+// A wave takes an atom, its lanes the support's W x ceil(W / ZV) groups of ZV
+// neighbouring z at one y, each summing its columns over x against phi_x,
+// phi'_x (phi''_x), then over its z.  The potentials are read where they lie
+// (their rows padded with their own beginning, so that a group never wraps):
+// consecutive waves take atoms in bin order, which share most of their
+// support in the caches.  16,384 atoms on 96^3 points: 13 us at W = 10, 59 us
+// at W = 17, the latter bound by the lines it takes through L2 (a support's
+// row of 136 bytes spans two or three; the same with one to five passes'
+// loads in flight).  With the region of a tile staged in LDS 15 and 52 us,
+// but 12 us instead of 5 for 2,000 atoms on 48^3 (few workgroups, each first
+// waiting for its region).
+//
+// IND (an SCF field of one configuration, no surface term): the field of
+// k_combine64<ES_IND> is formed here too, with the block partials of its
+// residual (or p.Ap) rows in ca.rpart: 15 and 62 us, against 5.6 us more in a
+// launch of its own.
+template <typename R, bool SECOND, bool IND, int BA>
 __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_gather(
-    Ext e, const R* __restrict__ G, const double4* __restrict__ s4, const R* __restrict__ tab,
-    const R* __restrict__ tab2, const int* __restrict__ perm, const int* __restrict__ cfg, int count, int n,
-    double* __restrict__ out) {
-  constexpr int W = Mat<R>::W;
-  constexpr int IT = (W * W + 63) / 64;
+    Ext e, const R* __restrict__ P, const int4* __restrict__ l0, const R* __restrict__ tab,
+    const R* __restrict__ tab2, const int* __restrict__ perm, const int* __restrict__ cfg,
+    int count, int apw, int n, double* __restrict__ out, CombineArgs ca) {
+  constexpr int W = Mat<R>::W, ZV = Mat<R>::ZV, NG = (W + ZV - 1) / ZV;
+  constexpr int IT = (W * NG + 63) / 64;
   constexpr int NV = SECOND ? 9 : 3;
-  const int lane = threadIdx.x & 63;
-  const int blk = xcd_tile(blockIdx.x, (count + 3) / 4);
-  const int h = blk * 4 + (threadIdx.x >> 6);
-  if (h >= count) return;
-  const int i = __builtin_amdgcn_readfirstlane(perm[h]);
-  const double4 sf = s4[i];
-  double u;
-  const int l0x = support<W>(sf.x, e.M[0], u), l0y = support<W>(sf.y, e.M[1], u),
-            l0z = support<W>(sf.z, e.M[2], u);
-  const R* g = G + (cfg ? (size_t)cfg[i] * e.ng : 0);
-  const R* T = tab + (size_t)i * 6 * W;
-  const R* T2 = tab2 + (size_t)i * 3 * W;
-  const size_t px = (size_t)e.M[1] * e.M[2];
-  R v[NV];
+  __shared__ double red[2][4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int per = 4 * apw;
+  const int nb = (count + per - 1) / per;
+  const int blk = xcd_tile(blockIdx.x, nb);
+  if (blk >= nb) return;
+  const int P3 = e.M[2] + Mat<R>::PADZ;
+  const size_t px = (size_t)e.M[1] * P3;
+  // BA atoms of a wave at a time, their loads issued together: a dependent
+  // load here costs a microsecond (the data was written by other XCDs)
+  double acc0 = 0.0, acc1 = 0.0;
+  const double c1 = 1.0 / (4.0 * MDFF_PI), c2 = -1.0 / (8.0 * MDFF_PI * MDFF_PI);
+  const double Mx = e.M[0], My = e.M[1], Mz = e.M[2];
+  const size_t N = n;
+  for (int k0 = 0; k0 < apw; k0 += BA) {
+    const int h0 = (blk * 4 + wv) * apw + k0;
+    const int left = min(min(count - h0, apw - k0), BA);
+    if (left <= 0) break;
+    // lanes 3 j + r: component r of atom j in the combine
+    const int ej = min(lane / 3, left - 1), er3 = lane % 3;
+    const int ei = perm[h0 + ej];
+    int id[BA], lx[BA], ly[BA], lz[BA];
+    {
+      const int4 l = l0[ei];
 #pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = R(0);
-#pragma unroll
-  for (int it = 0; it < IT; ++it) {
-    const int c = lane + 64 * it;
-    const bool in = c < W * W;
-    const int b = in ? c / W : 0, d = in ? c % W : 0;
-    const R* s = g + (size_t)wrap(l0y + b, e.M[1]) * e.M[2] + wrap(l0z + d, e.M[2]);
-    R x[W];
-#pragma unroll
-    for (int a = 0; a < W; ++a) x[a] = s[wrap(l0x + a, e.M[0]) * px];
-    R s0 = 0, s1 = 0, s2 = 0;
-#pragma unroll
-    for (int a = 0; a < W; ++a) {
-      s0 += T[a] * x[a];
-      s1 += T[W + a] * x[a];
-      if (SECOND) s2 += T2[a] * x[a];
+      for (int j = 0; j < BA; ++j) {
+        id[j] = __builtin_amdgcn_readlane(ei, 3 * j);
+        lx[j] = __builtin_amdgcn_readlane(l.x, 3 * j);
+        ly[j] = __builtin_amdgcn_readlane(l.y, 3 * j);
+        lz[j] = __builtin_amdgcn_readlane(l.z, 3 * j);
+      }
     }
-    const R on = in ? R(1) : R(0);
-    const R fy = T[2 * W + b] * on, gy = T[3 * W + b] * on;
-    const R fz = T[4 * W + d], gz = T[5 * W + d];
-    v[0] += s1 * (fy * fz);
-    v[1] += s0 * (gy * fz);
-    v[2] += s0 * (fy * gz);
-    if (SECOND) {
-      const R hy = T2[W + b] * on, hz = T2[2 * W + d];
-      v[3] += s2 * (fy * fz);
-      v[4] += s0 * (hy * fz);
-      v[5] += s0 * (fy * hz);
-      v[6] += s1 * (gy * fz);
-      v[7] += s1 * (fy * gz);
-      v[8] += s0 * (gy * gz);
+    double m0 = 0, m1 = 0, m2 = 0, efd = 0, est = 0;
+    int ety = 0;
+    if (IND) {
+      m0 = ca.mu[ei];
+      m1 = ca.mu[ei + N];
+      m2 = ca.mu[ei + 2 * N];
+      efd = ca.ef_dir[ei + er3 * N];
+      ety = ca.typ[ei];
+      if (!ca.cg_Ap) est = ca.E_stat[ei + er3 * N];
+    }
+    R v[BA][NV];
+#pragma unroll
+    for (int j = 0; j < BA; ++j)
+#pragma unroll
+      for (int c = 0; c < NV; ++c) v[j][c] = R(0);
+    // not unrolled at W = 17: five passes' loads would leave two waves per SIMD
+#pragma unroll (IT > 2 ? 1 : IT)
+    for (int it = 0; it < IT; ++it) {
+      const int c = lane + 64 * it;
+      const bool in = c < W * NG;
+      const int b = in ? c / NG : 0, zg = in ? c % NG * ZV : 0;
+      R x[BA][W][ZV], fy[BA], gy[BA], hy[BA], fz[BA][ZV], gz[BA][ZV], hz[BA][ZV];
+#pragma unroll
+      for (int j = 0; j < BA; ++j) {
+        const R* T = tab + (size_t)id[j] * 6 * W;
+        const R* T2 = tab2 + (size_t)id[j] * 3 * W;
+        const R* s = P + (cfg ? (size_t)cfg[id[j]] * e.M[0] * px : 0) +
+                     (size_t)wrap(ly[j] + b, e.M[1]) * P3 + lz[j] + zg;
+#pragma unroll
+        for (int a = 0; a < W; ++a)
+          __builtin_memcpy(x[j][a], s + wrap(lx[j] + a, e.M[0]) * px, sizeof(x[j][a]));
+        fy[j] = T[2 * W + b];
+        gy[j] = T[3 * W + b];
+        if (SECOND) hy[j] = T2[W + b];
+#pragma unroll
+        for (int z = 0; z < ZV; ++z) {
+          const int d = min(zg + z, W - 1);
+          fz[j][z] = T[4 * W + d];
+          gz[j][z] = T[5 * W + d];
+          if (SECOND) hz[j][z] = T2[2 * W + d];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < BA; ++j) {
+        const R* T = tab + (size_t)id[j] * 6 * W;
+        const R* T2 = tab2 + (size_t)id[j] * 3 * W;
+#pragma unroll
+        for (int z = 0; z < ZV; ++z) {
+          R s0 = 0, s1 = 0, s2 = 0;
+#pragma unroll
+          for (int a = 0; a < W; ++a) {
+            s0 += T[a] * x[j][a][z];
+            s1 += T[W + a] * x[j][a][z];
+            if (SECOND) s2 += T2[a] * x[j][a][z];
+          }
+          const R on = in && zg + z < W ? R(1) : R(0);
+          s0 *= on;
+          s1 *= on;
+          s2 *= on;
+          v[j][0] += s1 * (fy[j] * fz[j][z]);
+          v[j][1] += s0 * (gy[j] * fz[j][z]);
+          v[j][2] += s0 * (fy[j] * gz[j][z]);
+          if (SECOND) {
+            v[j][3] += s2 * (fy[j] * fz[j][z]);
+            v[j][4] += s0 * (hy[j] * fz[j][z]);
+            v[j][5] += s0 * (fy[j] * hz[j][z]);
+            v[j][6] += s1 * (gy[j] * fz[j][z]);
+            v[j][7] += s1 * (fy[j] * gz[j][z]);
+            v[j][8] += s0 * (gy[j] * gz[j][z]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < BA; ++j)
+#pragma unroll
+      for (int c = 0; c < NV; ++c) v[j][c] = wave_total(v[j][c]);
+    // the sums of this lane's atom
+    R w[NV];
+#pragma unroll
+    for (int c = 0; c < NV; ++c) {
+      w[c] = v[0][c];
+#pragma unroll
+      for (int j = 1; j < BA; ++j) w[c] = ej == j ? v[j][c] : w[c];
+    }
+    const double u0 = c1 * Mx * (double)w[0], u1 = c1 * My * (double)w[1],
+                 u2 = c1 * Mz * (double)w[2];
+    if (lane >= 3 * left) continue;
+    if (IND) {
+      const int r = er3;
+      const double* B = ca.cell.B;
+      const double b0 = r == 0 ? B[0] : r == 1 ? B[1] : B[2],
+                   b1 = r == 0 ? B[3] : r == 1 ? B[4] : B[5],
+                   b2 = r == 0 ? B[6] : r == 1 ? B[7] : B[8];
+      const double fe = -2.0 * ca.fpi_V * (2.0 * MDFF_PI);
+      const double er = fe * (b0 * u0 + b1 * u1 + b2 * u2);
+      const double mr = r == 0 ? m0 : r == 1 ? m1 : m2;
+      const double ef = (efd + er) + 2.0 * ca.selfa2 * mr;
+      if (ca.cg_Ap) {
+        // Ap = alpha^-1 p - T p and p.Ap
+        const double* ip = ca.T->invpol[ety];
+        const double ap = ip[r] * m0 + ip[r + 3] * m1 + ip[r + 6] * m2 - ef;
+        ca.cg_Ap[ei + r * N] = ap;
+        acc0 += mr * ap;
+      } else {
+        // E and the stopping criterion's rows (resid_terms)
+        const double E = est + ef;
+        ca.E[ei + r * N] = E;
+        const double pa = ca.T->pol[ety][r + 3 * r];
+        const double d = pa == 0.0 ? 0.0 : mr / pa - E;
+        acc0 += d * d;
+        if (r == 0) acc1 += 1.0;
+      }
+    } else if (er3 == 0) {
+      double* r = out + ei;
+      r[0] = u0;
+      r[N] = u1;
+      r[2 * N] = u2;
+      if (SECOND) {
+        r[3 * N] = c2 * Mx * Mx * (double)w[3];
+        r[4 * N] = c2 * My * My * (double)w[4];
+        r[5 * N] = c2 * Mz * Mz * (double)w[5];
+        r[6 * N] = c2 * Mx * My * (double)w[6];
+        r[7 * N] = c2 * Mx * Mz * (double)w[7];
+        r[8 * N] = c2 * My * Mz * (double)w[8];
+      }
     }
   }
-#pragma unroll
-  for (int k = 0; k < NV; ++k)
-    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
-  if (lane == 0) {
-    const double f1 = 1.0 / (4.0 * MDFF_PI), f2 = -1.0 / (8.0 * MDFF_PI * MDFF_PI);
-    const double Mx = e.M[0], My = e.M[1], Mz = e.M[2];
-    double* r = out + i;
-    const size_t N = n;
-    r[0] = f1 * Mx * (double)v[0];
-    r[N] = f1 * My * (double)v[1];
-    r[2 * N] = f1 * Mz * (double)v[2];
-    if (SECOND) {
-      r[3 * N] = f2 * Mx * Mx * (double)v[3];
-      r[4 * N] = f2 * My * My * (double)v[4];
-      r[5 * N] = f2 * Mz * Mz * (double)v[5];
-      r[6 * N] = f2 * Mx * My * (double)v[6];
-      r[7 * N] = f2 * Mx * Mz * (double)v[7];
-      r[8 * N] = f2 * My * Mz * (double)v[8];
+  if (IND) {
+    acc0 = wave_total(acc0);
+    acc1 = wave_total(acc1);
+    if (lane == 0) {
+      red[0][wv] = acc0;
+      red[1][wv] = acc1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      ca.rpart[blk] = ((red[0][0] + red[0][1]) + red[0][2]) + red[0][3];
+      ca.rpart[nb + blk] = ((red[1][0] + red[1][1]) + red[1][2]) + red[1][3];
     }
   }
 }
@@ -1123,13 +1283,15 @@ static bool setup(Plan* p) {
     }
   }
   double* d_tw = nullptr;
-  R *d_poly = nullptr, *d_G = nullptr, *d_tab = nullptr, *d_tab2 = nullptr;
+  R *d_poly = nullptr, *d_G = nullptr, *d_P = nullptr, *d_tab = nullptr, *d_tab2 = nullptr;
   if (!take(p, &d_tw, tw.size()) || !take(p, &p->d_phat, ph.size()) ||
-      !take(p, &d_poly, poly.size()) || !take(p, &d_G, e.ng * e.nseg * p->split) ||
+      !take(p, &d_poly, poly.size()) || !take(p, &d_G, e.ng * e.nseg * p->split) || !take(p, &p->d_l0, p->natom) ||
+      !take(p, &d_P, (size_t)e.nseg * e.M[0] * e.M[1] * (e.M[2] + Mat<R>::PADZ)) ||
       !take(p, &d_tab, (size_t)p->natom * 6 * W) || !take(p, &d_tab2, (size_t)p->natom * 3 * W))
     return false;
   p->d_poly = d_poly;
   p->d_G = d_G;
+  p->d_P = d_P;
   p->d_tab = d_tab;
   p->d_tab2 = d_tab2;
   for (int a = 0; a < 3; ++a) {
@@ -1194,7 +1356,7 @@ Plan* create(hipStream_t st, const std::vector<Seg>& segs, const int kmax[3], bo
   for (const auto& b : big)
     if (b.second > 65536)
       ok = ok && hipFuncSetAttribute(b.first, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     160 * 1024) == hipSuccess;
+                                     (int)b.second) == hipSuccess;
   if (!ok) {
     (void)hipGetLastError();
     destroy(p);
@@ -1290,22 +1452,23 @@ void prepare(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double4* s4) {
     k_grid_lists<W64><<<g, MDFF_BLOCK, 0, st>>>(e, mg, s4, p->d_start, p->d_perm, p->cap, p->d_ov,
                                                 p->d_cnt);
     k_grid_tab<double><<<gt, MDFF_BLOCK, 0, st>>>(p->natom, e, s4, (const double*)p->d_poly,
-                                                  (double*)p->d_tab, (double*)p->d_tab2);
+                                                  (double*)p->d_tab, (double*)p->d_tab2, (int*)p->d_l0);
   } else {
     k_grid_lists<W32><<<g, MDFF_BLOCK, 0, st>>>(e, mg, s4, p->d_start, p->d_perm, p->cap, p->d_ov,
                                                 p->d_cnt);
     k_grid_tab<float><<<gt, MDFF_BLOCK, 0, st>>>(p->natom, e, s4, (const float*)p->d_poly,
-                                                 (float*)p->d_tab, (float*)p->d_tab2);
+                                                 (float*)p->d_tab, (float*)p->d_tab2, (int*)p->d_l0);
   }
 }
 
 template <typename R>
-static int sums_t(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double4* s4, const double* q,
+static int sums_t(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,
                   const double* mu, bool chg, bool dip, bool second, bool src_active, bool dst_active,
-                  double* out, double* pout) {
+                  double* out, double* pout, const CombineArgs* ind) {
   const Ext& e = p->e;
   const int n = p->natom;
   R* G = static_cast<R*>(p->d_G);
+  R* P = static_cast<R*>(p->d_P);
   const R* tab = static_cast<const R*>(p->d_tab);
   const R* tab2 = static_cast<const R*>(p->d_tab2);
   const dim3 gt(xcd_blocks(e.ntile), e.nseg, p->split);
@@ -1338,25 +1501,43 @@ static int sums_t(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double4* s4, 
     k_grid_mid<false><<<gm, MDFF_BLOCK, lds_mid(e), st>>>(e, p->tw, p->d_D, p->d_T, en);
   }
   const dim3 gi(e.M[0], (e.M[1] / 2 + 15) / 16, e.nseg);
-  k_grid_inv<R><<<gi, MDFF_BLOCK, lds_inv(e), st>>>(e, p->tw, p->d_T, G);
+  k_grid_inv<R><<<gi, MDFF_BLOCK, lds_inv(e), st>>>(e, p->tw, p->d_T, P);
   }
   ProfScope _ps(ctx, K_GRID_GATHER);
   const int count = dst_active ? p->nact : n;
-  const int gg = xcd_blocks((count + 3) / 4);
-  if (second)
-    k_grid_gather<R, true><<<gg, MDFF_BLOCK, 0, st>>>(e, G, s4, tab, tab2, p->d_perm, p->cfg, count, n,
-                                                      out);
+  // about 4096 waves of a large system take the atoms in turn
+  const int apw = std::max(1, count / (sizeof(R) == 8 ? 8192 : 4096));
+  const int nb = (count + 4 * apw - 1) / (4 * apw);
+  if (count == 0) return ind ? 0 : (e.NCC + 7) / 8;
+  const int gg = xcd_blocks(nb);
+  CombineArgs ca;
+  std::memset(&ca, 0, sizeof(ca));
+  if (ind) ca = *ind;
+  auto go = [&](auto kernel) {
+    kernel<<<gg, MDFF_BLOCK, 0, st>>>(e, P, p->d_l0, tab, tab2, p->d_perm, p->cfg, count, apw, n,
+                                      out, ca);
+  };
+  // FP32 waves that take several atoms load four at once (registers)
+  constexpr int BA = sizeof(R) == 4 ? 4 : 1;
+  if (ind && apw > 1)
+    go(k_grid_gather<R, false, true, BA>);
+  else if (ind)
+    go(k_grid_gather<R, false, true, 1>);
+  else if (second)
+    go(k_grid_gather<R, true, false, 1>);
+  else if (apw > 1)
+    go(k_grid_gather<R, false, false, BA>);
   else
-    k_grid_gather<R, false><<<gg, MDFF_BLOCK, 0, st>>>(e, G, s4, tab, tab2, p->d_perm, p->cfg, count, n,
-                                                       out);
-  return (e.NCC + 7) / 8;
+    go(k_grid_gather<R, false, false, 1>);
+  return ind ? nb : (e.NCC + 7) / 8;
 }
 
-int sums(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double4* s4, const double* q,
+int sums(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,
          const double* mu, bool chg, bool dip,
-         bool second, bool src_active, bool dst_active, double* out, double* pout) {
-  return p->fp64 ? sums_t<double>(p, ctx, st, s4, q, mu, chg, dip, second, src_active, dst_active, out, pout)
-                 : sums_t<float>(p, ctx, st, s4, q, mu, chg, dip, second, src_active, dst_active, out, pout);
+         bool second, bool src_active, bool dst_active, double* out, double* pout,
+         const CombineArgs* ind) {
+  return p->fp64 ? sums_t<double>(p, ctx, st, q, mu, chg, dip, second, src_active, dst_active, out, pout, ind)
+                 : sums_t<float>(p, ctx, st, q, mu, chg, dip, second, src_active, dst_active, out, pout, ind);
 }
 
 }  // namespace grid

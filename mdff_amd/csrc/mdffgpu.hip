@@ -168,6 +168,7 @@ struct mdffgpu_ctx {
   double* d_cg = nullptr;     // conjugate-gradient SCF: r, z, p, Ap (3N each)
   double* cg_Ap = nullptr;    // set while ES_IND calls are the CG's T p products
   int cg_npap = 0;            // block partials of p.Ap the last such call wrote
+  int nresid = 0;             // block partials per residual row of the last ES_IND call
   bool upol_pending = false;
   double* h_sc = nullptr;  // pinned
   double* h_sc_dev = nullptr;  // device address of h_sc
@@ -841,14 +842,21 @@ void es_call(mdffgpu_ctx* c, int mode, const double* q, const double* mu, int ta
   // does the combine (no surface term)
   int fused_parts = 0;
   c->cg_npap = gb;
+  c->nresid = gb;
   if (c->gp) {
     // the induced dipoles sit on the active (polarizable) atoms, where alone
     // the static and SCF calls' field is read
-    const int nb = grid::sums(c->gp, c, st, c->d_s4, q, mu, chg, dip, efgv, mode == ES_IND,
+    const bool fuse = mode == ES_IND && !P.lsurf;
+    const int nb = grid::sums(c->gp, c, st, q, mu, chg, dip, efgv, mode == ES_IND,
                               mode != ES_FINAL, c->d_apart,
-                              mode == ES_FINAL ? c->d_part : nullptr);
+                              mode == ES_FINAL ? c->d_part : nullptr, fuse ? &ca : nullptr);
     check_launch(c, "grid sums");
     if (mode == ES_FINAL) reduce(c, 7, nb, SC_REC);
+    if (fuse) {
+      // the interpolation did the combine
+      c->cg_npap = c->nresid = nb;
+      return;
+    }
     nsplit_apply = 1;
   } else if (mxk && c->nchunk > 0) {
     const bool fuse = (mode == ES_IND) && c->cg_Ap && !P.lsurf;
@@ -1303,13 +1311,14 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
       // moments (the reference tests convergence after the corrector)
       const int eo = aspc_order(P, itime);
       extrap(c, 5, eo, W_ASPC[eo], c->d_part);
+      c->nresid = gb;
       upol_new = true;
     }
     if (spec) {
       // residual rows of the ES_IND combine, straight into pinned memory
       {
         ProfScope _ps(c, K_REDUCE);
-        k_reduce_rows2<<<2, MDFF_BLOCK, 0, st>>>(c->d_part, gb, c->d_sc + SC_RMSD,
+        k_reduce_rows2<<<2, MDFF_BLOCK, 0, st>>>(c->d_part, c->nresid, c->d_sc + SC_RMSD,
                                                  c->h_sc_dev + SC_RMSD);
       }
       check_launch(c, "k_reduce_rows2");
@@ -1321,7 +1330,7 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
       // next stream synchronisation
       HCK(c, hipEventSynchronize(c->ev_sc));
     } else {
-      reduce(c, 2, gb, SC_RMSD);  // residual rows of the ES_IND combine
+      reduce(c, 2, c->nresid, SC_RMSD);  // residual rows of the ES_IND combine
       sync_scalars(c);
     }
     rmsd = std::sqrt(c->h_sc[SC_RMSD] / c->h_sc[SC_RMSD + 1]);
@@ -2015,7 +2024,7 @@ void efg_frame(mdffgpu_ctx* c, const mdffgpu_efg_opts& o, mdffgpu_energies* en) 
         grid::prepare(c->gp, c, st, c->d_s4);
         grid::unbin(c->gp);
       }
-      grid::sums(c->gp, c, st, c->d_s4, q, mu, true, dip, true, false, false, c->d_apart, nullptr);
+      grid::sums(c->gp, c, st, q, mu, true, dip, true, false, false, c->d_apart, nullptr);
       check_launch(c, "grid sums");
       ca.rec = c->d_apart;
       ca.nrec = 1;
