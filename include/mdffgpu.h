@@ -524,8 +524,10 @@ int mdffgpu_batch_set_tuning(mdffgpu_batch* b, int32_t apply_lanes);
 
 /* Launch shape of the FP32 batch's matrix-core reciprocal sums, chosen by
    the autotuner: K slices of the field apply (1, 2 or 4) and atoms per
-   structure-factor split (a multiple of 128).  MDFFGPU_ERR_UNSUPPORTED when
-   the batch has no such path (FP64, or configurations with different kmax).
+   structure-factor split (a multiple of 128).  A small batch takes the grid
+   sums, which have no such shape: there the arguments are checked only.
+   MDFFGPU_ERR_UNSUPPORTED when the batch has no such path (FP64, or
+   configurations with different kmax).
    No counterpart in the reference. */
 int mdffgpu_batch_set_mixed_tuning(mdffgpu_batch* b, int32_t apply_slices,
                                    int32_t split_atoms);

@@ -656,6 +656,150 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_b_damp_adj(EsDirArgs a, DampSlot
     for (int m = 0; m < NDAMP_MAX; ++m) part[(size_t)m * gridDim.x + blockIdx.x] = acc[m];
 }
 
+// ---------------------------------------------------------------------------
+// Reverse pass of the electrostatic forces.  F_i = -dU/dr_i of the energy U of
+// the moments (q, mu), so that with x = sum_i g_i . F_i
+//   v_i = dx/dmu_i = +d/de E_i   and   w_i = dx/dq_i = -d/de phi_i
+// where E_i = -dU/dmu_i and phi_i = dU/dq_i are the field and potential and e
+// displaces every atom by e g_i.  This is the real-space part (without
+// coul_unit) in the arithmetic R: with r = r_i - r_j, p = g_i - g_j and the
+// radial functions of the energy, g1 = F1/d^3, g2 = 3 F2/d^5, g3 = 15 F3/d^7,
+// damped by h1 = (1 - f)/d^3, h2 = 3 (1 - f + d fd/3)/d^5 where a charge meets
+// a dipole (src/field.f90:2205-2231, 2363-2538):
+//   dE = q_j [(g1 - h1) p - (g2 - h2)(r.p) r]
+//      + g2 [(p.mu_j) r + (r.mu_j) p + (r.p) mu_j] - g3 (r.p)(r.mu_j) r
+//   dphi = -q_j g1 (r.p) + (g1 - h1')(p.mu_j) - (g2 - h2')(r.p)(r.mu_j)
+// (h of the centre's slot, h' of the neighbour's).
+template <typename R>
+__global__ __launch_bounds__(MDFF_BLOCK) void k_b_rev_dir(EsDirArgs a, int dip,
+                                                           const double* __restrict__ g,
+                                                           double* __restrict__ v,
+                                                           double* __restrict__ w) {
+  const int n = a.n;
+  const PairTables* T = a.T;
+  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = tid / LPA, sub = tid % LPA;
+  R dv[3] = {R(0), R(0), R(0)}, dw = R(0);
+  if (i < n) {
+    const double4 si = a.s4[i];
+    const int ti = a.typ[i];
+    const BatchCfg& bcf = a.bc[a.cfg[i]];
+    const R alpha = (R)bcf.alpha, cut2 = (R)bcf.cut2;
+    const R gi[3] = {(R)g[i], (R)g[i + n], (R)g[i + 2 * (size_t)n]};
+    const R alpha2 = alpha * alpha, alpha3 = alpha2 * alpha, alpha5 = alpha3 * alpha2;
+    const R piroot = R(1.77245385090551602730);
+    const int c = a.cnt[i];
+    const int* nb = a.nbr + (size_t)i * a.maxnb;
+    for (int k = sub; k < c; k += LPA) {
+      const int j = nb[k];
+      const double4 sj = a.s4[j];
+      R r[3];
+      const R d2 = min_image_t<R>(bcf.cell, si.x - sj.x, si.y - sj.y, si.z - sj.z, r[0], r[1], r[2]);
+      const R qj = (R)a.q[j];
+      R m[3] = {R(0), R(0), R(0)};
+      if (dip)
+        for (int x = 0; x < 3; ++x) m[x] = (R)a.mu[j + x * (size_t)n];
+      R p[3];
+      for (int x = 0; x < 3; ++x) p[x] = gi[x] - (R)g[j + x * (size_t)n];
+      if (d2 > cut2) continue;
+      const int tj = a.typ[j];
+      const R d = sqrt(d2), d3 = d2 * d, d5 = d3 * d2;
+      const R dm3 = R(1) / d3, dm5 = dm3 / d2, dm7 = dm5 / d2;
+      const R ex = rexp<R>(-alpha2 * d2) / piroot;
+      const R F1 = errfc_t<R>(alpha * d) + R(2) * alpha * d * ex;
+      const R F2 = F1 + R(4) * alpha3 * d3 * ex / R(3);
+      const R F3 = F2 + R(8) * alpha5 * d5 * ex / R(15);
+      const R g1 = F1 * dm3, g2 = R(3) * F2 * dm5, g3 = R(15) * F3 * dm7;
+      R h1 = R(0), h2 = R(0), h1j = R(0), h2j = R(0);
+      const int o = (i < j) ? 0 : 1;
+      const int pij = ti + MDFF_NT * tj, pji = tj + MDFF_NT * ti;
+      if (dip && T->dmp_on[o][pij]) {
+        R f, fd;
+        tt_damp_t<R>(a.tt, (R)T->dmp_b[o][pij], (R)T->dmp_c[o][pij], d, T->dmp_k[o][pij], f, fd);
+        h1 = (R(1) - f) * dm3;
+        h2 = R(3) * (R(1) - f + d * fd / R(3)) * dm5;
+        tt_damp_t<R>(a.tt, (R)T->dmp_b[1 - o][pji], (R)T->dmp_c[1 - o][pji], d,
+                     T->dmp_k[1 - o][pji], f, fd);
+        h1j = (R(1) - f) * dm3;
+        h2j = R(3) * (R(1) - f + d * fd / R(3)) * dm5;
+      }
+      const R rp = r[0] * p[0] + r[1] * p[1] + r[2] * p[2];
+      const R rm = r[0] * m[0] + r[1] * m[1] + r[2] * m[2];
+      const R pm = p[0] * m[0] + p[1] * m[1] + p[2] * m[2];
+      const R cr = -qj * (g2 - h2) * rp + g2 * pm - g3 * rp * rm;
+      const R cp = qj * (g1 - h1) + g2 * rm;
+      const R cm = g2 * rp;
+      for (int x = 0; x < 3; ++x) dv[x] += cr * r[x] + cp * p[x] + cm * m[x];
+      dw += -qj * g1 * rp + (g1 - h1j) * pm - (g2 - h2j) * rp * rm;
+    }
+  }
+  for (int off = LPA / 2; off > 0; off >>= 1) {
+    for (int x = 0; x < 3; ++x) dv[x] += __shfl_xor(dv[x], off, 64);
+    dw += __shfl_xor(dw, off, 64);
+  }
+  if (i < n && sub == 0) {
+    for (int x = 0; x < 3; ++x) v[i + x * (size_t)n] = dv[x];
+    w[i] = -dw;
+  }
+}
+
+// v and w with the reciprocal part: ap holds the U, V sums of (q, mu), ad the U
+// sums and the potential of the displaced sources (grid::adjoint_sums).  With
+// grad psi = 4 pi B U and grad grad psi = -8 pi^2 B V B^T:
+//   v += -(4 pi/V) [grad grad psi . g + grad psi'],  w += -(4 pi/V) [grad psi . g + psi'].
+__global__ __launch_bounds__(MDFF_BLOCK) void k_b_rev_fields(
+    int N, const int* __restrict__ cfg, const BatchCfg* __restrict__ bc, double coul_unit,
+    const double* __restrict__ ap, const double* __restrict__ ad, const double* __restrict__ g,
+    double* __restrict__ v, double* __restrict__ w) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= N) return;
+  const BatchCfg& b = bc[cfg[i]];
+  const double* B = b.cell.B;
+  const size_t n = N;
+  const double fpi = 4.0 * MDFF_PI;
+  double gs[3];  // B^T g
+  for (int a = 0; a < 3; ++a)
+    gs[a] = B[3 * a] * g[i] + B[3 * a + 1] * g[i + n] + B[3 * a + 2] * g[i + 2 * n];
+  double V[6];
+  for (int c = 0; c < 6; ++c) V[c] = ap[i + (3 + c) * n];
+  const double Vm[3][3] = {{V[0], V[3], V[4]}, {V[3], V[1], V[5]}, {V[4], V[5], V[2]}};
+  double x[3], pg = 0.0;
+  for (int a = 0; a < 3; ++a) {
+    const double u = ap[i + a * n];
+    pg += fpi * u * gs[a];
+    x[a] = fpi * ad[i + a * n] -
+           2.0 * fpi * MDFF_PI * (Vm[a][0] * gs[0] + Vm[a][1] * gs[1] + Vm[a][2] * gs[2]);
+  }
+  for (int r = 0; r < 3; ++r)
+    v[i + r * n] = coul_unit * (v[i + r * n] -
+                                b.fpi_V * (B[r] * x[0] + B[r + 3] * x[1] + B[r + 6] * x[2]));
+  w[i] = coul_unit * (w[i] - b.fpi_V * (pg + ad[i + 3 * n]));
+}
+
+// part: scale x [sum_i S_i . lam_i (S given) + sum over species a of w_i (w
+// given)].  Rows of S where lam is zero are not read.
+__global__ __launch_bounds__(MDFF_BLOCK) void k_b_rev_dot(int N, double scale,
+                                                           const double* __restrict__ S,
+                                                           const double* __restrict__ lam,
+                                                           const double* __restrict__ w,
+                                                           const int* __restrict__ typ, int a,
+                                                           double* __restrict__ part) {
+  __shared__ double red[4];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  double acc[1] = {0.0};
+  if (i < N) {
+    if (S)
+      for (int c = 0; c < 3; ++c) {
+        const size_t x = i + (size_t)c * N;
+        if (lam[x] != 0.0) acc[0] += S[x] * lam[x];
+      }
+    if (w && typ[i] == a) acc[0] += w[i];
+  }
+  acc[0] *= scale;
+  block_sum<1>(acc, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
+}
+
 }  // namespace batch
 }  // namespace mdff
 
@@ -694,7 +838,8 @@ struct mdffgpu_batch {
   // reciprocal sums through the uniform grid (configurations with a common
   // kmax), its U, V sums per atom
   mdff::grid::Plan* gp = nullptr;
-  double* d_apart = nullptr;
+  bool grid_calls = false;  // the Ewald calls go through it (grid_state)
+  double *d_apart = nullptr, *d_adj = nullptr, *d_v = nullptr, *d_w = nullptr;
   long long epoch = 0;
   int pol_type[MDFF_NT];
   double pol_alpha[MDFF_NT];
@@ -910,13 +1055,19 @@ bool common_kmax(const mdffgpu_batch* b) {
   return true;
 }
 
-// Grid plan of an FP64 batch whose configurations share kmax, binned at the
-// current positions (set_positions: never inside a graph capture).  Loss and
-// gradient, per-k kernels against the grid: 12 configurations (5,400 atoms,
-// kmax 8) 51.2 -> 10.4 ms, 64 (58,000 atoms) 119 -> 55 ms, 2 (400 atoms, kmax
-// 5) 13.4 -> 4.8 ms.
+// Grid plan of a batch whose configurations share kmax, binned at the current
+// positions (set_positions: never inside a graph capture).  The reverse pass
+// always uses it.  The Ewald calls do in FP64 (loss and gradient by tangents,
+// per-k kernels against the grid: 12 configurations, 5,400 atoms, kmax 8,
+// 51.2 -> 10.4 ms, 64, 58,000 atoms, 119 -> 55 ms, 2, 400 atoms, kmax 5,
+// 13.4 -> 4.8 ms) and in mixed precision up to GRID_POINTS grid points in all,
+// beyond which the matrix-core sums over every k are as fast (they grow with
+// the atoms, the grid with the k mesh): 12 configurations of up to 800 atoms
+// 9.5 -> 6.8 ms, 32 of up to 1000 (2.5 M points) 12.4 -> 11.8, 64 of up to
+// 1536 (4.9 M points) 19.4 against 22.6 ms.
+constexpr size_t GRID_POINTS = 2500000;
 void grid_state(mdffgpu_batch* b) {
-  if (!b->P.lcoulomb || b->mixed || !common_kmax(b)) return;
+  if (!b->P.lcoulomb || !common_kmax(b)) return;
   if (!b->gp) {
     std::vector<grid::Seg> segs(b->bc_h.size());
     for (size_t c = 0; c < segs.size(); ++c) {
@@ -927,6 +1078,10 @@ void grid_state(mdffgpu_batch* b) {
     }
     b->gp = grid::create(b->st, segs, b->bc_h[0].kmax, !b->mixed);
     if (!b->gp) bfail(b, MDFFGPU_ERR_ALLOC, "reciprocal-space grid");
+    b->grid_calls = !b->mixed || grid::points(b->gp) * segs.size() <= GRID_POINTS;
+    balloc(b, &b->d_adj, 4 * (size_t)b->N);
+    balloc(b, &b->d_v, 3 * (size_t)b->N);
+    balloc(b, &b->d_w, (size_t)b->N);
     balloc(b, &b->d_apart, 9 * (size_t)b->N);
     BCK(b, hipMemsetAsync(b->d_apart, 0, 9 * (size_t)b->N * sizeof(double), b->st));
   }
@@ -992,7 +1147,7 @@ void es_call(mdffgpu_batch* b, int mode, const double* q, const double* mu, cons
   launch_check(b, "batch real space");
   const int chg = (mode != ES_IND) ? 1 : 0;
   const int dip = (mode != ES_STATIC && b->pim) ? 1 : 0;
-  if (b->gp) {
+  if (b->grid_calls) {
     // the induced dipoles sit on the polarizable atoms, where alone the
     // static and SCF calls' field is read
     grid::sums(b->gp, nullptr, b->st, q, mu, chg, dip, mode == ES_FINAL, mode == ES_IND,
@@ -1086,6 +1241,60 @@ int forward(mdffgpu_batch* b, int iters, double* rmsd) {
   return n_scf;
 }
 
+// Gradients of the charges, polarizabilities and damping b (slot ..) by one
+// reverse solve: g . dF/dtheta = v . dmu/dtheta + w . dq/dtheta, and the
+// dipole tangent of any parameter is dmu = sum_k (alpha T)^k alpha S of its
+// field source S, a symmetric operator, so that v . dmu = S . lam with lam the
+// same sum applied to v.  Two SCF solves in all (the forward one and this)
+// instead of one more per parameter with two force evaluations each: with
+// four parameters 19.4 -> 8.2 ms per loss and gradient of 64 configurations in
+// mixed precision, 10.4 -> 4.2 ms of 12 in FP64.  The factor 2 is halved again on the host (the tangents' slots hold twice the
+// gradient).
+template <typename R>
+void reverse(mdffgpu_batch* b, int n_scf, int slot) {
+  const int N = b->N;
+  const size_t n3 = 3 * (size_t)N;
+  const int gb = nblk(N), gbl = nblk((size_t)N * LPA);
+  const mdffgpu_params& P = b->P;
+  // the U, V sums that the forward pass's final call left
+  const double* ap = b->grid_calls ? b->d_apart : mdff::mixed::batch_sums(b->mx);
+  k_b_rev_dir<R><<<gbl, MDFF_BLOCK, 0, b->st>>>(es_args(b, b->d_q, b->d_mu), b->pim ? 1 : 0,
+                                                b->d_g, b->d_v, b->d_w);
+  grid::adjoint_sums(b->gp, b->st, b->d_q, b->d_mu, b->d_g, b->d_adj);
+  k_b_rev_fields<<<gb, MDFF_BLOCK, 0, b->st>>>(N, b->d_cfg, b->d_bc, P.coul_unit, ap, b->d_adj,
+                                               b->d_g, b->d_v, b->d_w);
+  launch_check(b, "batch reverse fields");
+  double rms;
+  double* lam = b->d_dmu;
+  if (b->pim) jacobi<R>(b, b->d_v, lam, b->d_Et, n_scf, &rms);
+  auto dot = [&](const double* S, const double* w, int a) {
+    k_b_rev_dot<<<gb, MDFF_BLOCK, 0, b->st>>>(N, 2.0, S, lam, w, b->d_typ, a, b->d_part);
+    reduce(b, 1, gb, slot++);
+  };
+  for (int a = 0; a < b->ntype; ++a) {
+    if (b->pim) {
+      k_b_qsrc<<<gb, MDFF_BLOCK, 0, b->st>>>(N, b->d_typ, a, b->d_q, b->d_qsrc, b->d_qp, b->d_qm);
+      es_call<R>(b, ES_STATIC, b->d_qsrc, b->d_zero, nullptr, b->d_S);
+    }
+    dot(b->pim ? b->d_S : nullptr, b->d_w, a);
+  }
+  for (int m = 0; m < b->npol; ++m) {
+    k_b_asrc<<<gb, MDFF_BLOCK, 0, b->st>>>(N, b->d_typ, b->pol_type[m], b->pol_alpha[m], b->d_mu,
+                                           b->d_S);
+    dot(b->d_S, nullptr, 0);
+  }
+  if (b->ndamp > 0) {
+    // explicit derivatives of the static field and the final force after the
+    // parameter slots, 1 + nparam ..
+    k_b_damp_adj<<<gbl, MDFF_BLOCK, 0, b->st>>>(es_args(b, b->d_q, b->d_mu), b->dslots, b->d_g,
+                                                P.coul_unit, b->ndamp, b->d_dEs, b->d_part);
+    launch_check(b, "batch damping adjoint");
+    reduce(b, b->ndamp, gbl, 1 + b->nparam);
+    for (int m = 0; m < b->ndamp; ++m) dot(b->d_dEs + (size_t)m * n3, nullptr, 0);
+  }
+  launch_check(b, "batch reverse pass");
+}
+
 // Backward pass after forward(): loss and gradient into d_out[0 ..].
 //   d_out[0]                   loss
 //   d_out[1 + NSR p + k]       BMHFTD parameter k of unordered pair p
@@ -1121,6 +1330,10 @@ void backward(mdffgpu_batch* b, int n_scf) {
   double rms;
   if (!P.lcoulomb) {
     fill(b, b->d_out + slot, b->ntype + b->npol + 2 * b->ndamp, 0.0);
+    return;
+  }
+  if (b->gp && (b->grid_calls || mx_state(b))) {
+    reverse<R>(b, n_scf, slot);
     return;
   }
   for (int a = 0; a < b->ntype; ++a, ++slot) {
@@ -1502,7 +1715,7 @@ void set_positions_impl(mdffgpu_batch* b, const double* d_pos) {
   b->positions_set = true;
   ++b->epoch;
   grid_state(b);
-  if (b->mixed && !b->gp) mx_state(b);  // allocates: never first inside a graph capture
+  if (b->mixed && !b->grid_calls) mx_state(b);  // allocates: never first inside a graph capture
   if (b->gexec) {
     (void)hipGraphExecDestroy(b->gexec);
     b->gexec = nullptr;
@@ -1700,6 +1913,9 @@ int mdffgpu_batch_set_tuning(mdffgpu_batch* b, int32_t apply_lanes) {
 
 int mdffgpu_batch_set_mixed_tuning(mdffgpu_batch* b, int32_t apply_slices, int32_t split_atoms) {
   if (!b) return MDFFGPU_ERR_ARG;
+  // the grid sums have no such launch shape
+  if (b->mixed && b->grid_calls)
+    return mdff::mixed::valid_tuning(apply_slices, split_atoms) ? MDFFGPU_OK : MDFFGPU_ERR_ARG;
   if (!b->mx) return MDFFGPU_ERR_UNSUPPORTED;
   if (b->gexec) {
     (void)hipGraphExecDestroy(b->gexec);

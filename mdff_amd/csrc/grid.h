@@ -69,5 +69,14 @@ int sums(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q, const doubl
          bool dip, bool second, bool src_active, bool dst_active, double* out, double* pout,
          const CombineArgs* ind = nullptr);
 
+// Potentials of the displaced sources, d/de at r_j + e g_j of all atoms (g SoA
+// of stride n): out rows U1 U2 U3 as above and, row 3, psi = sum over every k
+// of A_k S e^{-ikr}.
+void adjoint_sums(Plan* p, hipStream_t st, const double* q, const double* mu, const double* g,
+                  double* out);
+
+// Points of one configuration's grid.
+size_t points(const Plan* p);
+
 }  // namespace grid
 }  // namespace mdff

@@ -633,6 +633,94 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_spread(
     g[(size_t)(x0 + Mat<R>::row(lane, i)) * e.M[1] * e.M[2]] = acc[i];
 }
 
+// The sources of the displaced moments, d/de of q_j, mu_j at r_j + e g_j: dipoles
+// q g and quadrupoles g mu,
+//   G = sum_j (g . d/dr_j)(q_j + mu_j . d/dr_j) prod phi,
+// as k_grid_spread with three terms per atom (phi_x, phi'_x, phi''_x) of the
+// four of a matrix step.  Once per gradient evaluation: not pipelined.
+template <typename R>
+__global__ __launch_bounds__(MDFF_BLOCK) void k_grid_spread_adj(
+    Ext e, const Seg* __restrict__ segs, const double* __restrict__ q,
+    const double* __restrict__ mu, const double* __restrict__ gv, int n,
+    const R* __restrict__ tab, const R* __restrict__ tab2, const int2* __restrict__ list,
+    const int2* __restrict__ cnt, int cap, R* __restrict__ G) {
+  constexpr int W = Mat<R>::W;
+  typedef typename Mat<R>::acc acc_t;
+  __shared__ R lx[SCH][3][TX], ly[SCH][3][TY], lz[SCH][3][TZ];
+  // per x term the coefficients of f f, f' f, f f', f'' f, f f'', f' f' in (y, z)
+  __shared__ R co[SCH][4][6];
+  const int tile = xcd_tile(blockIdx.x, e.ntile), seg = blockIdx.y;
+  if (tile >= e.ntile) return;
+  const size_t at = (size_t)seg * e.ntile + tile;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int m = cnt[at].y;
+  const int2* lst = list + at * cap;
+  const int z0 = (tile % e.nt[2]) * TZ, y0 = ((tile / e.nt[2]) % e.nt[1]) * TY,
+            x0 = tile / (e.nt[2] * e.nt[1]) * TX;
+  const Cell& cell = segs[seg].cell;
+  const int al = t >> 3, pp = t & 7;
+  const int row = lane & 15, kk = lane >> 4;
+  const int yy = 2 * wv + (row >> 3), zz = row & 7;
+  acc_t acc = {0, 0, 0, 0};
+  for (int c0 = 0; c0 < m; c0 += SCH) {
+    const bool in = c0 + al < m;
+    const int2 en = lst[min(c0 + al, m - 1)];
+    const int i = en.x;
+    const R* T = tab + (size_t)i * 6 * W;
+    const R* T2 = tab2 + (size_t)i * 3 * W;
+    const int o[3] = {(en.y & 255) - 64, (en.y >> 8 & 255) - 64, (en.y >> 16 & 255) - 64};
+    auto point = [&](int ax, int p, R* f, int stride) {
+      int d = p - o[ax];
+      d += d < 0 ? e.M[ax] : 0;
+      const R on = in && d < W ? R(1) : R(0);
+      d = min(d, W - 1);
+      f[0] = on * T[2 * ax * W + d];
+      f[stride] = on * T[(2 * ax + 1) * W + d];
+      f[2 * stride] = on * T2[ax * W + d];
+    };
+    point(0, pp, &lx[al][0][pp], TX);
+    point(0, pp + 8, &lx[al][0][pp + 8], TX);
+    point(1, pp, &ly[al][0][pp], TY);
+    point(2, pp, &lz[al][0][pp], TZ);
+    if (pp == 0) {
+      double gg[3], mm[3];
+      for (int a = 0; a < 3; ++a) {
+        const double* b = cell.B + 3 * a;
+        gg[a] = e.M[a] * (b[0] * gv[i] + b[1] * gv[i + n] + b[2] * gv[i + 2 * (size_t)n]);
+        mm[a] = e.M[a] * (b[0] * mu[i] + b[1] * mu[i + n] + b[2] * mu[i + 2 * (size_t)n]);
+      }
+      const double qi = q[i];
+      R(*c)[6] = co[al];
+      for (int k = 0; k < 4; ++k)
+        for (int j = 0; j < 6; ++j) c[k][j] = R(0);
+      c[0][1] = (R)(qi * gg[1]);
+      c[0][2] = (R)(qi * gg[2]);
+      c[0][3] = (R)(gg[1] * mm[1]);
+      c[0][4] = (R)(gg[2] * mm[2]);
+      c[0][5] = (R)(gg[1] * mm[2] + gg[2] * mm[1]);
+      c[1][0] = (R)(qi * gg[0]);
+      c[1][1] = (R)(gg[0] * mm[1] + gg[1] * mm[0]);
+      c[1][2] = (R)(gg[0] * mm[2] + gg[2] * mm[0]);
+      c[2][0] = (R)(gg[0] * mm[0]);
+    }
+    __syncthreads();
+    const int left = min(SCH, m - c0);
+    for (int a = 0; a < left; ++a) {
+      const R* c = co[a][kk];
+      const R f = ly[a][0][yy], f1 = ly[a][1][yy], f2 = ly[a][2][yy];
+      const R h = lz[a][0][zz], h1 = lz[a][1][zz], h2 = lz[a][2][zz];
+      const R b = c[0] * f * h + c[1] * f1 * h + c[2] * f * h1 + c[3] * f2 * h + c[4] * f * h2 +
+                  c[5] * f1 * h1;
+      acc = Mat<R>::mma(lx[a][min(kk, 2)][row], b, acc);
+    }
+    __syncthreads();
+  }
+  R* g = G + (size_t)seg * e.ng + (size_t)(y0 + yy) * e.M[2] + z0 + zz;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    g[(size_t)(x0 + Mat<R>::row(lane, i)) * e.M[1] * e.M[2]] = acc[i];
+}
+
 // ---------------------------------------------------------------------------
 // transforms (FP64 matrix cores)
 
@@ -1024,14 +1112,15 @@ __device__ __forceinline__ R wave_total(R x) {
 // k_combine64<ES_IND> is formed here too, with the block partials of its
 // residual (or p.Ap) rows in ca.rpart: 15 and 62 us, against 5.6 us more in a
 // launch of its own.
-template <typename R, bool SECOND, bool IND, int BA>
+// VAL: also the potential psi itself, in row 3.
+template <typename R, bool SECOND, bool IND, int BA, bool VAL = false>
 __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_gather(
     Ext e, const R* __restrict__ P, const int4* __restrict__ l0, const R* __restrict__ tab,
     const R* __restrict__ tab2, const int* __restrict__ perm, const int* __restrict__ cfg,
     int count, int apw, int n, double* __restrict__ out, CombineArgs ca) {
   constexpr int W = Mat<R>::W, ZV = Mat<R>::ZV, NG = (W + ZV - 1) / ZV;
   constexpr int IT = (W * NG + 63) / 64;
-  constexpr int NV = SECOND ? 9 : 3;
+  constexpr int NV = SECOND ? 9 : VAL ? 4 : 3;
   __shared__ double red[2][4];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int per = 4 * apw;
@@ -1126,6 +1215,7 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_gather(
           v[j][0] += s1 * (fy[j] * fz[j][z]);
           v[j][1] += s0 * (gy[j] * fz[j][z]);
           v[j][2] += s0 * (fy[j] * gz[j][z]);
+          if (VAL) v[j][3] += s0 * (fy[j] * fz[j][z]);
           if (SECOND) {
             v[j][3] += s2 * (fy[j] * fz[j][z]);
             v[j][4] += s0 * (hy[j] * fz[j][z]);
@@ -1182,6 +1272,7 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_gather(
       r[0] = u0;
       r[N] = u1;
       r[2 * N] = u2;
+      if (VAL) r[3 * N] = (double)w[3];
       if (SECOND) {
         r[3 * N] = c2 * Mx * Mx * (double)w[3];
         r[4 * N] = c2 * My * My * (double)w[4];
@@ -1382,6 +1473,7 @@ void set_cells(Plan* p, hipStream_t st, const std::vector<Seg>& segs) {
                                            p->d_D);
 }
 
+size_t points(const Plan* p) { return p->e.ng; }
 bool binned(const Plan* p) { return p->is_binned; }
 void unbin(Plan* p) { p->is_binned = false; }
 
@@ -1461,34 +1553,15 @@ void prepare(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double4* s4) {
   }
 }
 
+// Spread grids to potentials: the three transform kernels.
 template <typename R>
-static int sums_t(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,
-                  const double* mu, bool chg, bool dip, bool second, bool src_active, bool dst_active,
-                  double* out, double* pout, const CombineArgs* ind) {
-  const Ext& e = p->e;
-  const int n = p->natom;
-  R* G = static_cast<R*>(p->d_G);
-  R* P = static_cast<R*>(p->d_P);
-  const R* tab = static_cast<const R*>(p->d_tab);
-  const R* tab2 = static_cast<const R*>(p->d_tab2);
-  const dim3 gt(xcd_blocks(e.ntile), e.nseg, p->split);
-  const int sa = src_active ? 1 : 0;
-  {
-  ProfScope _ps(ctx, K_GRID_SPREAD);
-  if (chg && dip)
-    k_grid_spread<R, true, true><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
-                                                            p->d_cnt, p->cap, sa, G);
-  else if (dip)
-    k_grid_spread<R, false, true><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
-                                                             p->d_cnt, p->cap, sa, G);
-  else
-    k_grid_spread<R, true, false><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
-                                                             p->d_cnt, p->cap, sa, G);
-  }
-  {
+static void convolve(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, int split, double* pout) {
   ProfScope _ps(ctx, K_GRID_FT);
+  const Ext& e = p->e;
+  const R* G = static_cast<const R*>(p->d_G);
+  R* P = static_cast<R*>(p->d_P);
   const dim3 gf(e.M[0], (e.N3c + 15) / 16, e.nseg);
-  k_grid_fwd<R><<<gf, MDFF_BLOCK, lds_fwd(e), st>>>(e, p->tw, p->split, G, p->d_T);
+  k_grid_fwd<R><<<gf, MDFF_BLOCK, lds_fwd(e), st>>>(e, p->tw, split, G, p->d_T);
   const dim3 gm((e.NCC + 7) / 8, e.nseg);
   EnArgs en;
   std::memset(&en, 0, sizeof(en));
@@ -1502,7 +1575,33 @@ static int sums_t(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,
   }
   const dim3 gi(e.M[0], (e.M[1] / 2 + 15) / 16, e.nseg);
   k_grid_inv<R><<<gi, MDFF_BLOCK, lds_inv(e), st>>>(e, p->tw, p->d_T, P);
+}
+
+template <typename R>
+static int sums_t(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,
+                  const double* mu, bool chg, bool dip, bool second, bool src_active, bool dst_active,
+                  double* out, double* pout, const CombineArgs* ind) {
+  const Ext& e = p->e;
+  const int n = p->natom;
+  R* G = static_cast<R*>(p->d_G);
+  const R* P = static_cast<const R*>(p->d_P);
+  const R* tab = static_cast<const R*>(p->d_tab);
+  const R* tab2 = static_cast<const R*>(p->d_tab2);
+  const dim3 gt(xcd_blocks(e.ntile), e.nseg, p->split);
+  const int sa = src_active ? 1 : 0;
+  {
+    ProfScope _ps(ctx, K_GRID_SPREAD);
+    if (chg && dip)
+    k_grid_spread<R, true, true><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
+                                                            p->d_cnt, p->cap, sa, G);
+  else if (dip)
+    k_grid_spread<R, false, true><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
+                                                             p->d_cnt, p->cap, sa, G);
+  else
+    k_grid_spread<R, true, false><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
+                                                             p->d_cnt, p->cap, sa, G);
   }
+  convolve<R>(p, ctx, st, p->split, pout);
   ProfScope _ps(ctx, K_GRID_GATHER);
   const int count = dst_active ? p->nact : n;
   // about 4096 waves of a large system take the atoms in turn
@@ -1538,6 +1637,30 @@ int sums(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,
          const CombineArgs* ind) {
   return p->fp64 ? sums_t<double>(p, ctx, st, q, mu, chg, dip, second, src_active, dst_active, out, pout, ind)
                  : sums_t<float>(p, ctx, st, q, mu, chg, dip, second, src_active, dst_active, out, pout, ind);
+}
+
+template <typename R>
+static void adjoint_t(Plan* p, hipStream_t st, const double* q, const double* mu, const double* g,
+                      double* out) {
+  const Ext& e = p->e;
+  const int n = p->natom;
+  const R* tab = static_cast<const R*>(p->d_tab);
+  const R* tab2 = static_cast<const R*>(p->d_tab2);
+  k_grid_spread_adj<R><<<dim3(xcd_blocks(e.ntile), e.nseg), MDFF_BLOCK, 0, st>>>(
+      e, p->d_seg, q, mu, g, n, tab, tab2, p->d_ov, p->d_cnt, p->cap, static_cast<R*>(p->d_G));
+  convolve<R>(p, nullptr, st, 1, nullptr);
+  CombineArgs ca;
+  std::memset(&ca, 0, sizeof(ca));
+  k_grid_gather<R, false, false, 1, true><<<xcd_blocks((n + 3) / 4), MDFF_BLOCK, 0, st>>>(
+      e, static_cast<const R*>(p->d_P), p->d_l0, tab, tab2, p->d_perm, p->cfg, n, 1, n, out, ca);
+}
+
+void adjoint_sums(Plan* p, hipStream_t st, const double* q, const double* mu, const double* g,
+                  double* out) {
+  if (p->fp64)
+    adjoint_t<double>(p, st, q, mu, g, out);
+  else
+    adjoint_t<float>(p, st, q, mu, g, out);
 }
 
 }  // namespace grid

@@ -102,6 +102,8 @@ bool set_tuning(MixedState* m, int app_slices, int split_atoms);
 void kspace_batch(MixedState* m, hipStream_t st, const double* s, long long epoch,
                   const int* cfg, const double* q, const double* mu, bool chg, bool dip,
                   bool force, double* Erec, double* Frec);
+// The U, V sums (9 rows of N) the last kspace_batch call with force left.
+const double* batch_sums(const MixedState* m);
 
 }  // namespace mixed
 }  // namespace mdff

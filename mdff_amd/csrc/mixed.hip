@@ -2077,6 +2077,8 @@ float* dipole_weights(MixedState* m, int* npad) {
   return m->d_seg ? nullptr : m->Wt;  // a batch has its own slot layout
 }
 
+const double* batch_sums(const MixedState* m) { return m->apart; }
+
 void kspace_batch(MixedState* m, hipStream_t st, const double* s, long long epoch,
                   const int* cfg, const double* q, const double* mu, bool chg, bool dip,
                   bool force, double* Erec, double* Frec) {

@@ -95,3 +95,39 @@ def test_grid_batch_matches_oracle(oracle_lib):
             g = f[:, b.offsets[c]:b.offsets[c + 1]].T
             assert np.abs(g - o["f"]).max() <= 1e-10 * np.abs(o["f"]).max(), (kmaxes[c], c)
         b.close()
+
+
+@pytest.mark.parametrize("precision", [P.PREC_FP64, P.PREC_MIXED])
+def test_reverse_gradient_matches_tangents(precision):
+    """The reverse solve (configurations with one kmax) against the tangent
+    solves, which a batch takes whose kmax differ: the same configurations
+    with one more whose kmax is another, subtracted out by its own batch.
+    The sums differ by the rounding of the forces (FP64 1e-14, FP32 1e-6) of
+    gradients whose terms cancel to a tenth."""
+    import torch
+    from mdff_amd.batch import Batch, get_theta
+    systems = [C.silica(n, 2 * n, seed=60 + n, rc=4.5, kmax=4, pim=True, scf_tol=1e-12,
+                        pot_seed=9) for n in (17, 30, 16)]
+    systems[2].params.kES[:] = [5, 4, 4]
+    rng = np.random.default_rng(4)
+
+    def grads(group):
+        b = Batch.from_systems(group, precision=precision)
+        b.set_positions(torch.tensor(np.concatenate([s.r for s in group]).T.copy(), device="cuda"))
+        n = b.natm
+        target = torch.tensor(np.concatenate([tgt[id(s)] for s in group]).T.copy(), device="cuda")
+        loss, grad = b.loss_grad(target, 25)
+        assert len(get_theta(b.model)) == len(grad)
+        b.close()
+        return 3 * n * loss, 3 * n * grad
+
+    tgt = {id(s): 10.0 * rng.standard_normal(s.r.shape) for s in systems}
+    l3, g3 = grads(systems)  # tangents: the kmax differ
+    l2, g2 = grads(systems[:2])  # reverse
+    l1, g1 = grads(systems[2:])
+    tol = 1e-10 if precision == P.PREC_FP64 else 2e-5
+    assert abs(l1 + l2 - l3) <= tol * l3
+    assert np.abs(g1 + g2 - g3).max() <= tol * np.abs(g3).max(), (g1 + g2, g3)
+    # the electrostatic parameters, several orders smaller, on their own scale
+    e = np.abs((g1 + g2 - g3)[-4:]).max()
+    assert e <= 10 * tol * np.abs(g3[-4:]).max(), (g1 + g2, g3)
