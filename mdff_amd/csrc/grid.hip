@@ -1169,7 +1169,7 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_gather(
 #pragma unroll
       for (int c = 0; c < NV; ++c) v[j][c] = R(0);
     // not unrolled at W = 17: five passes' loads would leave two waves per SIMD
-#pragma unroll (IT > 2 ? 1 : IT)
+#pragma unroll IT > 2 ? 1 : IT
     for (int it = 0; it < IT; ++it) {
       const int c = lane + 64 * it;
       const bool in = c < W * NG;

@@ -265,6 +265,10 @@ struct NhcMass {
 };
 __global__ void k_vv_pos(MdArgs a);
 __global__ void k_vv_vel(MdArgs a);
+__global__ void k_vv_step(MdArgs a, int vel, int adv, Cell cell, const int* ext, const int* typ,
+                          const double* ref, double* s, double4* s4, double* dmax);
+__global__ void k_md_reduce(const double* sr, int nsr, int nsb, int sr0, const double* kin, int nb,
+                            int kin0, const double* dmax, int d0, double* out, double* out2);
 __global__ void k_kick_drift(MdArgs a);
 __global__ void k_kick(MdArgs a);
 __global__ void k_vscale(MdArgs a, const NhcState* s);

@@ -29,6 +29,7 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_prepare(
   // compare it) + its species (s4_type)
   const long long w = 16ll * (ext ? ext[i] : i) + typ[i];
   s4[i] = make_double4(s1, s2, s3, (double)w);
+  if (!eph) return;  // phases of the direct reciprocal sums
   double sn, cs;
   sincospi(2.0 * s1, &sn, &cs);
   eph[i] = make_double2(cs, sn);

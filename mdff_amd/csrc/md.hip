@@ -54,6 +54,98 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_vv_vel(MdArgs a) {
   kin_partial(mv2, a.part);
 }
 
+// One launch between two force evaluations of a velocity Verlet run: the
+// second half of a step (vel: k_vv_vel), then the first half of the next (adv:
+// k_vv_pos) with its fractional coordinates (k_prepare) and the block maxima of
+// the squared displacements since the last list build (k_disp).  All per
+// atom; 4 us against 3 + 3 + 3 + 2 us and their launches.
+__global__ __launch_bounds__(MDFF_BLOCK) void k_vv_step(MdArgs a, int vel, int adv, Cell cell,
+                                                        const int* __restrict__ ext,
+                                                        const int* __restrict__ typ,
+                                                        const double* __restrict__ ref,
+                                                        double* __restrict__ s,
+                                                        double4* __restrict__ s4,
+                                                        double* __restrict__ dmax) {
+  __shared__ double red[MDFF_BLOCK / 64];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  double mv2 = 0.0, d2 = 0.0;
+  if (i < a.n) {
+    const double m = a.mass[i];
+    double v[3], p[3], f[3];
+    for (int c = 0; c < 3; ++c) {
+      const size_t k = i + (size_t)c * a.n;
+      f[c] = a.f[k];
+      v[c] = a.vel[k];
+      if (vel) {
+        v[c] = v[c] + (a.fs[k] + f[c]) * a.dt2 / m;
+        a.vel[k] = v[c];
+      }
+      if (adv) {
+        a.fs[k] = f[c];
+        p[c] = a.pos[k] + v[c] * a.dt + (f[c] * a.dtsq2) / m;
+        a.pos[k] = p[c];
+      }
+    }
+    mv2 = (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) * m;
+    if (adv) {
+      const double* B = cell.B;
+      double q[3];
+      for (int c = 0; c < 3; ++c) {
+        q[c] = p[0] * B[3 * c] + p[1] * B[3 * c + 1] + p[2] * B[3 * c + 2];
+        s[i + (size_t)c * a.n] = q[c];
+        const double d = p[c] - ref[i + (size_t)c * a.n];
+        d2 = c == 0 ? d * d : d2 + d * d;
+      }
+      s4[i] = make_double4(q[0], q[1], q[2], (double)(16ll * (ext ? ext[i] : i) + typ[i]));
+    }
+  }
+  if (vel) kin_partial(mv2, a.part);
+  if (adv) {
+    for (int off = 32; off > 0; off >>= 1) d2 = fmax(d2, __shfl_down(d2, off, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = d2;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double m = 0.0;
+      for (int w = 0; w < MDFF_BLOCK / 64; ++w) m = fmax(m, red[w]);
+      dmax[blockIdx.x] = m;
+    }
+  }
+}
+
+// The sums of a step into device scalars and mapped host memory in one
+// launch: nsr rows of pair partials (sr, nsb per row) to slot sr0, the kinetic
+// partials (kin) to slot kin0 and the maximum of dmax to slot d0; blocks
+// without a source (null) write nothing.  Sums in k_reduce_rows' order.
+__global__ __launch_bounds__(MDFF_BLOCK) void k_md_reduce(const double* __restrict__ sr, int nsr,
+                                                          int nsb, int sr0,
+                                                          const double* __restrict__ kin, int nb,
+                                                          int kin0,
+                                                          const double* __restrict__ dmax, int d0,
+                                                          double* __restrict__ out, double* out2) {
+  __shared__ double red[4];
+  const int r = blockIdx.x;
+  const bool is_max = r == nsr + 1;
+  const double* src = r < nsr ? (sr ? sr + (size_t)r * nsb : nullptr) : is_max ? dmax : kin;
+  if (!src) return;
+  const int len = r < nsr ? nsb : nb;
+  double acc[1] = {0.0};
+  if (is_max) {
+    for (int b = threadIdx.x; b < len; b += blockDim.x) acc[0] = fmax(acc[0], src[b]);
+    for (int off = 32; off > 0; off >>= 1) acc[0] = fmax(acc[0], __shfl_down(acc[0], off, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc[0];
+    __syncthreads();
+    acc[0] = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+  } else {
+    for (int b = threadIdx.x; b < len; b += blockDim.x) acc[0] += src[b];
+    block_sum<1>(acc, red);
+  }
+  if (threadIdx.x == 0) {
+    const int slot = r < nsr ? sr0 + r : is_max ? d0 : kin0;
+    out[slot] = acc[0];
+    out2[slot] = acc[0];
+  }
+}
+
 // prop_pos_vel_verlet, first half: v += f dt2 / m; r += v dt
 __global__ __launch_bounds__(MDFF_BLOCK) void k_kick_drift(MdArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;

@@ -127,3 +127,30 @@ def test_cell_list_small_box_falls_back(oracle_lib):
     info = ff.list_info()
     ff.close()
     assert not info["cell_search"]
+
+
+@pytest.mark.parametrize("ncell,chunks", [(4, 1), (4, 6), (7, 2)])
+def test_nve_vv_pairs_rebuilds(oracle_lib, ncell, chunks):
+    """Pair-force steps (one fused launch between force evaluations) in one
+    or many calls (the last step of a call without the next one's positions),
+    fast enough that the skin is crossed inside and between them; atoms in
+    one partial block and a ragged last one."""
+    s = C.lj_fcc(ncell)
+    s.r = s.r + 0.03 * np.random.default_rng(8).standard_normal(s.r.shape)
+    v0 = C.maxwell_velocities(s, 40.0, seed=3)
+    mdp = P.md_params("nve-vv", dt=0.002, mass=(1.0,), lreduced=True)
+    gs, os_, g, o, _, info = _md_both(oracle_lib, s, mdp, v0, 12, chunks)
+    assert info["builds"] >= 2
+    _check(gs, os_, g, o, ("u_lj", "vir_lj", "e_kin", "temp_r", "tau_nonb"))
+
+
+def test_nve_vv_pairs_bmhftd(oracle_lib):
+    """The same steps with the species pairs of a melt without charges (two
+    masses, renumbered atoms)."""
+    s = C.silica(100, 200, seed=12, pim=False, dmin=2.0)
+    s.params.lcoulomb = 0
+    m = C.species_masses(s)
+    v0 = C.maxwell_velocities(s, 2000.0, seed=4)
+    mdp = P.md_params("nve-vv", dt=0.0005, mass=m)
+    gs, os_, g, o, _, _ = _md_both(oracle_lib, s, mdp, v0, 6, 2)
+    _check(gs, os_, g, o, ("u_bmhft", "e_kin", "temp_r", "tau_nonb"))
