@@ -1098,7 +1098,6 @@ void grid_state(mdffgpu_batch* b) {
 template <typename R>
 void es_call(mdffgpu_batch* b, int mode, const double* q, const double* mu, const double* S,
              double* out) {
-  using R4 = typename std::conditional<sizeof(R) == sizeof(double), double4, float4>::type;
   const int N = b->N;
   const int gbl = nblk((size_t)N * LPA);
   EsDirArgs da = es_args(b, q, mu);
@@ -1108,13 +1107,16 @@ void es_call(mdffgpu_batch* b, int mode, const double* q, const double* mu, cons
     k_es_dir<ES_STATIC, R, true><<<gbl, MDFF_BLOCK, 0, b->st>>>(da);
   } else if (mode == ES_IND) {
     da.ef = b->d_dir;
-    R4* m4 = reinterpret_cast<R4*>(b->d_mu4);
-    k_pack_mu<R4><<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, mu, m4);
+    const size_t cap = (size_t)b->maxnb * N;
     if constexpr (sizeof(R) == sizeof(double)) {
-      k_dd_field<<<nblk((size_t)N * DD_LANES), MDFF_BLOCK, 0, b->st>>>(da, (const double*)b->d_t2,
-                                                                     m4);
+      double2* smu = reinterpret_cast<double2*>(b->d_t2);
+      const double2* tab = smu + 3 * (size_t)N;
+      k_pack_smu<<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, b->d_s4, mu, nullptr, smu);
+      dd_tab64_launch(b->st, N, b->maxnb, tab, reinterpret_cast<const int*>(tab + cap), smu, Cell{},
+                      b->d_bc, b->d_cfg, nullptr, b->d_polrows, b->npolrows, b->d_dir);
     } else {
-      const size_t cap = (size_t)b->maxnb * N;
+      float4* m4 = reinterpret_cast<float4*>(b->d_mu4);
+      k_pack_mu<float4><<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, mu, m4);
       const uint4* u4 = reinterpret_cast<const uint4*>(b->d_t2);
       const float2* tab = reinterpret_cast<const float2*>(u4 + N);
       const int* tj = reinterpret_cast<const int*>(tab + cap);
@@ -1647,12 +1649,13 @@ void create_impl(const mdffgpu_params* model, int nconf, const mdffgpu_batch_con
 template <typename R>
 void build_pairs(mdffgpu_batch* b) {
   EsDirArgs da = es_args(b, b->d_q, b->d_zero);
-  // FP64: five doubles per list entry; FP32: the fixed-point positions
-  // (uint4 per atom), compacted (A2, A1) float2 + index per entry, then the
-  // per-atom counts
+  // FP64: positions and dipoles (three double2 per atom), FP32: the
+  // fixed-point positions (uint4 per atom); then compacted (A2, A1) + index
+  // per entry and the per-atom counts
   const size_t cap = (size_t)b->maxnb * b->N;
   const size_t need = sizeof(R) == sizeof(double)
-                          ? 5 * cap * sizeof(double)
+                          ? 3 * (size_t)b->N * sizeof(double2) +
+                                cap * (sizeof(double2) + sizeof(int)) + (size_t)b->N * sizeof(int)
                           : (size_t)b->N * sizeof(uint4) + cap * (sizeof(float2) + sizeof(int)) +
                                 (size_t)b->N * sizeof(int);
   if (need > b->t2_cap) {
@@ -1665,18 +1668,21 @@ void build_pairs(mdffgpu_batch* b) {
     b->allocs.push_back(b->d_t2);
     b->t2_cap = need;
   }
+  da.dd16 = dd_idx16(b->N);
   if constexpr (sizeof(R) == sizeof(double)) {
-    k_pairs_t2<true><<<nblk((size_t)b->N * LPA), MDFF_BLOCK, 0, b->st>>>(da, (double*)b->d_t2);
+    double2* tab = reinterpret_cast<double2*>(b->d_t2) + 3 * (size_t)b->N;
+    int* tj = reinterpret_cast<int*>(tab + cap);
+    k_dd_table<true, double><<<nblk((size_t)b->N * 64), MDFF_BLOCK, 0, b->st>>>(da, b->polmask, tab,
+                                                                                tj, tj + cap);
   } else {
     uint4* u4 = reinterpret_cast<uint4*>(b->d_t2);
     float2* tab = reinterpret_cast<float2*>(u4 + b->N);
     int* tj = reinterpret_cast<int*>(tab + cap);
-    da.dd16 = dd_idx16(b->N);
     // fractional coordinates in each configuration's own cell: the fixed-
     // point difference is that cell's minimum image
     k_pack_u4<<<nblk(b->N), MDFF_BLOCK, 0, b->st>>>(b->N, b->d_s, nullptr, u4);
-    k_dd_table<true><<<nblk((size_t)b->N * 64), MDFF_BLOCK, 0, b->st>>>(da, tab, tj,
-                                                                                tj + cap);
+    k_dd_table<true, float><<<nblk((size_t)b->N * 64), MDFF_BLOCK, 0, b->st>>>(da, b->polmask, tab,
+                                                                               tj, tj + cap);
   }
   launch_check(b, "batch pair table");
 }

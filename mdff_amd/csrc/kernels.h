@@ -13,7 +13,7 @@ namespace mdff {
 constexpr int KC_MAX = 16;      // k vectors per chunk (consecutive n3)
 constexpr int RHO_TILE = 32;    // atoms per LDS tile in the structure factor
 constexpr int APPLY_TILE = 64;  // k chunks per LDS tile in the apply
-constexpr int DD_LANES = 64;    // lanes per atom of the SCF dipole field
+constexpr int DD64_U = 3;       // entries per lane and trip of the FP64 SCF dipole field
 
 enum { ES_STATIC = 0, ES_IND = 1, ES_FINAL = 2 };
 enum { SR_LJ = 1, SR_BM = 2, SR_BMD = 4, SR_MO = 8, SR_TRUNC1 = 16, SR_TRUNC2 = 32 };
@@ -281,24 +281,43 @@ template <typename R, bool BATCH = false>
 __global__ void k_shortrange(SrArgs a);
 template <int MODE, typename R, bool BATCH = false>
 __global__ void k_es_dir(EsDirArgs a);
-template <bool BATCH = false>
-__global__ void k_pairs_t2(EsDirArgs a, double* tab);
-__global__ void k_dd_field(EsDirArgs a, const double* tab, const double4* mu4);
 template <typename R4>
 __global__ void k_pack_mu(int n, const double* mu, R4* mu4);
 __global__ void k_pack_mu_ranked(int n, const double* mu, const int* rank, float4* mu4);
 template <typename R4>
 __global__ void k_pack_qmu(int n, const double* q, const double* mu, R4* qm);
-template <bool BATCH>
-__global__ void k_dd_table(EsDirArgs a, float2* tab, int* tj, int* tcnt);
+template <bool BATCH, typename R, typename R2>
+__global__ void k_dd_table(EsDirArgs a, unsigned fieldmask, R2* tab, int* tj, int* tcnt);
+__global__ void k_pack_smu(int n, const double4* s4, const double* mu, const int* rank,
+                           double2* smu);
+template <typename IT>
+__global__ void k_dd_tab64(int n, int maxnb, const double2* tab, const IT* tj, const int* tcnt,
+                           const double2* smu, Cell cell, const BatchCfg* bc, const int* cfg,
+                           const int* perm, const int* rows, int nrows, double* ef);
 __global__ void k_pack_u4(int n, const double* s, const int* rank, uint4* u4);
 template <typename IT, int U>
 __global__ void k_dd_tab2(int n, int maxnb, const float2* tab, const IT* tj, const int* tcnt,
                           const float4* mu4, const uint4* u4, Cell cell, const BatchCfg* bc,
                           const int* cfg, const int* perm, const int* rows, int nrows,
                           double* ef);
-// neighbour slots of the FP32 pair table fit 16 bits
+// neighbour slots of the pair table fit 16 bits
 inline bool dd_idx16(long long n) { return n <= 65536; }
+// k_dd_tab64 over nrows rows of a table of n rows (counts behind the slots).
+inline void dd_tab64_launch(hipStream_t st, int n, int maxnb, const double2* tab, const int* tj,
+                            const double2* smu, const Cell& cell, const BatchCfg* bc,
+                            const int* cfg, const int* perm, const int* rows, int nrows,
+                            double* ef) {
+  if (nrows <= 0) return;
+  const int nb = (int)(((size_t)nrows * 64 + MDFF_BLOCK - 1) / MDFF_BLOCK);
+  const int* cnt = tj + (size_t)maxnb * n;
+  if (dd_idx16(n))
+    k_dd_tab64<unsigned short><<<nb, MDFF_BLOCK, 0, st>>>(
+        n, maxnb, tab, reinterpret_cast<const unsigned short*>(tj), cnt, smu, cell, bc, cfg, perm,
+        rows, nrows, ef);
+  else
+    k_dd_tab64<int><<<nb, MDFF_BLOCK, 0, st>>>(n, maxnb, tab, tj, cnt, smu, cell, bc, cfg, perm,
+                                               rows, nrows, ef);
+}
 // Grid of k_dd_tab2 (persistent waves): four per SIMD of the device, at most
 // one per atom.
 inline int dd_tab_blocks(int n) {

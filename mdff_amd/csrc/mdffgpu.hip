@@ -620,6 +620,14 @@ int* dd_tj(mdffgpu_ctx* c) {
   return reinterpret_cast<int*>(dd_tab(c) + (size_t)c->maxnb * c->n);
 }
 
+// The FP64 one: 48 bytes of position and dipole per slot, the (A2, A1)
+// entries, the neighbour slots, the row counts.
+double2* dd64_smu(mdffgpu_ctx* c) { return reinterpret_cast<double2*>(c->d_t2); }
+double2* dd64_tab(mdffgpu_ctx* c) { return dd64_smu(c) + 3 * (size_t)c->n; }
+int* dd64_tj(mdffgpu_ctx* c) {
+  return reinterpret_cast<int*>(dd64_tab(c) + (size_t)c->maxnb * c->n);
+}
+
 // Entries per lane of k_dd_tab2's pipeline: the expected row of the table
 // (the polarizable neighbours inside the cutoff, from their density) with
 // 15 % to spare, as 4, 6 or 8.
@@ -666,18 +674,13 @@ void es_ind_dir(mdffgpu_ctx* c, const double* mu, bool packed = false) {
     else if (c->npolrows > 0)
       launch_dd_tab2(c, tab, tj, tj + cap, m4);
   } else {
-    EsDirArgs da;
-    std::memset(&da, 0, sizeof(da));
-    da.n = n;
-    da.maxnb = c->maxnb;
-    da.cnt = c->d_cnt;
-    da.nbr = c->d_nbr;
-    da.perm = c->d_perm;
-    da.ef = c->d_efdir;
-    da.typ = c->d_typ;
-    da.polmask = c->fieldmask;
-    k_pack_mu<double4><<<gb, MDFF_BLOCK, 0, st>>>(n, mu, c->d_mu4);
-    k_dd_field<<<nblk(n * DD_LANES), MDFF_BLOCK, 0, st>>>(da, (const double*)c->d_t2, c->d_mu4);
+    // the rows of the polarizable atoms; with quadrupole-polarizable species
+    // the field is read elsewhere too (empty rows give zeros)
+    const bool all = c->fieldmask != c->polmask;
+    k_pack_smu<<<gb, MDFF_BLOCK, 0, st>>>(n, c->d_s4, mu, c->d_rank, dd64_smu(c));
+    dd_tab64_launch(c->st, n, c->maxnb, dd64_tab(c), dd64_tj(c), dd64_smu(c), c->cell,
+                    nullptr, nullptr, c->d_perm, all ? nullptr : c->d_polrows,
+                    all ? n : c->npolrows, c->d_efdir);
   }
   check_launch(c, "k_dd_field");
 }
@@ -990,18 +993,19 @@ void es_call(mdffgpu_ctx* c, int mode, const double* q, const double* mu, int ta
   check_launch(c, "k_combine64");
 }
 
-// Pair table of the SCF dipole field (k_pairs_t2): once per evaluation,
+// Pair table of the SCF dipole field (k_dd_table): once per evaluation,
 // positions are fixed during the SCF.
 void build_t2(mdffgpu_ctx* c) {
   const int n = c->n;
   const bool mx = (c->P.precision == MDFFGPU_PREC_MIXED) &&
                   !(c->P.mixed_fp64_parts & MDFFGPU_MIXED_FP64_SCF_FIELD);
-  // FP64: five doubles per list entry; mixed: the fixed-point positions,
-  // (A2, A1) float2 + index per entry, the per-atom counts
+  // mixed: the fixed-point positions, FP64: positions and dipoles; then
+  // (A2, A1) and index per entry and the per-atom counts
   const size_t cap = (size_t)c->maxnb * n;
   const size_t need = mx ? (size_t)n * sizeof(uint4) + cap * (sizeof(float2) + sizeof(int)) +
                                (size_t)n * sizeof(int)
-                         : 5 * cap * sizeof(double);
+                         : 3 * (size_t)n * sizeof(double2) +
+                               cap * (sizeof(double2) + sizeof(int)) + (size_t)n * sizeof(int);
   if (need > c->t2_cap) {
     char* t2 = static_cast<char*>(c->d_t2);
     dalloc(c, &t2, need);
@@ -1036,13 +1040,14 @@ void build_t2(mdffgpu_ctx* c) {
   ProfScope _ps(c, K_PAIRS_T2);
   if (mx) {
     int* tj = dd_tj(c);
-    k_dd_table<false><<<nblk(n * 64), MDFF_BLOCK, 0, c->st>>>(da, dd_tab(c), tj, tj + cap);
+    k_dd_table<false, float><<<nblk(n * 64), MDFF_BLOCK, 0, c->st>>>(da, c->polmask, dd_tab(c), tj,
+                                                                     tj + cap);
   } else {
-    da.typ = c->d_typ;
-    da.polmask = c->fieldmask;
-    k_pairs_t2<<<nblk(n * LPA), MDFF_BLOCK, 0, c->st>>>(da, (double*)c->d_t2);
+    int* tj = dd64_tj(c);
+    k_dd_table<false, double><<<nblk(n * 64), MDFF_BLOCK, 0, c->st>>>(da, c->fieldmask,
+                                                                      dd64_tab(c), tj, tj + cap);
   }
-  check_launch(c, "k_pairs_t2");
+  check_launch(c, "k_dd_table");
 }
 
 void sync_scalars(mdffgpu_ctx* c) {
@@ -1410,7 +1415,7 @@ void cell_sort(mdffgpu_ctx* c) {
   k_cell_fill<<<nblk(n), MDFF_BLOCK, 0, st>>>(n, c->d_cellof, c->d_ccur, c->d_polrows);
   k_cell_order<<<nblk(n), MDFF_BLOCK, 0, st>>>(n, c->d_cellof, c->d_cstart, c->d_polrows,
                                                c->d_perm, c->d_rank);
-  if (c->linduced && scf_field_fp32(c))
+  if (c->linduced)
     k_pol_rows<<<1, 1024, 0, st>>>(n, c->d_perm, c->d_typ, c->polmask, c->d_polrows);
   check_launch(c, "cell sort");
 }

@@ -506,58 +506,6 @@ template __global__ void k_es_dir<ES_FINAL, double, true>(EsDirArgs);
 template __global__ void k_es_dir<ES_STATIC, float, true>(EsDirArgs);
 template __global__ void k_es_dir<ES_FINAL, float, true>(EsDirArgs);
 
-// ---------------------------------------------------------------------------
-// Dipole field tensor of the SCF (multipole_ES_dir with task d-d and no
-// damping, :2407-2421), FP64 path.  The pair geometry is fixed during the
-// SCF, so k_pairs_t2 stores for every directed pair inside the cutoff, in the
-// row layout of nbr, the four-vector (r, 3F2/d^5) and then, in a plane of
-// its own, F1/d^3; pairs outside the cutoff get zero factors.  k_dd_field
-// applies E_i = sum_j [r (r.mu_j) 3F2/d^5 - mu_j F1/d^3].  With polmask set,
-// both run over the atoms of its species only (the field is used at the
-// polarizable atoms only; elsewhere it is not written).
-template <bool BATCH>
-__global__ __launch_bounds__(MDFF_BLOCK) void k_pairs_t2(EsDirArgs a, double* __restrict__ tab) {
-  const int n = a.n;
-  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i0 = tid / LPA, sub = tid % LPA;
-  if (i0 >= n) return;
-  const int i = a.perm ? a.perm[i0] : i0;  // atoms in spatial order
-  const int cf = BATCH ? a.cfg[i] : 0;
-  const Cell& cell = BATCH ? a.bc[cf].cell : a.cell;
-  const double cut2 = BATCH ? a.bc[cf].cut2 : a.cut2;
-  const double alpha = BATCH ? a.bc[cf].alpha : a.alpha;
-  const double alpha2 = alpha * alpha, alpha3 = alpha2 * alpha;
-  const double piroot = sqrt(MDFF_PI);
-  const double si1 = a.s[i], si2 = a.s[i + n], si3 = a.s[i + 2 * n];
-  // rows of the species in polmask only (all with 0): k_dd_field skips
-  // the others
-  if (a.polmask && !((a.polmask >> a.typ[i]) & 1u)) return;
-  const int c = a.cnt[i];
-  const size_t plane = (size_t)a.maxnb * n;
-  for (int k = sub; k < c; k += LPA) {
-    const size_t e = (size_t)i * a.maxnb + k;
-    const int j = a.nbr[e];
-    double rx, ry, rz, A2 = 0.0, A1 = 0.0;
-    const double d2 =
-        min_image(cell, si1 - a.s4[j].x, si2 - a.s4[j].y, si3 - a.s4[j].z, rx, ry, rz);
-    if (!(d2 > cut2)) {
-      const double d = sqrt(d2);
-      const double d3 = d2 * d;
-      const double dm1 = 1.0 / d;
-      const double dm3 = dm1 / d2;
-      const double dm5 = dm3 / d2;
-      const double expon = exp(-alpha2 * d2) / piroot;
-      const double F0 = errfc_nr(alpha * d);
-      const double F1 = F0 + 2.0 * alpha * d * expon;
-      const double F2 = F1 + 4.0 * alpha3 * d3 * expon / 3.0;
-      A2 = 3.0 * F2 * dm5;
-      A1 = F1 * dm3;
-    }
-    reinterpret_cast<double4*>(tab)[e] = make_double4(rx, ry, rz, A2);
-    tab[4 * plane + e] = A1;
-  }
-}
-
 // Dipoles of the SCF iteration in FP32, stored at the atom's spatial rank:
 // a row of the compacted pair table lists its neighbours by rank, so the
 // lanes of one gather read neighbouring 16-byte slots.
@@ -602,75 +550,57 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_pack_mu(int n, const double* __r
   mu4[i] = v;
 }
 
-// DD_LANES lanes per atom (a whole wave), pairs taken 2 at a time per lane
-// (loads in flight together), accumulated in list order per lane.  A
-// neighbour without a dipole contributes exact zeros.
-__global__ __launch_bounds__(MDFF_BLOCK) void k_dd_field(EsDirArgs a,
-                                                         const double* __restrict__ tab,
-                                                         const double4* __restrict__ mu4) {
-  using R = double;
-  using R4 = double4;
-  const int n = a.n;
-  const int tid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i0 = tid / DD_LANES, sub = tid % DD_LANES;
-  const int i = (a.perm && i0 < n) ? a.perm[i0] : i0;  // atoms in spatial order
-  R e0 = 0, e1 = 0, e2 = 0;
-  const size_t plane = (size_t)a.maxnb * n;
-  const R4* t4 = reinterpret_cast<const R4*>(tab);
-  const R* t1 = tab + 4 * plane;
-  const bool act = i < n && (!a.polmask || ((a.polmask >> a.typ[i]) & 1u));
-  const int c = act ? a.cnt[i] : 0;
-  const size_t row = (size_t)(act ? i : 0) * a.maxnb;
-  constexpr int U = 2;
-  for (int k0 = sub; k0 < c; k0 += U * DD_LANES) {
-    int jj[U];
-    R4 g[U], m[U];
-    R A1[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + u * DD_LANES;
-      const size_t e = row + (k < c ? k : 0);
-      jj[u] = a.nbr[e];
-      g[u] = t4[e];
-      A1[u] = t1[e];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) m[u] = mu4[jj[u]];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (k0 + u * DD_LANES >= c) break;
-      const R rmj = g[u].x * m[u].x + g[u].y * m[u].y + g[u].z * m[u].z;
-      e0 += g[u].x * rmj * g[u].w - m[u].x * A1[u];
-      e1 += g[u].y * rmj * g[u].w - m[u].y * A1[u];
-      e2 += g[u].z * rmj * g[u].w - m[u].z * A1[u];
-    }
-  }
-  for (int off = DD_LANES / 2; off > 0; off >>= 1) {
-    e0 += __shfl_xor(e0, off, 64);
-    e1 += __shfl_xor(e1, off, 64);
-    e2 += __shfl_xor(e2, off, 64);
-  }
-  if (act && sub == 0) {
-    a.ef[i] = e0;
-    a.ef[i + n] = e1;
-    a.ef[i + 2 * n] = e2;
-  }
+// ---------------------------------------------------------------------------
+// SCF dipole field (multipole_ES_dir with task d-d and no damping,
+// src/field.f90:2407-2421) from a compacted pair table: the pair geometry is
+// fixed during the SCF.  Once per evaluation k_dd_table (or the static FP32
+// real-space pass) keeps, per atom of a species in fieldmask and in list
+// order, only the list entries inside the cutoff whose species (polmask) can
+// hold an induced dipole, with A2 = 3F2/d^5, A1 = F1/d^3 and the neighbour's
+// slot in the dipole array (its spatial rank when a.rank is given, else its
+// index).  Rows and counts are in the processing order i0 (atom perm[i0] when
+// perm is given).  Each SCF iteration then applies
+// E_i = sum_j [A2 r (r.mu_j) - A1 mu_j].  FP32 (mixed path, factors formed
+// from an FP64 fractional difference): k_dd_tab2, r from 32-bit fixed-point
+// positions, 10 bytes of table and one 32-byte gather per pair.  FP64:
+// k_dd_tab64, r from the fractional coordinates by the same formula as here,
+// 18 bytes (20 above 65,536 atoms) of table and one 48-byte gather.
+template <typename R>
+__device__ __forceinline__ void dd_factors(R d2, R alpha, R c43a3, R& A2, R& A1);
+
+template <>
+__device__ __forceinline__ void dd_factors<float>(float d2, float alpha, float c43a3, float& A2,
+                                                  float& A1) {
+  const float d = sqrtf(d2);
+  const float dm1 = 1.f / d;
+  const float dm3 = dm1 * dm1 * dm1;
+  const float expon = __expf(-alpha * alpha * d2) * 0.56418958354775628f;  // 1/sqrt(pi)
+  const float F1 = errfc_t<float>(alpha * d) + 2.f * alpha * d * expon;
+  const float F2 = F1 + c43a3 * d2 * d * expon;
+  A2 = 3.f * F2 * dm3 * dm1 * dm1;
+  A1 = F1 * dm3;
 }
 
-// ---------------------------------------------------------------------------
-// SCF dipole field of the mixed path, from a compacted FP32 pair table.  Once
-// per evaluation k_dd_table (or the static FP32 real-space pass) keeps, per
-// atom and in list order, only the list entries inside the cutoff, with
-// A2 = 3F2/d^5, A1 = F1/d^3 (the undamped d-d terms of
-// src/field.f90:2407-2421, formed in FP32 from an FP64 fractional
-// difference) and the neighbour's slot in the dipole array (its spatial
-// rank when a.rank is given, else its index).  Rows and counts are in the
-// processing order i0 (atom perm[i0] when perm is given).  Each SCF
-// iteration then applies E_i = sum_j [A2 r (r.mu_j) - A1 mu_j] (k_dd_tab2),
-// forming r from 32-bit fixed-point positions: 10 bytes of table and one
-// 32-byte gather per pair.
-template <bool BATCH>
-__global__ __launch_bounds__(MDFF_BLOCK) void k_dd_table(EsDirArgs a, float2* __restrict__ tab,
+template <>
+__device__ __forceinline__ void dd_factors<double>(double d2, double alpha, double, double& A2,
+                                                   double& A1) {
+  const double alpha2 = alpha * alpha, alpha3 = alpha2 * alpha;
+  const double d = sqrt(d2);
+  const double d3 = d2 * d;
+  const double dm1 = 1.0 / d;
+  const double dm3 = dm1 / d2;
+  const double dm5 = dm3 / d2;
+  const double expon = exp(-alpha2 * d2) / sqrt(MDFF_PI);
+  const double F0 = errfc_nr(alpha * d);
+  const double F1 = F0 + 2.0 * alpha * d * expon;
+  const double F2 = F1 + 4.0 * alpha3 * d3 * expon / 3.0;
+  A2 = 3.0 * F2 * dm5;
+  A1 = F1 * dm3;
+}
+
+template <bool BATCH, typename R, typename R2>
+__global__ __launch_bounds__(MDFF_BLOCK) void k_dd_table(EsDirArgs a, unsigned fieldmask,
+                                                         R2* __restrict__ tab,
                                                          int* __restrict__ tj,
                                                          int* __restrict__ tcnt) {
   const int n = a.n;
@@ -680,39 +610,33 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_dd_table(EsDirArgs a, float2* __
   const int i = a.perm ? a.perm[i0] : i0;  // atoms in spatial order
   const int cf = BATCH ? a.cfg[i] : 0;
   const Cell& cell = BATCH ? a.bc[cf].cell : a.cell;
-  const float cut2 = (float)(BATCH ? a.bc[cf].cut2 : a.cut2);
+  const R cut2 = (R)(BATCH ? a.bc[cf].cut2 : a.cut2);
   const double alphad = BATCH ? a.bc[cf].alpha : a.alpha;
-  const float alpha = (float)alphad, alpha2 = alpha * alpha;
-  const float c43a3 = (float)(4.0 / 3.0 * alphad * alphad * alphad);
+  const R alpha = (R)alphad;
+  const R c43a3 = (R)(4.0 / 3.0 * alphad * alphad * alphad);
   const double4 si = a.s4[i];
-  // only pairs of two species in polmask (all with 0)
+  // only pairs of a species in fieldmask and one in polmask (all with 0)
   const unsigned pm = a.polmask ? a.polmask : ~0u;
-  const bool pol_i = (pm >> (BATCH ? a.typ[i] : s4_type(si))) & 1u;
-  const int c = pol_i ? a.cnt[i] : 0;
+  const unsigned fm = fieldmask ? fieldmask : ~0u;
+  const bool fld_i = (fm >> (BATCH ? a.typ[i] : s4_type(si))) & 1u;
+  const int c = fld_i ? a.cnt[i] : 0;
   const size_t lrow = (size_t)i * a.maxnb;  // the atom's list row
   const size_t row = (size_t)i0 * a.maxnb;  // its table row: processing order
   const unsigned long long below = (1ull << lane) - 1ull;
   int base = 0;
   for (int k0 = 0; k0 < c; k0 += 64) {
     const int k = k0 + lane;
-    float2 v = make_float2(0.f, 0.f);
+    R2 v;
+    v.x = v.y = 0;
     int j = 0;
     bool in = false;
     if (k < c) {
       j = a.nbr[lrow + k];
       const double4 sj = a.s4[j];
-      float rx, ry, rz;
-      const float d2 = min_image_t<float>(cell, si.x - sj.x, si.y - sj.y, si.z - sj.z, rx, ry, rz);
+      R rx, ry, rz;
+      const R d2 = min_image_t<R>(cell, si.x - sj.x, si.y - sj.y, si.z - sj.z, rx, ry, rz);
       in = !(d2 > cut2) && ((pm >> (BATCH ? a.typ[j] : s4_type(sj))) & 1u);
-      if (in) {
-        const float d = sqrtf(d2);
-        const float dm1 = 1.f / d;
-        const float dm3 = dm1 * dm1 * dm1;
-        const float expon = __expf(-alpha2 * d2) * 0.56418958354775628f;  // 1/sqrt(pi)
-        const float F1 = errfc_t<float>(alpha * d) + 2.f * alpha * d * expon;
-        const float F2 = F1 + c43a3 * d2 * d * expon;
-        v = make_float2(3.f * F2 * dm3 * dm1 * dm1, F1 * dm3);
-      }
+      if (in) dd_factors<R>(d2, alpha, c43a3, v.x, v.y);
     }
     const unsigned long long m = __ballot(in);
     if (in) {
@@ -728,13 +652,95 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_dd_table(EsDirArgs a, float2* __
   }
   if (lane == 0) {
     tcnt[i0] = base;
-    if (base == 0) {  // a row without pairs holds one zero entry (k_dd_tab2 reads it)
-      tab[row] = make_float2(0.f, 0.f);
+    if (base == 0) {  // a row without pairs holds one zero entry (the field kernels read it)
+      R2 z;
+      z.x = z.y = 0;
+      tab[row] = z;
       if (a.dd16)
         reinterpret_cast<unsigned short*>(tj)[row] = 0;
       else
         tj[row] = 0;
     }
+  }
+}
+
+// Fractional coordinates and dipoles of the FP64 field, 48 bytes per atom at
+// its slot (rank, or index without rank): (x, y), (z, mu_x), (mu_y, mu_z).
+__global__ __launch_bounds__(MDFF_BLOCK) void k_pack_smu(int n, const double4* __restrict__ s4,
+                                                         const double* __restrict__ mu,
+                                                         const int* __restrict__ rank,
+                                                         double2* __restrict__ smu) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  double2* o = smu + 3 * (size_t)(rank ? rank[i] : i);
+  const double4 s = s4[i];
+  o[0] = make_double2(s.x, s.y);
+  o[1] = make_double2(s.z, mu[i]);
+  o[2] = make_double2(mu[i + n], mu[i + 2 * n]);
+}
+
+// The FP64 SCF dipole field from the table: one wave per row listed in rows
+// (all n rows in order when rows is null; the field of atoms with an empty
+// row is zero), DD64_U entries per lane and trip with every load issued
+// unconditionally (indexes clamped to the row's last entry, a row without
+// pairs holds one zero entry; factors past the count are zero).  Bound by
+// the gathers: three 16-byte loads per pair.
+template <typename IT>
+__global__ __launch_bounds__(MDFF_BLOCK) void k_dd_tab64(
+    int n, int maxnb, const double2* __restrict__ tab, const IT* __restrict__ tj,
+    const int* __restrict__ tcnt, const double2* __restrict__ smu, Cell cell,
+    const BatchCfg* __restrict__ bc, const int* __restrict__ cfg, const int* __restrict__ perm,
+    const int* __restrict__ rows, int nrows, double* __restrict__ ef) {
+  constexpr int U = DD64_U;
+  const int lane = threadIdx.x & 63;
+  const int v =
+      __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+  if (v >= nrows) return;
+  const int r = rows ? rows[v] : v;
+  const int c = tcnt[r];
+  const int i = perm ? perm[r] : r;
+  const Cell& cl = bc ? bc[cfg[i]].cell : cell;
+  const double2 a0 = smu[3 * (size_t)r], a1 = smu[3 * (size_t)r + 1];
+  const double2* trow = tab + (size_t)r * maxnb;
+  const IT* jrow = tj + (size_t)r * maxnb;
+  const int last = max(c - 1, 0);
+  double e0 = 0.0, e1 = 0.0, e2 = 0.0;
+  for (int k0 = lane; k0 - lane < c; k0 += U * 64) {
+    int jj[U];
+    double2 g[U], q0[U], q1[U], q2[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = min(k0 + u * 64, last);
+      jj[u] = jrow[k];
+      g[u] = trow[k];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const double2* p = smu + 3 * (size_t)jj[u];
+      q0[u] = p[0];
+      q1[u] = p[1];
+      q2[u] = p[2];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (k0 + u * 64 >= c) g[u] = make_double2(0.0, 0.0);
+      double rx, ry, rz;
+      min_image(cl, a0.x - q0[u].x, a0.y - q0[u].y, a1.x - q1[u].x, rx, ry, rz);
+      const double rm = (rx * q1[u].y + ry * q2[u].x + rz * q2[u].y) * g[u].x;
+      e0 += rx * rm - q1[u].y * g[u].y;
+      e1 += ry * rm - q2[u].x * g[u].y;
+      e2 += rz * rm - q2[u].y * g[u].y;
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    e0 += __shfl_xor(e0, off, 64);
+    e1 += __shfl_xor(e1, off, 64);
+    e2 += __shfl_xor(e2, off, 64);
+  }
+  if (lane == 0) {
+    ef[i] = e0;
+    ef[i + n] = e1;
+    ef[i + 2 * n] = e2;
   }
 }
 
@@ -886,11 +892,18 @@ MDFF_DD_TAB2(unsigned short, 4)
 MDFF_DD_TAB2(unsigned short, 6)
 MDFF_DD_TAB2(unsigned short, 8)
 #undef MDFF_DD_TAB2
-template __global__ void k_pairs_t2<false>(EsDirArgs, double*);
-template __global__ void k_pairs_t2<true>(EsDirArgs, double*);
-template __global__ void k_dd_table<false>(EsDirArgs, float2*, int*, int*);
-template __global__ void k_dd_table<true>(EsDirArgs, float2*, int*, int*);
-template __global__ void k_pack_mu<double4>(int, const double*, double4*);
+template __global__ void k_dd_table<false, float, float2>(EsDirArgs, unsigned, float2*, int*, int*);
+template __global__ void k_dd_table<true, float, float2>(EsDirArgs, unsigned, float2*, int*, int*);
+template __global__ void k_dd_table<false, double, double2>(EsDirArgs, unsigned, double2*, int*, int*);
+template __global__ void k_dd_table<true, double, double2>(EsDirArgs, unsigned, double2*, int*, int*);
+template __global__ void k_dd_tab64<int>(int, int, const double2*, const int*, const int*,
+                                         const double2*, Cell, const BatchCfg*, const int*,
+                                         const int*, const int*, int, double*);
+template __global__ void k_dd_tab64<unsigned short>(int, int, const double2*,
+                                                    const unsigned short*, const int*,
+                                                    const double2*, Cell, const BatchCfg*,
+                                                    const int*, const int*, const int*, int,
+                                                    double*);
 template __global__ void k_pack_mu<float4>(int, const double*, float4*);
 
 }  // namespace mdff
