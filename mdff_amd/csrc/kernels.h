@@ -288,6 +288,14 @@ template <typename R4>
 __global__ void k_pack_qmu(int n, const double* q, const double* mu, R4* qm);
 template <bool BATCH, typename R, typename R2>
 __global__ void k_dd_table(EsDirArgs a, unsigned fieldmask, R2* tab, int* tj, int* tcnt);
+// One slot of the FP64 field's positions and dipoles.
+__device__ __forceinline__ void smu_store(double2* smu, int slot, double4 s, double mx, double my,
+                                          double mz) {
+  double2* o = smu + 3 * (size_t)slot;
+  o[0] = make_double2(s.x, s.y);
+  o[1] = make_double2(s.z, mx);
+  o[2] = make_double2(my, mz);
+}
 __global__ void k_pack_smu(int n, const double4* s4, const double* mu, const int* rank,
                            double2* smu);
 template <typename IT>
@@ -377,7 +385,8 @@ __global__ void k_cg_update(CgArgs a);
 __global__ void k_cg_dir(CgArgs a);
 __global__ void k_cg_upol(CgArgs a);
 __global__ void k_induced(int n, const int* typ, const TypeTables* T, const double* E,
-                          double* mu, double* part, const int* rank, float4* mu4, double* th);
+                          double* mu, double* part, const int* rank, float4* mu4, double* th, const double4* s4,
+                          double2* smu);
 __global__ void k_scf_resid(int n, const int* typ, const TypeTables* T, const double* mu,
                             const double* E, double* part);
 

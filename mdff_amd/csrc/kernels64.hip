@@ -633,7 +633,8 @@ template __global__ void k_combine64<ES_FINAL>(CombineArgs);
 // induced_moment (src/field.f90:1716-1803): mu = alpha E on polarizable
 // atoms; partial row 0 = sum mu alpha^-1 mu (u_pol before the 1/2).
 // With mu4 (the FP32 SCF field of the mixed path), the moments are also
-// stored as float4 at the atom's spatial rank (k_pack_mu_ranked fused).
+// stored as float4 at the atom's spatial rank (k_pack_mu_ranked fused); with
+// smu (the FP64 field) with the positions (k_pack_smu fused).
 // induced_moment (src/field.f90:1716-1803) of one atom: mu = alpha E on
 // ldip_polar or lquad_polar species, theta = polquad E (when th is given),
 // and its u_pol term: mu alpha^-1 mu / 2 on ldip_polar species,
@@ -672,7 +673,8 @@ __device__ __forceinline__ double induced_atom(const TypeTables* T, int t, int n
 __global__ __launch_bounds__(MDFF_BLOCK) void k_induced(
     int n, const int* __restrict__ typ, const TypeTables* __restrict__ T,
     const double* __restrict__ E, double* __restrict__ mu, double* __restrict__ part,
-    const int* __restrict__ rank, float4* __restrict__ mu4, double* __restrict__ th) {
+    const int* __restrict__ rank, float4* __restrict__ mu4, double* __restrict__ th,
+    const double4* __restrict__ s4, double2* __restrict__ smu) {
   __shared__ double red[4];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   double acc[1] = {0.0};
@@ -683,6 +685,7 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_induced(
     mu[i + n] = m[1];
     mu[i + 2 * n] = m[2];
     if (mu4) mu4[rank[i]] = make_float4((float)m[0], (float)m[1], (float)m[2], 0.f);
+    if (smu) smu_store(smu, rank[i], s4[i], m[0], m[1], m[2]);
   }
   block_sum<1>(acc, red);
   if (threadIdx.x == 0) part[blockIdx.x] = acc[0];

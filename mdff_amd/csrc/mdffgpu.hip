@@ -81,6 +81,8 @@ struct mdffgpu_ctx {
   int* d_nlr = nullptr;  // per-range neighbour counts, then offsets, of a list build
   double *d_q = nullptr, *d_qzero = nullptr, *d_dip = nullptr, *d_mu = nullptr,
          *d_muind = nullptr, *d_mup = nullptr;
+  // FP64 SCF: the next iteration's moments and u_pol partials, queued ahead
+  double *d_muind2 = nullptr, *d_upart2 = nullptr;
   double4* d_s4 = nullptr;   // fractional coordinates, one double4 per atom
   // spatial order of the atoms (cells of about 4 A, row-major, atom index
   // within a cell), refreshed with the neighbour list: perm[rank] = atom
@@ -554,6 +556,10 @@ void alloc_atoms(mdffgpu_ctx* c) {
   dalloc(c, &c->d_mu4, n);
   dalloc(c, &c->d_s4, n);
   dalloc(c, &c->d_upart, nblk(c->n));
+  if (!c->noalloc) {
+    dalloc(c, &c->d_muind2, 3 * n);
+    dalloc(c, &c->d_upart2, nblk(c->n));
+  }
   if (c->P.scf_solver == MDFFGPU_SCF_PCG) dalloc(c, &c->d_cg, 12 * n);
   dalloc(c, &c->d_perm, n);
   dalloc(c, &c->d_rank, n);
@@ -610,7 +616,8 @@ bool scf_field_fp32(const mdffgpu_ctx* c) {
 
 // Real-space part of the SCF dipole field (ES_IND): E_dir of the dipoles mu
 // into d_efdir, from the pair table of the evaluation.  With packed, the
-// FP32 rank-ordered copy of mu is already in d_mu4 (k_induced wrote it).
+// rank-ordered copy of mu is already in d_mu4 (FP32) or with the positions
+// (FP64): k_induced wrote it.
 // FP32 SCF pair table of the mixed path in d_t2: the evaluation's
 // fixed-point positions (uint4 per rank), the (A2, A1) entries and the
 // neighbour slots (maxnb per row), the row counts.
@@ -677,7 +684,8 @@ void es_ind_dir(mdffgpu_ctx* c, const double* mu, bool packed = false) {
     // the rows of the polarizable atoms; with quadrupole-polarizable species
     // the field is read elsewhere too (empty rows give zeros)
     const bool all = c->fieldmask != c->polmask;
-    k_pack_smu<<<gb, MDFF_BLOCK, 0, st>>>(n, c->d_s4, mu, c->d_rank, dd64_smu(c));
+    if (!packed)
+      k_pack_smu<<<gb, MDFF_BLOCK, 0, st>>>(n, c->d_s4, mu, c->d_rank, dd64_smu(c));
     dd_tab64_launch(c->st, n, c->maxnb, dd64_tab(c), dd64_tj(c), dd64_smu(c), c->cell,
                     nullptr, nullptr, c->d_perm, all ? nullptr : c->d_polrows,
                     all ? n : c->npolrows, c->d_efdir);
@@ -1142,26 +1150,32 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
   // mu = alpha E and their real-space field), so that the GPU does not idle
   // through the round trip.  A solve that stops there keeps those moments:
   // one Jacobi step past the accepted iterate, with a change below the
-  // residual just accepted.  The FP64 path follows the reference's
-  // sequence exactly.
-  const bool spec = mixed_prec;
+  // residual just accepted.  The FP64 path follows the reference's sequence
+  // exactly: the queued moments and their u_pol partials go to buffers of
+  // their own, taken over when the solve goes on (not in the allocation-free
+  // context, whose host memory is pageable, nor with induced quadrupoles).
+  // An evaluation of 3000 atoms (14 iterations) 1.65 -> 1.38 ms, of 24,576
+  // (12 iterations) 4.28 -> 4.06 ms.
+  const bool spec64 = !mixed_prec && !c->noalloc && !c->lqpol;
+  const bool spec = mixed_prec || spec64;
   if (spec && !c->ev_sc) {
     HCK(c, hipEventCreateWithFlags(&c->ev_sc, hipEventDisableTiming));
     HCK(c, hipHostGetDevicePointer((void**)&c->h_sc_dev, c->h_sc, 0));
   }
-  // with the FP32 SCF field, k_induced also packs the moments for k_dd_tab2
-  auto induced = [&](bool pack) {
+  // k_induced into mu and up; with pack also in the layout of the real-space
+  // field (FP32: k_dd_tab2, else k_dd_tab64)
+  auto induced = [&](bool pack, double* mu, double* up) {
+    const bool p32 = pack && scf_field_fp32(c);
     {
       ProfScope _ps(c, K_INDUCED);
-      k_induced<<<gb, MDFF_BLOCK, 0, st>>>(n, c->d_typ, c->d_tt, c->d_E, c->d_muind, c->d_upart,
-                                           c->d_rank,
-                                           pack ? reinterpret_cast<float4*>(c->d_mu4) : nullptr,
-                                           c->lqpol ? c->d_thind : nullptr);
+      k_induced<<<gb, MDFF_BLOCK, 0, st>>>(n, c->d_typ, c->d_tt, c->d_E, mu, up, c->d_rank,
+                                           p32 ? reinterpret_cast<float4*>(c->d_mu4) : nullptr,
+                                           c->lqpol ? c->d_thind : nullptr, c->d_s4,
+                                           pack && !p32 ? dd64_smu(c) : nullptr);
     }
     check_launch(c, "k_induced");
     upol_new = true;
   };
-  const bool pack = spec && scf_field_fp32(c);
   bool queued = false;  // this iteration's moments and real-space field are queued
   if (P.scf_solver == MDFFGPU_SCF_PCG) {
     // Preconditioned conjugate gradient on (alpha^-1 - T) mu = E_stat from
@@ -1202,7 +1216,7 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
     }
     ++iscf;
     if (P.calc_mode == 0)
-      induced(false);
+      induced(false, c->d_muind, c->d_upart);
     else if (P.algo_ext_dipole == MDFFGPU_EXT_POLY)
       extrap(c, (P.extrapolate_order == 0) ? 0 : (itime > P.extrapolate_order ? 1 : 2), 0, 0.0);
     else
@@ -1292,13 +1306,21 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
     check_launch(c, "k_cg_upol");
     upol_new = true;
   }
+  double rmsd_prev = 0.0;  // the residual before the current one
   while (P.scf_solver != MDFFGPU_SCF_PCG &&
          ((iscf < P.max_scf_pol_iter && rmsd > tol) || iscf < P.min_scf_pol_iter) && !stalled) {
     ++iscf;
+    bool packed = queued;
     if (queued) {
       // k_induced and the real-space field were queued by the last iteration
+      if (spec64) {
+        std::swap(c->d_muind, c->d_muind2);
+        std::swap(c->d_upart, c->d_upart2);
+        upol_new = true;
+      }
     } else if (iscf != 1 || P.calc_mode == 0) {
-      induced(false);
+      induced(true, c->d_muind, c->d_upart);
+      packed = true;
     } else if (P.algo_ext_dipole == MDFFGPU_EXT_POLY) {
       int op = (P.extrapolate_order == 0) ? 0 : (itime > P.extrapolate_order ? 1 : 2);
       extrap(c, op, 0, 0.0);
@@ -1307,8 +1329,9 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
     }
     // induced moments: dipole-dipole and quadrupole-quadrupole tasks
     // (src/field.f90:3304-3306)
-    es_call(c, ES_IND, c->d_qzero, c->d_muind, TASK_DD | (c->lqpol ? TASK_QUADQ : 0), 1, 0,
-            queued, c->lqpol ? c->d_thind : nullptr);
+    if (!queued) es_ind_dir(c, c->d_muind, packed);
+    es_call(c, ES_IND, c->d_qzero, c->d_muind, TASK_DD | (c->lqpol ? TASK_QUADQ : 0), 1, 0, true,
+            c->lqpol ? c->d_thind : nullptr);
     queued = false;
     ++*n_es;
     if (iscf == 1 && P.calc_mode == 1 && P.algo_ext_dipole == MDFFGPU_EXT_ASPC) {
@@ -1328,9 +1351,23 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
       }
       check_launch(c, "k_reduce_rows2");
       HCK(c, hipEventRecord(c->ev_sc, st));
-      induced(pack);
-      es_ind_dir(c, c->d_muind, pack);
-      queued = true;
+      if (spec64) {
+        // nothing is queued when the last two residuals, extrapolated
+        // geometrically, put this one below the tolerance
+        queued = !(iscf >= P.min_scf_pol_iter &&
+                   (iscf >= P.max_scf_pol_iter ||
+                    (rmsd_prev > 0.0 && rmsd * (rmsd / rmsd_prev) < tol)));
+        const bool u0 = upol_new;
+        if (queued) {
+          induced(true, c->d_muind2, c->d_upart2);
+          es_ind_dir(c, c->d_muind2, true);
+        }
+        upol_new = u0;
+      } else {
+        induced(true, c->d_muind, c->d_upart);
+        es_ind_dir(c, c->d_muind, true);
+        queued = true;
+      }
       // the profiling events of the queued launches are folded in at the
       // next stream synchronisation
       HCK(c, hipEventSynchronize(c->ev_sc));
@@ -1338,6 +1375,7 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
       reduce(c, 2, c->nresid, SC_RMSD);  // residual rows of the ES_IND combine
       sync_scalars(c);
     }
+    rmsd_prev = iscf > 1 ? rmsd : 0.0;
     rmsd = std::sqrt(c->h_sc[SC_RMSD] / c->h_sc[SC_RMSD + 1]);
     if (iscf == 1) rmsd_first = rmsd;
     if (rmsd < rmsd_best) {
@@ -2525,6 +2563,7 @@ void mdffgpu_destroy(mdffgpu_ctx* c) {
                   c->d_mup, c->d_Estat, c->d_E, c->d_efdir, c->d_efgdir, c->d_fdir,
                   c->d_force, c->d_ef, c->d_efg, c->d_apart, c->d_Ak, c->d_kcoe, c->d_kvec,
                   c->d_part, c->d_sc, c->d_hist, c->d_upart, c->d_cg, c->d_efgq,
+                  c->d_muind2, c->d_upart2,
                   c->d_efgmu, c->d_efgpart, c->d_efgcells, c->d_efgout};
   for (double* p : dp)
     if (p) (void)hipFree(p);

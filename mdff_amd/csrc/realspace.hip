@@ -665,18 +665,14 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_dd_table(EsDirArgs a, unsigned f
 }
 
 // Fractional coordinates and dipoles of the FP64 field, 48 bytes per atom at
-// its slot (rank, or index without rank): (x, y), (z, mu_x), (mu_y, mu_z).
+// its slot (rank, or index without rank).
 __global__ __launch_bounds__(MDFF_BLOCK) void k_pack_smu(int n, const double4* __restrict__ s4,
                                                          const double* __restrict__ mu,
                                                          const int* __restrict__ rank,
                                                          double2* __restrict__ smu) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  double2* o = smu + 3 * (size_t)(rank ? rank[i] : i);
-  const double4 s = s4[i];
-  o[0] = make_double2(s.x, s.y);
-  o[1] = make_double2(s.z, mu[i]);
-  o[2] = make_double2(mu[i + n], mu[i + 2 * n]);
+  smu_store(smu, rank ? rank[i] : i, s4[i], mu[i], mu[i + n], mu[i + 2 * n]);
 }
 
 // The FP64 SCF dipole field from the table: one wave per row listed in rows
