@@ -356,6 +356,64 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_b_grid_fields(
     Frec[i + r * n] = q[i] * er[r] + fg * (B[r] * w[0] + B[r + 3] * w[1] + B[r + 6] * w[2]);
 }
 
+// The end of one SCF iteration in one launch: the reciprocal field from the
+// grid sums ap (k_b_grid_fields) or, without them, rec, k_b_combine<ES_IND>
+// of atom i (the same operations in the same order), then either the next iteration's moments (next: x = alpha
+// E, also packed for the real-space field, mu4 or s4 and smu) or, with part,
+// the residual rows of k_scf_resid.  4.8 us at 12 configurations (9,800
+// atoms) against 4.7 + 3.8 + 3.8 + 2.6 us and their launches.
+__global__ __launch_bounds__(MDFF_BLOCK) void k_b_scf_step(
+    int N, const int* __restrict__ cfg, const BatchCfg* __restrict__ bc,
+    const int* __restrict__ typ, const TypeTables* __restrict__ T, const double* __restrict__ ap,
+    const double* __restrict__ rec, const double* __restrict__ dir, const double* __restrict__ S,
+    double* __restrict__ x, double* __restrict__ E, int next, float4* __restrict__ mu4, const double4* __restrict__ s4,
+    double2* __restrict__ smu, double* __restrict__ part) {
+  __shared__ double red[4 * 2];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t n = N;
+  double acc[2] = {0.0, 0.0};
+  if (i < N) {
+    const BatchCfg& b = bc[cfg[i]];
+    const double* B = b.cell.B;
+    const double fe = -2.0 * b.fpi_V * (2.0 * MDFF_PI);
+    const double sa2 = b.selfa2;
+    const double* src = ap ? ap : rec;
+    const double U[3] = {src[i], src[i + n], src[i + 2 * n]};
+    const int t = typ[i];
+    double e[3];
+    for (int r = 0; r < 3; ++r) {
+      const double er = ap ? fe * (B[r] * U[0] + B[r + 3] * U[1] + B[r + 6] * U[2]) : U[r];
+      double v = dir[i + r * n] + er + 2.0 * sa2 * x[i + r * n];
+      v += S[i + r * n];
+      e[r] = v;
+      E[i + r * n] = v;
+    }
+    if (next) {
+      double m[3] = {0.0, 0.0, 0.0};
+      if (T->polar[t] || T->qpolar[t])
+        for (int r = 0; r < 3; ++r)
+          for (int c = 0; c < 3; ++c) m[r] = m[r] + T->pol[t][r + 3 * c] * e[c];
+      for (int r = 0; r < 3; ++r) x[i + r * n] = m[r];
+      if (mu4) mu4[i] = make_float4((float)m[0], (float)m[1], (float)m[2], 0.f);
+      if (smu) smu_store(smu, i, s4[i], m[0], m[1], m[2]);
+    } else if (part && T->polar[t]) {
+      acc[1] = 1.0;
+      for (int r = 0; r < 3; ++r) {
+        const double pa = T->pol[t][r + 3 * r];
+        if (pa == 0.0) continue;
+        const double d = x[i + r * n] / pa - e[r];
+        acc[0] = acc[0] + d * d;
+      }
+    }
+  }
+  if (!part) return;
+  block_sum<2>(acc, red);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = acc[0];
+    part[gridDim.x + blockIdx.x] = acc[1];
+  }
+}
+
 // small vector kernels (graph-safe replacements of memset / memcpy)
 __global__ __launch_bounds__(MDFF_BLOCK) void k_b_fill(size_t n, double v, double* __restrict__ x) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1091,13 +1149,21 @@ void grid_state(mdffgpu_batch* b) {
   launch_check(b, "batch grid bins");
 }
 
+// What an SCF iteration's ES_IND call ends with (k_b_scf_step; x are its
+// dipoles): the next moments, or the residual partials.
+struct ScfStep {
+  double* x;
+  int next;
+  double* part;
+};
+
 // One multipole_ES call over the batch with sources (q, mu):
 //   STATIC  out = static field (charges only)
 //   IND     out = S + dipole field of mu (the SCF field operator)
 //   FINAL   out = electrostatic forces * coul_unit
 template <typename R>
 void es_call(mdffgpu_batch* b, int mode, const double* q, const double* mu, const double* S,
-             double* out) {
+             double* out, bool packed = false, const ScfStep* step = nullptr) {
   const int N = b->N;
   const int gbl = nblk((size_t)N * LPA);
   EsDirArgs da = es_args(b, q, mu);
@@ -1111,12 +1177,12 @@ void es_call(mdffgpu_batch* b, int mode, const double* q, const double* mu, cons
     if constexpr (sizeof(R) == sizeof(double)) {
       double2* smu = reinterpret_cast<double2*>(b->d_t2);
       const double2* tab = smu + 3 * (size_t)N;
-      k_pack_smu<<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, b->d_s4, mu, nullptr, smu);
+      if (!packed) k_pack_smu<<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, b->d_s4, mu, nullptr, smu);
       dd_tab64_launch(b->st, N, b->maxnb, tab, reinterpret_cast<const int*>(tab + cap), smu, Cell{},
                       b->d_bc, b->d_cfg, nullptr, b->d_polrows, b->npolrows, b->d_dir);
     } else {
       float4* m4 = reinterpret_cast<float4*>(b->d_mu4);
-      k_pack_mu<float4><<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, mu, m4);
+      if (!packed) k_pack_mu<float4><<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, mu, m4);
       const uint4* u4 = reinterpret_cast<const uint4*>(b->d_t2);
       const float2* tab = reinterpret_cast<const float2*>(u4 + N);
       const int* tj = reinterpret_cast<const int*>(tab + cap);
@@ -1154,8 +1220,9 @@ void es_call(mdffgpu_batch* b, int mode, const double* q, const double* mu, cons
     // static and SCF calls' field is read
     grid::sums(b->gp, nullptr, b->st, q, mu, chg, dip, mode == ES_FINAL, mode == ES_IND,
                mode != ES_FINAL, b->d_apart, nullptr);
-    k_b_grid_fields<<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, b->d_cfg, b->d_bc, b->d_apart, q, mu,
-                                                       mode == ES_FINAL, b->d_rec, b->d_frec);
+    if (!step)
+      k_b_grid_fields<<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, b->d_cfg, b->d_bc, b->d_apart, q, mu,
+                                                         mode == ES_FINAL, b->d_rec, b->d_frec);
   } else if (sizeof(R) == sizeof(float) && mx_state(b)) {
     mdff::mixed::kspace_batch(b->mx, b->st, b->d_s, b->epoch, b->d_cfg, q, mu, chg, dip,
                               mode == ES_FINAL, b->d_rec, b->d_frec);
@@ -1169,6 +1236,16 @@ void es_call(mdffgpu_batch* b, int mode, const double* q, const double* mu, cons
   }
   launch_check(b, "batch k space");
   const int gb = nblk(N);
+  if (step) {
+    constexpr bool f64 = sizeof(R) == sizeof(double);
+    k_b_scf_step<<<gb, MDFF_BLOCK, 0, b->st>>>(
+        N, b->d_cfg, b->d_bc, b->d_typ, b->d_ty, b->grid_calls ? b->d_apart : nullptr, b->d_rec,
+        b->d_dir, S, step->x, out, step->next,
+        f64 ? nullptr : reinterpret_cast<float4*>(b->d_mu4), b->d_s4,
+        f64 ? reinterpret_cast<double2*>(b->d_t2) : nullptr, step->part);
+    launch_check(b, "batch SCF step");
+    return;
+  }
   const double cu = b->P.coul_unit;
   if (mode == ES_STATIC)
     k_b_combine<ES_STATIC><<<gb, MDFF_BLOCK, 0, b->st>>>(N, b->d_cfg, b->d_bc, cu, b->d_dir,
@@ -1196,13 +1273,17 @@ int jacobi(mdffgpu_batch* b, const double* S, double* x, double* E, int iters, d
   int it = 0;
   *rmsd = 0.0;
   const int nmax = iters > 0 ? iters : std::max(P.max_scf_pol_iter, 1);
+  bool have = false;  // the last iteration's step wrote this one's moments
   while (it < nmax) {
     ++it;
-    k_induced<<<gb, MDFF_BLOCK, 0, b->st>>>(N, b->d_typ, b->d_ty, E, x, b->d_part, nullptr,
-                                            nullptr, nullptr, nullptr, nullptr);
-    es_call<R>(b, ES_IND, b->d_zero, x, S, E);
+    if (!have)
+      k_induced<<<gb, MDFF_BLOCK, 0, b->st>>>(N, b->d_typ, b->d_ty, E, x, b->d_part, nullptr,
+                                              nullptr, nullptr, nullptr, nullptr);
+    const bool next = iters > 0 && it < nmax;
+    const ScfStep step = {x, next ? 1 : 0, iters == 0 ? b->d_part : nullptr};
+    es_call<R>(b, ES_IND, b->d_zero, x, S, E, have, &step);
+    have = next;
     if (iters == 0) {
-      k_scf_resid<<<gb, MDFF_BLOCK, 0, b->st>>>(N, b->d_typ, b->d_ty, x, E, b->d_part);
       reduce(b, 2, gb, 0);
       BCK(b, hipMemcpyAsync(b->h_out, b->d_out, 2 * sizeof(double), hipMemcpyDeviceToHost,
                             b->st));
