@@ -1225,6 +1225,13 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
     ++*n_es;
     k_cg_init<<<gb, MDFF_BLOCK, 0, st>>>(g);
     check_launch(c, "k_cg_init");
+    // T p of the direction (k_cg_init and k_cg_dir wrote its FP32 copy)
+    auto product = [&]() {
+      es_ind_dir(c, g.p, pk);
+      c->cg_Ap = g.Ap;
+      es_call(c, ES_IND, c->d_qzero, g.p, TASK_DD, 1, 0, true);
+      c->cg_Ap = nullptr;
+    };
     int cur = 0;  // triple of the current r.z, |r|^2, npol
     auto base = [](int k) { return SC_CG + 3 * k; };
     // the initial sums into the device scalars and mapped host memory; the
@@ -1237,31 +1244,19 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
     }
     check_launch(c, "k_reduce_rows2");
     HCK(c, hipEventRecord(c->ev_sc, st));
-    bool first_queued = iscf < P.max_scf_pol_iter;
-    if (first_queued) {
-      c->cg_Ap = g.Ap;
-      es_call(c, ES_IND, c->d_qzero, g.p, TASK_DD, 1, 0);
-      c->cg_Ap = nullptr;
-    }
+    bool queued_p = iscf < P.max_scf_pol_iter;  // the next product is queued
+    if (queued_p) product();
     HCK(c, hipEventSynchronize(c->ev_sc));
     rmsd = std::sqrt(c->h_sc[base(cur) + 1] / c->h_sc[base(cur) + 2]);
     rmsd_first = rmsd;
     rmsd_best = rmsd;
-    bool queued_p = false;  // the direction and its real-space field are queued
     double rmsd_prev = 0.0;  // the residual before the current one
     while (((iscf < P.max_scf_pol_iter && rmsd > tol) || iscf < P.min_scf_pol_iter) && !stalled) {
       ++iscf;
       // T p by an ES_IND call whose combine forms Ap = alpha^-1 p - T p and
       // the partials of p.Ap (row 0); the update sums those itself and
       // writes its own partials to rows 1..3
-      if (first_queued) {
-        first_queued = false;  // the product queued after the initial sums
-      } else {
-        c->cg_Ap = g.Ap;
-        es_call(c, ES_IND, c->d_qzero, g.p, TASK_DD, 1, 0, queued_p && pk);
-        c->cg_Ap = nullptr;
-      }
-      queued_p = false;
+      if (!queued_p) product();
       ++*n_es;
       g.s_rz = base(cur);
       g.pap_part = c->d_part;
@@ -1278,15 +1273,18 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
       check_launch(c, "k_cg_dir");
       c->wt_ready = (g.wt != nullptr);
       HCK(c, hipEventRecord(c->ev_sc, st));
-      // the new direction's real-space field is queued behind the residual
-      // unless the last two residuals, extrapolated geometrically, put this
-      // one below the tolerance (then the solve most likely stops here)
+      // the next T p is queued behind the residual unless the last two
+      // residuals, extrapolated geometrically, put this one below the
+      // tolerance (then the solve most likely stops here; a product queued
+      // in vain overwrites nothing that is read afterwards).  With the
+      // real-space field alone queued the GPU idled 8 us per iteration at
+      // 3000 atoms, where that field takes 5 us.
       const bool last_likely =
           iscf >= P.min_scf_pol_iter &&
           (iscf >= P.max_scf_pol_iter ||
            (iscf >= 2 && rmsd_prev > 0.0 && rmsd * (rmsd / rmsd_prev) < tol));
-      queued_p = pk && !last_likely;
-      if (queued_p) es_ind_dir(c, g.p, true);
+      queued_p = !last_likely;
+      if (queued_p) product();
       HCK(c, hipEventSynchronize(c->ev_sc));
       cur = nxt;
       rmsd_prev = rmsd;
