@@ -1424,8 +1424,11 @@ Plan* create(hipStream_t st, const std::vector<Seg>& segs, const int kmax[3], bo
     e.ng *= e.M[a];
   }
   e.ntile = e.nt[0] * e.nt[1] * e.nt[2];
-  // two workgroups per CU of the spread
-  p->split = std::max(1, std::min(4, 512 / (e.ntile * e.nseg)));
+  // two workgroups per CU of the spread, but at most two partial grids: at
+  // 48^3 points (108 tiles) spread and forward transform, which reads them
+  // all from a few dozen CUs, take 11.7 + 6.1 us with one, 7.7 + 7.7 with two
+  // and 6.8 + 10.7 with four
+  p->split = std::max(1, std::min(2, 512 / (e.ntile * e.nseg)));
   e.N2f = 2 * kmax[1] + 1;
   e.N3c = kmax[2] + 1;
   e.NCC = e.N2f * e.N3c;
