@@ -236,6 +236,13 @@ __global__ void k_cell_order(int n, const int* cellof, const int* cnt, const int
                              int* rank);
 __global__ void k_pol_rows(int n, const int* perm, const int* typ, unsigned polmask, int* rows);
 __global__ void k_nlist_cells(NlCellArgs a);
+// Planes of n doubles copied across the numbering in one launch (k_planes).
+constexpr int PLANES_MAX = 27;
+struct PlaneMap {
+  const double* src[PLANES_MAX];
+  double* dst[PLANES_MAX];
+};
+__global__ void k_planes(int n, const int* idx, int scatter, PlaneMap m);
 __global__ void k_perm_gather(int n, int inner, int planes, const int* idx, const double* src,
                               double* dst);
 __global__ void k_perm_scatter(int n, int inner, int planes, const int* idx, const double* src,

@@ -144,3 +144,42 @@ def test_shuffled_standalone_efg(oracle_lib):
     assert g["n_scf"] == ref["n_scf"]
     assert_close(g["efg"], ref["efg"], what="efg")
     assert_close(g["mu"], ref["mu"], what="mu")
+
+
+@pytest.mark.parametrize("natoms", [(1, 2), (85, 171)])
+def test_host_outputs_by_subset(natoms):
+    """The host entry point stages the wanted outputs in one transfer: every
+    subset of the optional arrays gives the arrays of the full call, bitwise,
+    with atoms below and across a workgroup."""
+    import ctypes
+    import itertools
+
+    from mdff_amd import _lib
+    from mdff_amd.field import ForceField
+    from mdff_amd.params import MdffEnergies
+    s = C.silica(*natoms, seed=31, rc=3.0, kmax=4, pim=True, efg=True, scf_tol=1e-9,
+                 dmin=1.0 if natoms[0] == 1 else None)
+    n = s.natm
+    dp = ctypes.POINTER(ctypes.c_double)
+    sizes = (3, 9, 3, 9)  # mu, theta, ef, efg
+
+    def call(want):
+        ff = ForceField(s.params, s.itype, s.A)
+        r = [np.ascontiguousarray(s.r[:, k]) for k in range(3)]
+        f = np.zeros((3, n))
+        out = [np.full(k * n, 7.0) for k in sizes]
+        en = MdffEnergies()
+        st = _lib.lib().mdffgpu_engforce(
+            ff.handle, *[a.ctypes.data_as(dp) for a in r], 0, *[a.ctypes.data_as(dp) for a in f],
+            *[a.ctypes.data_as(dp) if w else None for a, w in zip(out, want)], ctypes.byref(en))
+        _lib.check(st, ff.handle)
+        ff.close()
+        return f, out
+
+    f0, full = call((1, 1, 1, 1))
+    assert np.abs(f0).max() > 0 and np.all(full[1] == 0)
+    for want in itertools.product((0, 1), repeat=4):
+        f, out = call(want)
+        np.testing.assert_array_equal(f, f0)
+        for w, a, b in zip(want, out, full):
+            np.testing.assert_array_equal(a, b if w else np.full_like(a, 7.0))
