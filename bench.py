@@ -189,6 +189,17 @@ def time_path(args, sys_, precision, frames_dev, scf=None, tuning=None, table=Tr
                                              n_dip=npol, n_fld=npol) / cnt
             peak, bound = FL.PEAK_FP16_MFMA_TFLOPS, "mfma"
             pipe = "fp16 matrix core (operands split in fp16 hi + lo, 3 products)"
+        elif name in ("grid_spread", "grid_gather", "grid_transform"):
+            fp64 = precision != P.PREC_MIXED
+            flop = FL.grid_flops(name, n, npol, list(p.kES), len(sampled), nsc, p.doefg,
+                                 17 if fp64 else 10) / cnt
+            # the transforms run on the FP64 matrix cores on both paths
+            if fp64 or name == "grid_transform":
+                peak, pipe = FL.PEAK_FP64_TFLOPS, "fp64 matrix and vector units"
+            else:
+                peak, pipe = FL.PEAK_FP32_TFLOPS, "fp32 matrix and vector units"
+            bound = "valu" if name == "grid_gather" else "mfma"
+            executed = flop
     if flop:
         achieved = flop / avg_s / 1e12
         traffic, source = profile_traffic(name)

@@ -298,13 +298,12 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_b_apply(int N, const int* __rest
 // Sum of the parts of one multipole_ES call (src/field.f90:1817-2054,
 // without surface term):
 //   STATIC  E_out = E_dir + E_rec + 2 selfa2 mu
-//   IND     E_out = S + E_dir + E_rec + 2 selfa2 mu
 //   FINAL   F_out = (F_dir + F_rec) coul_unit
 template <int MODE>
 __global__ __launch_bounds__(MDFF_BLOCK) void k_b_combine(
     int N, const int* __restrict__ cfg, const BatchCfg* __restrict__ bc, double coul_unit,
     const double* __restrict__ dir, const double* __restrict__ rec,
-    const double* __restrict__ mu, const double* __restrict__ S, double* __restrict__ out) {
+    const double* __restrict__ mu, double* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
   const double sa2 = bc[cfg[i]].selfa2;
@@ -313,9 +312,7 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_b_combine(
     if (MODE == ES_FINAL) {
       out[x] = (dir[x] + rec[x]) * coul_unit;
     } else {
-      double v = dir[x] + rec[x] + 2.0 * sa2 * mu[x];
-      if (MODE == ES_IND) v += S[x];
-      out[x] = v;
+      out[x] = dir[x] + rec[x] + 2.0 * sa2 * mu[x];
     }
   }
 }
@@ -357,17 +354,18 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_b_grid_fields(
 }
 
 // The end of one SCF iteration in one launch: the reciprocal field from the
-// grid sums ap (k_b_grid_fields) or, without them, rec, k_b_combine<ES_IND>
-// of atom i (the same operations in the same order), then either the next iteration's moments (next: x = alpha
-// E, also packed for the real-space field, mu4 or s4 and smu) or, with part,
-// the residual rows of k_scf_resid.  4.8 us at 12 configurations (9,800
-// atoms) against 4.7 + 3.8 + 3.8 + 2.6 us and their launches.
+// grid sums ap (k_b_grid_fields) or, without them, rec, the SCF field
+// E = S + E_dir + E_rec + 2 selfa2 x of atom i, then either the next
+// iteration's moments (next: x = alpha E, also packed for the real-space
+// field, mu4 or s4 and smu) or, with part, the residual rows of k_scf_resid.
+// Bound by its launch: 4.8 us for 12 configurations against 4.7 + 3.8 + 3.8 +
+// 2.6 us in four launches.
 __global__ __launch_bounds__(MDFF_BLOCK) void k_b_scf_step(
     int N, const int* __restrict__ cfg, const BatchCfg* __restrict__ bc,
     const int* __restrict__ typ, const TypeTables* __restrict__ T, const double* __restrict__ ap,
     const double* __restrict__ rec, const double* __restrict__ dir, const double* __restrict__ S,
-    double* __restrict__ x, double* __restrict__ E, int next, float4* __restrict__ mu4, const double4* __restrict__ s4,
-    double2* __restrict__ smu, double* __restrict__ part) {
+    double* __restrict__ x, double* __restrict__ E, int next, float4* __restrict__ mu4,
+    const double4* __restrict__ s4, double2* __restrict__ smu, double* __restrict__ part) {
   __shared__ double red[4 * 2];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const size_t n = N;
@@ -1249,13 +1247,10 @@ void es_call(mdffgpu_batch* b, int mode, const double* q, const double* mu, cons
   const double cu = b->P.coul_unit;
   if (mode == ES_STATIC)
     k_b_combine<ES_STATIC><<<gb, MDFF_BLOCK, 0, b->st>>>(N, b->d_cfg, b->d_bc, cu, b->d_dir,
-                                                         b->d_rec, mu, S, out);
-  else if (mode == ES_IND)
-    k_b_combine<ES_IND><<<gb, MDFF_BLOCK, 0, b->st>>>(N, b->d_cfg, b->d_bc, cu, b->d_dir,
-                                                      b->d_rec, mu, S, out);
+                                                         b->d_rec, mu, out);
   else
     k_b_combine<ES_FINAL><<<gb, MDFF_BLOCK, 0, b->st>>>(N, b->d_cfg, b->d_bc, cu, b->d_dir,
-                                                        b->d_frec, mu, S, out);
+                                                        b->d_frec, mu, out);
   launch_check(b, "batch combine");
 }
 

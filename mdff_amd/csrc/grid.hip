@@ -502,7 +502,7 @@ static int xcd_blocks(int n) { return (n + 7) / 8 * 8; }
 // (zero outside an atom's support), the next 32 loaded while the current
 // ones multiply; no zeroed grid and no atomics.  The tile shape makes 2.6
 // (W = 10) to 3.5 (W = 16) products per term of the support.  Where the grid
-// has few tiles, gridDim.z blocks share a tile's atoms and write partial
+// has few tiles, gridDim.z (one or two) blocks share a tile's atoms and write partial
 // grids, which the forward transform adds.
 constexpr int SCH = 32;  // atoms per LDS chunk
 
@@ -1595,14 +1595,14 @@ static int sums_t(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,
   {
     ProfScope _ps(ctx, K_GRID_SPREAD);
     if (chg && dip)
-    k_grid_spread<R, true, true><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
-                                                            p->d_cnt, p->cap, sa, G);
-  else if (dip)
-    k_grid_spread<R, false, true><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
-                                                             p->d_cnt, p->cap, sa, G);
-  else
-    k_grid_spread<R, true, false><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
-                                                             p->d_cnt, p->cap, sa, G);
+      k_grid_spread<R, true, true><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
+                                                              p->d_cnt, p->cap, sa, G);
+    else if (dip)
+      k_grid_spread<R, false, true><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab,
+                                                               p->d_ov, p->d_cnt, p->cap, sa, G);
+    else
+      k_grid_spread<R, true, false><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab,
+                                                               p->d_ov, p->d_cnt, p->cap, sa, G);
   }
   convolve<R>(p, ctx, st, p->split, pout);
   ProfScope _ps(ctx, K_GRID_GATHER);

@@ -11,6 +11,8 @@ unit of the k-space kernels: one (atom, k) pair, k over the half-space mesh
 unit of the real-space kernels: one directed neighbour pair inside the
 cutoff (each pair is evaluated from both atoms).
 """
+import math
+
 
 # structure factor rho(k) = sum_j w_j e^{ik.r_j}
 RHO_CHG = 10      # phase step 6 + 2 FMA (q weight)
@@ -89,3 +91,31 @@ def mixed_kspace_flops(kernel: str, natm: int, kmax, steps: int, n_scf_total: in
         return sum(3 * 2.0 * r * 2 * ch * k for r, k in calls)
     calls = [(2 * 3 * n1, nf)] * (steps + n_scf_total) + [(2 * (6 if efg else 3) * n1, natm)] * steps
     return sum(3 * 2.0 * rows * 2 * ch * c for c, rows in calls)
+
+
+def grid_extents(kmax) -> tuple:
+    """Points per axis of the reciprocal-space grid (grid.hip): at least 1.95
+    per wave number of -kmax .. kmax, x in steps of 16, y and z of 8."""
+    return tuple(-(-int(math.ceil(1.95 * (2 * k + 1))) // m) * m for k, m in zip(kmax, (16, 8, 8)))
+
+
+def grid_flops(kernel: str, natm: int, npol: int, kmax, steps: int, n_ind_total: int, efg: bool,
+               width: int) -> float:
+    """Algorithmic flops of the reciprocal sums through the grid over `steps`
+    evaluations (one static, one final call each) with `n_ind_total`
+    induced-dipole calls; width: points of the kernel per axis (17 in FP64,
+    10 in FP32).  Spread and interpolation: 4 flops per point of an atom's
+    support (2 for charges alone, 6 with second derivatives), the SCF's calls
+    over the polarizable atoms; transforms: the six folded cosine / sine
+    products of a call, without padding."""
+    w3 = float(width) ** 3
+    if kernel == "grid_spread":
+        return w3 * (steps * (2 + 4) * natm + n_ind_total * 4 * npol)
+    if kernel == "grid_gather":
+        return w3 * (steps * ((6 if efg else 4) * natm + 4 * npol) + n_ind_total * 4 * npol)
+    m1, m2, m3 = grid_extents(kmax)
+    k1, k2, k3 = kmax
+    z = m1 * m2 * (k3 + 1) * (m3 // 2) * 4.0
+    y = m1 * 2 * (k3 + 1) * (k2 + 1) * (m2 // 2) * 4.0
+    x = (2 * k2 + 1) * (k3 + 1) * 2 * (k1 + 1) * (m1 // 2) * 4.0
+    return 2.0 * (x + y + z) * (2 * steps + n_ind_total)
