@@ -1162,7 +1162,7 @@ void scf(mdffgpu_ctx* c, int itime, int* n_scf, double* rmsd_out, int* n_es,
   // their own, taken over when the solve goes on (not in the allocation-free
   // context, whose host memory is pageable, nor with induced quadrupoles).
   // An evaluation of 3000 atoms (14 iterations) 1.65 -> 1.38 ms, of 24,576
-  // (12 iterations) 4.28 -> 4.06 ms.
+  // (15 iterations) 4.28 -> 4.06 ms.
   const bool spec64 = !mixed_prec && !c->noalloc && !c->lqpol;
   const bool spec = mixed_prec || spec64;
   if (spec && !c->ev_sc) {
