@@ -1041,7 +1041,9 @@ void build_t2(mdffgpu_ctx* c) {
   da.rank = c->d_rank;
   da.perm = c->d_perm;
   da.dd16 = dd_idx16(n);
-  da.polmask = c->polmask;
+  // partners: the species that hold induced dipoles (k_induced), in FP64 the
+  // quadrupole-polarizable ones too
+  da.polmask = mx ? c->polmask : c->fieldmask;
   // the FP32 table with an FP32 static real-space pass: written by that
   // pass (the SCF's first Ewald call, after this one in every evaluation)
   if (mx) {

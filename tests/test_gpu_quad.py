@@ -57,6 +57,19 @@ def test_quadrupoles_match_oracle(oracle_lib, static, polar):
     assert np.abs(g["theta"]).max() > 0.0
 
 
+def test_quad_polarizable_species_with_a_dipole_polarizability(oracle_lib):
+    """O with lquad_polar but not ldip_polar beside dipole-polarizable Si: its
+    poldip still gives it an induced dipole (src/field.f90:1716-1803), which
+    is a source of the SCF field at the other polarizable atoms."""
+    s = _melt(True, True)
+    s.params.ldip_polar[0], s.params.ldip_polar[1] = 1, 0
+    for a in range(3):
+        s.params.poldip[16 * (a + 3 * a)] = 0.2
+    (g, o), = _both(oracle_lib, s, [s.r])
+    assert np.abs(o["mu"][s.itype == 2]).max() > 0.0
+    _check(g, o)
+
+
 def test_quadrupoles_aspc_trajectory(oracle_lib):
     """Induced quadrupoles with the ASPC predictor-corrector over a short
     trajectory (theta_ind zeroed by the predictor, polquad E from the
