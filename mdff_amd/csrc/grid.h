@@ -78,5 +78,8 @@ void adjoint_sums(Plan* p, hipStream_t st, const double* q, const double* mu, co
 // Points of one configuration's grid.
 size_t points(const Plan* p);
 
+// Doubles that pout and ind->rpart need at most.
+size_t partials(const Plan* p);
+
 }  // namespace grid
 }  // namespace mdff

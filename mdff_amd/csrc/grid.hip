@@ -1399,6 +1399,9 @@ static bool setup(Plan* p) {
              hipSuccess;
 }
 
+// blocks of k_grid_mid: 8 columns of the (n2, n3) plane each
+static int mid_blocks(const Ext& e) { return (e.NCC + 7) / 8; }
+
 // dynamic LDS of the kernels
 static size_t lds_fwd(const Ext& e) { return (size_t)e.M[1] * HS * sizeof(double); }
 static size_t lds_mid(const Ext& e) {
@@ -1477,6 +1480,12 @@ void set_cells(Plan* p, hipStream_t st, const std::vector<Seg>& segs) {
 }
 
 size_t points(const Plan* p) { return p->e.ng; }
+
+size_t partials(const Plan* p) {
+  // seven energy and stress rows of k_grid_mid, two rows of the SCF
+  // interpolation (at most a block per four atoms)
+  return std::max<size_t>((size_t)7 * mid_blocks(p->e), (size_t)2 * ((p->natom + 3) / 4));
+}
 bool binned(const Plan* p) { return p->is_binned; }
 void unbin(Plan* p) { p->is_binned = false; }
 
@@ -1565,7 +1574,7 @@ static void convolve(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, int split, doubl
   R* P = static_cast<R*>(p->d_P);
   const dim3 gf(e.M[0], (e.N3c + 15) / 16, e.nseg);
   k_grid_fwd<R><<<gf, MDFF_BLOCK, lds_fwd(e), st>>>(e, p->tw, split, G, p->d_T);
-  const dim3 gm((e.NCC + 7) / 8, e.nseg);
+  const dim3 gm(mid_blocks(e), e.nseg);
   EnArgs en;
   std::memset(&en, 0, sizeof(en));
   if (pout) {
@@ -1610,7 +1619,7 @@ static int sums_t(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,
   // about 4096 waves of a large system take the atoms in turn
   const int apw = std::max(1, count / (sizeof(R) == 8 ? 8192 : 4096));
   const int nb = (count + 4 * apw - 1) / (4 * apw);
-  if (count == 0) return ind ? 0 : (e.NCC + 7) / 8;
+  if (count == 0) return ind ? 0 : mid_blocks(e);
   const int gg = xcd_blocks(nb);
   CombineArgs ca;
   std::memset(&ca, 0, sizeof(ca));
@@ -1631,7 +1640,7 @@ static int sums_t(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,
     go(k_grid_gather<R, false, false, BA>);
   else
     go(k_grid_gather<R, false, false, 1>);
-  return ind ? nb : (e.NCC + 7) / 8;
+  return ind ? nb : mid_blocks(e);
 }
 
 int sums(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,

@@ -2380,6 +2380,7 @@ void create_impl(const mdffgpu_params* params, const int32_t* itype, const doubl
     if (grid_rule(c)) {
       c->gp = grid::create(c->st, grid_segs(c), c->kmax, grid_fp64(c));
       if (!c->gp) fail(c, MDFFGPU_ERR_ALLOC, "reciprocal-space grid");
+      ensure_part(c, grid::partials(c->gp));
     }
     if (c->P.precision == MDFFGPU_PREC_MIXED && !c->gp) {
       c->mx = mixed::create(c);

@@ -61,6 +61,17 @@ def test_grid_sums_match_oracle(oracle_lib, kmax, precision):
     ff.close()
 
 
+def test_grid_thin_mesh_matches_oracle(oracle_lib):
+    """kmax (1, 64, 64): the final call's energy partials (one set per eight
+    (n2, n3) columns) outnumber every other user of their buffer."""
+    from mdff_amd.field import ForceField
+    s = skewed_silica(24, 48, seed=6, kmax=(1, 64, 64), rc=4.5)
+    ff = ForceField(s.params, s.itype, s.A)
+    g = ff.engforce(s.r, itime=1)
+    ff.close()
+    compare_engforce(g, oracle_lib.Oracle(s.params, s.itype, s.A).engforce(s.r, itime=1))
+
+
 def test_grid_clustered_atoms(oracle_lib):
     """All atoms in one corner of a large cell: a few bins hold everything."""
     from mdff_amd.field import ForceField
