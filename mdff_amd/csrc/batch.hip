@@ -1135,11 +1135,14 @@ void grid_state(mdffgpu_batch* b) {
     b->gp = grid::create(b->st, segs, b->bc_h[0].kmax, !b->mixed);
     if (!b->gp) bfail(b, MDFFGPU_ERR_ALLOC, "reciprocal-space grid");
     b->grid_calls = !b->mixed || grid::points(b->gp) * segs.size() <= GRID_POINTS;
-    balloc(b, &b->d_adj, 4 * (size_t)b->N);
-    balloc(b, &b->d_v, 3 * (size_t)b->N);
-    balloc(b, &b->d_w, (size_t)b->N);
+  }
+  if (!b->d_apart) {
+    // also after a call that failed between these
+    if (!b->d_adj) balloc(b, &b->d_adj, 4 * (size_t)b->N);
+    if (!b->d_v) balloc(b, &b->d_v, 3 * (size_t)b->N);
+    if (!b->d_w) balloc(b, &b->d_w, (size_t)b->N);
     balloc(b, &b->d_apart, 9 * (size_t)b->N);
-    BCK(b, hipMemsetAsync(b->d_apart, 0, 9 * (size_t)b->N * sizeof(double), b->st));
+    fill(b, b->d_apart, 9 * (size_t)b->N, 0.0);
   }
   if (!grid::bin(b->gp, b->st, b->d_s4, b->d_typ, b->d_cfg, b->polmask, 0.0))
     bfail(b, MDFFGPU_ERR_ALLOC, "bins of the reciprocal-space grid");
@@ -1740,6 +1743,7 @@ void build_pairs(mdffgpu_batch* b) {
       b->allocs.erase(std::find(b->allocs.begin(), b->allocs.end(), b->d_t2));
     }
     b->d_t2 = nullptr;
+    b->t2_cap = 0;
     BCK(b, hipMalloc(&b->d_t2, need));
     b->allocs.push_back(b->d_t2);
     b->t2_cap = need;
@@ -1765,6 +1769,14 @@ void build_pairs(mdffgpu_batch* b) {
 
 void set_positions_impl(mdffgpu_batch* b, const double* d_pos) {
   const int N = b->N;
+  // nothing may run, nor a captured graph replay, on the buffers below until
+  // all of them are made anew
+  b->positions_set = false;
+  if (b->gexec) {
+    (void)hipGraphExecDestroy(b->gexec);
+    b->gexec = nullptr;
+    b->graph_iters = -1;
+  }
   BCK(b, hipMemcpyAsync(b->d_pos, d_pos, 3 * (size_t)N * sizeof(double),
                         hipMemcpyDeviceToDevice, b->st));
   k_b_prepare<<<nblk(N), MDFF_BLOCK, 0, b->st>>>(N, b->d_pos, b->d_cfg, b->d_bc, b->KX, b->KY,
@@ -1794,15 +1806,10 @@ void set_positions_impl(mdffgpu_batch* b, const double* d_pos) {
     else
       build_pairs<double>(b);
   }
-  b->positions_set = true;
   ++b->epoch;
   grid_state(b);
   if (b->mixed && !b->grid_calls) mx_state(b);  // allocates: never first inside a graph capture
-  if (b->gexec) {
-    (void)hipGraphExecDestroy(b->gexec);
-    b->gexec = nullptr;
-    b->graph_iters = -1;
-  }
+  b->positions_set = true;
 }
 
 // forward + backward on b->st; results in d_out, copied to h_out

@@ -1491,6 +1491,7 @@ void unbin(Plan* p) { p->is_binned = false; }
 
 bool bin(Plan* p, hipStream_t st, const double4* s4, const int* typ, const int* cfg,
          unsigned active, double drift) {
+  p->is_binned = false;  // until everything below has succeeded
   const Ext& e = p->e;
   const int n = p->natom;
   const int gn = (n + MDFF_BLOCK - 1) / MDFF_BLOCK;

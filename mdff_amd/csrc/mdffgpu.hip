@@ -1759,7 +1759,7 @@ void rebuild_list(mdffgpu_ctx* c) {
   hipStream_t st = c->st;
   HCK(c, hipMemcpyAsync(c->d_rref, c->d_pos, 3 * (size_t)n * sizeof(double),
                         hipMemcpyDeviceToDevice, st));
-  c->list_valid = true;
+  c->list_valid = false;  // until everything below has succeeded
   ++c->list_builds;
   {
     ProfScope _ps(c, K_NLIST);
@@ -1812,6 +1812,7 @@ void rebuild_list(mdffgpu_ctx* c) {
   // the grid's bins follow the list: no atom moves by more than skin/2
   // while it is valid
   if (c->gp) grid_bin(c, 0.5 * P.skindiff);
+  c->list_valid = true;
 }
 
 // The list rebuilt when invalid or when the skin test fails.

@@ -61,3 +61,106 @@ for kmax in ((1, 1, 1), (1, 58, 58), (2, 58, 58), (1, 64, 64), (2, 80, 80), (5, 
         L.mdffgpu_destroy(h)
         print(kmax, prec, seen, flush=True)
 """)
+
+
+# A call that has to grow the grid's tile lists: the displacement test asks for
+# a rebuild and the longest list comes out as GROWN; with `fail` the allocation
+# after it is refused.
+GROW = """
+import ctypes, host_hip as H
+import numpy as np
+from mdff_amd import configs as C, params as P
+names, arm, fail = [], set(), False
+def launch(name, gx, gy, gz, args):
+    names.append(name)
+    if b"k_disp" in name and "disp" in want:
+        arm.add("disp")
+    if b"k_grid_cap" in name and "cap" in want:
+        arm.add("cap")
+def d2h(dst, n):
+    if n == 4 and "cap" in arm:
+        arm.discard("cap")
+        ctypes.c_int.from_address(dst).value = GROWN
+    elif n == 8 and "disp" in arm:
+        arm.discard("disp")
+        ctypes.memset(dst, 0x41, n)
+def refuse(n, kind):
+    return 1 if fail and kind == 0 and any(b"k_grid_cap" in x for x in names) else 0
+want, GROWN = set(), 100000
+H.hooks(launch=launch, refuse=refuse, d2h=d2h)
+L = H.lib()
+"""
+
+
+def test_context_after_a_refused_bin_allocation(host_hip):
+    """The evaluation reports the error; the next one bins again before any
+    kernel reads the lists."""
+    host_hip(GROW + """
+s = C.silica(20, 40, seed=8, rc=4.0, kmax=3, pim=False)
+st, h = H.create(L, s)
+assert st == 0
+assert H.engforce_device(L, h, s.r) == 0
+del names[:]
+want.update(("disp", "cap"))
+fail = True
+assert H.engforce_device(L, h, s.r) == 3
+assert any(b"k_grid_cap" in x for x in names)
+assert not any(b"k_grid_lists" in x for x in names)
+fail = False
+want.clear()
+del names[:]
+assert H.engforce_device(L, h, s.r) == 0
+order = [k for x in names for k in (b"k_grid_bin", b"k_grid_lists") if k in x]
+assert order == [b"k_grid_bin", b"k_grid_lists"], order
+""")
+
+
+def test_batch_after_a_refused_allocation(host_hip):
+    """A batch whose set_positions failed refuses evaluations (its lists are
+    gone) until one succeeds."""
+    host_hip(GROW + """
+from mdff_amd import _lib
+_lib._lib = L
+from mdff_amd.batch import Batch
+systems = [C.silica(n, 2 * n, seed=30 + n, rc=4.5, kmax=4, pim=True, pot_seed=3) for n in (16, 21)]
+r = np.ascontiguousarray(np.concatenate([s.r for s in systems]).T)
+tgt, loss = np.zeros_like(r), ctypes.c_double()
+for prec in (P.PREC_FP64, P.PREC_MIXED):
+    b = Batch.from_systems(systems, precision=prec)
+    grad = np.zeros(b.nparam)
+    def evaluate():
+        return L.mdffgpu_batch_loss_grad(b._h, tgt.ctypes.data, None, ctypes.byref(loss),
+                                         grad.ctypes.data_as(H.dp), 3, None, None, None)
+    def positions():
+        del names[:]
+        return L.mdffgpu_batch_set_positions(b._h, r.ctypes.data, None)
+    # every allocation of the first call in turn
+    left = [0]
+    def refuse_nth(n, kind):
+        left[0] -= 1
+        return 1 if left[0] == 0 else 0
+    H.hooks(launch=launch, refuse=refuse_nth)
+    failed = 0
+    for nth in range(1, 64):
+        left[0] = nth
+        st = positions()
+        if left[0] > 0:
+            break
+        left[0] = 0
+        if st:
+            failed += 1
+            assert evaluate() == 1, (prec, nth)
+    assert st == 0 and failed > 0
+    assert evaluate() == 0
+    # and the growth of the lists
+    H.hooks(launch=launch, refuse=refuse, d2h=d2h)
+    want.add("cap")
+    fail = True
+    assert positions() == 3
+    assert evaluate() == 1
+    fail = False
+    want.clear()
+    assert positions() == 0
+    assert evaluate() == 0
+    b.close()
+""")
