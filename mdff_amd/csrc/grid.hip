@@ -43,6 +43,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -129,11 +130,16 @@ struct Plan {
   void* d_P = nullptr;       // potentials, [seg][x][y][M3 + PADZ]
   // bins: two classes (active atoms, the others) of nseg x ntile bins
   int *d_key = nullptr, *d_start = nullptr, *d_cur = nullptr, *d_perm0 = nullptr,
-      *d_perm = nullptr, *d_cap = nullptr;
+      *d_perm = nullptr;
   int margin[3] = {0, 0, 0};
-  int cap = 0, cap_alloc = 0;  // entries per tile of the lists
-  int2* d_ov = nullptr;   // tile lists
-  int2* d_cnt = nullptr;  // their lengths (active, all)
+  // tile lists one after the other, each with room for its candidates at the
+  // binning: the first slots (one more than tiles), their number and the
+  // slots allocated; per tile (first slot, active atoms, all atoms)
+  int* d_off = nullptr;
+  unsigned long long* d_total = nullptr;
+  long long slots = 0;
+  int2* d_ov = nullptr;
+  int4* d_cnt = nullptr;
   int nact = 0;           // active atoms
   int split = 1;          // partial grids of the spread
   bool is_binned = false;
@@ -342,11 +348,12 @@ struct Margin {
   int m[3];
 };
 
-// Longest candidate list of any tile.
+// Candidates of every tile (room[tile + 1], for k_cell_scan) and of all.
 template <int W>
 __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_cap(Ext e, Margin mg,
                                                          const int* __restrict__ start,
-                                                         int* __restrict__ cap) {
+                                                         int* __restrict__ room,
+                                                         unsigned long long* __restrict__ total) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= e.ntile * e.nseg) return;
   const Cands<W> c(e, mg.m, t % e.ntile);
@@ -354,7 +361,9 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_cap(Ext e, Margin mg,
   for (int cls = 0; cls < 2; ++cls)
     for (int r = 0; r < c.rows; ++r)
       tot += c.run(e, start, (cls * e.nseg + t / e.ntile) * e.ntile, r).y;
-  atomicMax(cap, tot);
+  if (t == 0) room[0] = 0;
+  room[t + 1] = tot;
+  atomicAdd(total, (unsigned long long)tot);
 }
 
 // ---------------------------------------------------------------------------
@@ -362,17 +371,19 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_cap(Ext e, Margin mg,
 
 // The atoms whose support overlaps a tile, active atoms first, each class in
 // bin order, as (atom, offsets of the support's start from the tile + 64 in
-// three bytes); cnt = (active, all).  One workgroup per tile tests the
+// three bytes); cnt = (first slot, active, all).  One workgroup per tile tests the
 // candidates of the neighbouring bins and compacts the hits with ballots, so
 // that the order is fixed.
 template <int W>
 __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_lists(
     Ext e, Margin mg, const double4* __restrict__ s4, const int* __restrict__ start,
-    const int* __restrict__ perm, int cap, int2* __restrict__ ov, int2* __restrict__ cnt) {
+    const int* __restrict__ perm, const int* __restrict__ off, int2* __restrict__ ov,
+    int4* __restrict__ cnt) {
   __shared__ int first[MDFF_BLOCK], pre[MDFF_BLOCK + 1], wsum[4];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int tile = blockIdx.x, seg = blockIdx.y;
   const size_t at = (size_t)seg * e.ntile + tile;
+  const int first_slot = off[at], cap = off[at + 1] - first_slot;
   const int z0 = (tile % e.nt[2]) * TZ, y0 = ((tile / e.nt[2]) % e.nt[1]) * TY,
             x0 = tile / (e.nt[2] * e.nt[1]) * TX;
   const Cands<W> c(e, mg.m, tile);
@@ -432,14 +443,14 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_lists(
           if (k < wv) po += wsum[k];
           nov += wsum[k];
         }
-        if (o && po < cap) ov[at * cap + po] = ent;
+        if (o && po < cap) ov[(size_t)first_slot + po] = ent;
         __syncthreads();
       }
       __syncthreads();
     }
     if (cls == 0) act = nov;
   }
-  if (t == 0) cnt[at] = make_int2(min(act, cap), min(nov, cap));
+  if (t == 0) cnt[at] = make_int4(first_slot, min(act, cap), min(nov, cap), 0);
 }
 
 // Kernel values of every atom: tab[atom][axis][phi, phi'][W] and
@@ -510,7 +521,7 @@ template <typename R, bool CHG, bool DIP>
 __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_spread(
     Ext e, const Seg* __restrict__ segs, const double* __restrict__ q,
     const double* __restrict__ mu, int n, const R* __restrict__ tab,
-    const int2* __restrict__ list, const int2* __restrict__ cnt, int cap, int act,
+    const int2* __restrict__ list, const int4* __restrict__ cnt, int act,
     R* __restrict__ G) {
   constexpr int W = Mat<R>::W;
   typedef typename Mat<R>::acc acc_t;
@@ -523,12 +534,12 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_spread(
   if (tile >= e.ntile) return;
   const size_t at = (size_t)seg * e.ntile + tile;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int2 cc = cnt[at];
+  const int4 cc = cnt[at];
   // this block's share of the list (gridDim.z partial grids)
-  const int tot = act ? cc.x : cc.y;
+  const int tot = act ? cc.y : cc.z;
   const int lo = (int)((long long)tot * blockIdx.z / gridDim.z);
   const int m = (int)((long long)tot * (blockIdx.z + 1) / gridDim.z) - lo;
-  const int2* lst = list + at * cap + lo;
+  const int2* lst = list + (size_t)cc.x + lo;
   const int z0 = (tile % e.nt[2]) * TZ, y0 = ((tile / e.nt[2]) % e.nt[1]) * TY,
             x0 = tile / (e.nt[2] * e.nt[1]) * TX;
   const Cell& cell = segs[seg].cell;
@@ -643,7 +654,7 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_spread_adj(
     Ext e, const Seg* __restrict__ segs, const double* __restrict__ q,
     const double* __restrict__ mu, const double* __restrict__ gv, int n,
     const R* __restrict__ tab, const R* __restrict__ tab2, const int2* __restrict__ list,
-    const int2* __restrict__ cnt, int cap, R* __restrict__ G) {
+    const int4* __restrict__ cnt, R* __restrict__ G) {
   constexpr int W = Mat<R>::W;
   typedef typename Mat<R>::acc acc_t;
   __shared__ R lx[SCH][3][TX], ly[SCH][3][TY], lz[SCH][3][TZ];
@@ -653,8 +664,9 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_spread_adj(
   if (tile >= e.ntile) return;
   const size_t at = (size_t)seg * e.ntile + tile;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const int m = cnt[at].y;
-  const int2* lst = list + at * cap;
+  const int4 cc = cnt[at];
+  const int m = cc.z;
+  const int2* lst = list + (size_t)cc.x;
   const int z0 = (tile % e.nt[2]) * TZ, y0 = ((tile / e.nt[2]) % e.nt[1]) * TY,
             x0 = tile / (e.nt[2] * e.nt[1]) * TX;
   const Cell& cell = segs[seg].cell;
@@ -1443,7 +1455,8 @@ Plan* create(hipStream_t st, const std::vector<Seg>& segs, const int kmax[3], bo
        take(p, &p->d_D, e.nseg * e.nm) && take(p, &p->d_key, p->natom) &&
        take(p, &p->d_start, nb + 1) && take(p, &p->d_cur, nb + 1) &&
        take(p, &p->d_perm0, p->natom) && take(p, &p->d_perm, p->natom) &&
-       take(p, &p->d_cap, 1) && take(p, &p->d_cnt, (size_t)e.nseg * e.ntile);
+       take(p, &p->d_total, 1) && take(p, &p->d_off, (size_t)e.nseg * e.ntile + 1) &&
+       take(p, &p->d_cnt, (size_t)e.nseg * e.ntile);
   // more LDS than the default limit of a launch
   const std::pair<const void*, size_t> big[] = {
       {fp64 ? (void*)k_grid_fwd<double> : (void*)k_grid_fwd<float>, lds_fwd(e)},
@@ -1509,7 +1522,7 @@ bool bin(Plan* p, hipStream_t st, const double4* s4, const int* typ, const int* 
     p->margin[a] = mg.m[a];
   }
   k_cell_zero<<<(nb + 1 + MDFF_BLOCK - 1) / MDFF_BLOCK, MDFF_BLOCK, 0, st>>>(nb + 1, p->d_start);
-  k_cell_zero<<<1, MDFF_BLOCK, 0, st>>>(1, p->d_cap);
+  k_cell_zero<<<1, MDFF_BLOCK, 0, st>>>(2, reinterpret_cast<int*>(p->d_total));
   if (p->fp64)
     k_grid_bin<W64><<<gn, MDFF_BLOCK, 0, st>>>(n, e, s4, typ, cfg, active, p->d_key, p->d_start);
   else
@@ -1517,28 +1530,31 @@ bool bin(Plan* p, hipStream_t st, const double4* s4, const int* typ, const int* 
   k_cell_scan<<<1, 1024, 0, st>>>(nb, p->d_start, p->d_cur);
   k_cell_fill<<<gn, MDFF_BLOCK, 0, st>>>(n, p->d_key, p->d_cur, p->d_perm0);
   k_cell_order<<<gn, MDFF_BLOCK, 0, st>>>(n, p->d_key, p->d_start, p->d_perm0, p->d_perm, nullptr);
-  const int gt = (e.nseg * e.ntile + MDFF_BLOCK - 1) / MDFF_BLOCK;
+  const int ntile = e.nseg * e.ntile;
+  const int gt = (ntile + MDFF_BLOCK - 1) / MDFF_BLOCK;
   if (p->fp64)
-    k_grid_cap<W64><<<gt, MDFF_BLOCK, 0, st>>>(e, mg, p->d_start, p->d_cap);
+    k_grid_cap<W64><<<gt, MDFF_BLOCK, 0, st>>>(e, mg, p->d_start, p->d_off, p->d_total);
   else
-    k_grid_cap<W32><<<gt, MDFF_BLOCK, 0, st>>>(e, mg, p->d_start, p->d_cap);
-  int cap = 0;
-  if (hipMemcpyAsync(&cap, p->d_cap, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess ||
+    k_grid_cap<W32><<<gt, MDFF_BLOCK, 0, st>>>(e, mg, p->d_start, p->d_off, p->d_total);
+  k_cell_scan<<<1, 1024, 0, st>>>(ntile, p->d_off, p->d_cur);
+  unsigned long long total = 0;
+  if (hipMemcpyAsync(&total, p->d_total, sizeof(total), hipMemcpyDeviceToHost, st) != hipSuccess ||
       hipMemcpyAsync(&p->nact, p->d_start + nb / 2, sizeof(int), hipMemcpyDeviceToHost, st) !=
           hipSuccess ||
       hipStreamSynchronize(st) != hipSuccess)
     return false;
-  p->cap = std::max(cap, 1);
-  if (p->cap > p->cap_alloc) {
+  if (total > (unsigned long long)INT_MAX) return false;  // slots are ints
+  if ((long long)total + 1 > p->slots) {
     release(p, p->d_ov);
     p->d_ov = nullptr;
-    p->cap_alloc = 0;
-    const int c = p->cap + p->cap / 8 + 8;
-    if (!take(p, &p->d_ov, (size_t)e.nseg * e.ntile * c)) {
+    p->slots = 0;
+    // one slot past the last list: a tile without atoms reads it, unused
+    const size_t c = total + total / 8 + 8;
+    if (!take(p, &p->d_ov, c)) {
       (void)hipGetLastError();
       return false;
     }
-    p->cap_alloc = c;
+    p->slots = (long long)c;
   }
   p->cfg = cfg;
   p->is_binned = true;
@@ -1554,12 +1570,12 @@ void prepare(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double4* s4) {
   const long long work = (long long)p->natom * 3 * (p->fp64 ? W64 : W32);
   const int gt = (int)std::min<long long>((work + MDFF_BLOCK - 1) / MDFF_BLOCK, 2048);
   if (p->fp64) {
-    k_grid_lists<W64><<<g, MDFF_BLOCK, 0, st>>>(e, mg, s4, p->d_start, p->d_perm, p->cap, p->d_ov,
+    k_grid_lists<W64><<<g, MDFF_BLOCK, 0, st>>>(e, mg, s4, p->d_start, p->d_perm, p->d_off, p->d_ov,
                                                 p->d_cnt);
     k_grid_tab<double><<<gt, MDFF_BLOCK, 0, st>>>(p->natom, e, s4, (const double*)p->d_poly,
                                                   (double*)p->d_tab, (double*)p->d_tab2, (int*)p->d_l0);
   } else {
-    k_grid_lists<W32><<<g, MDFF_BLOCK, 0, st>>>(e, mg, s4, p->d_start, p->d_perm, p->cap, p->d_ov,
+    k_grid_lists<W32><<<g, MDFF_BLOCK, 0, st>>>(e, mg, s4, p->d_start, p->d_perm, p->d_off, p->d_ov,
                                                 p->d_cnt);
     k_grid_tab<float><<<gt, MDFF_BLOCK, 0, st>>>(p->natom, e, s4, (const float*)p->d_poly,
                                                  (float*)p->d_tab, (float*)p->d_tab2, (int*)p->d_l0);
@@ -1606,13 +1622,13 @@ static int sums_t(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q,
     ProfScope _ps(ctx, K_GRID_SPREAD);
     if (chg && dip)
       k_grid_spread<R, true, true><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab, p->d_ov,
-                                                              p->d_cnt, p->cap, sa, G);
+                                                              p->d_cnt, sa, G);
     else if (dip)
       k_grid_spread<R, false, true><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab,
-                                                               p->d_ov, p->d_cnt, p->cap, sa, G);
+                                                               p->d_ov, p->d_cnt, sa, G);
     else
       k_grid_spread<R, true, false><<<gt, MDFF_BLOCK, 0, st>>>(e, p->d_seg, q, mu, n, tab,
-                                                               p->d_ov, p->d_cnt, p->cap, sa, G);
+                                                               p->d_ov, p->d_cnt, sa, G);
   }
   convolve<R>(p, ctx, st, p->split, pout);
   ProfScope _ps(ctx, K_GRID_GATHER);
@@ -1660,7 +1676,7 @@ static void adjoint_t(Plan* p, hipStream_t st, const double* q, const double* mu
   const R* tab = static_cast<const R*>(p->d_tab);
   const R* tab2 = static_cast<const R*>(p->d_tab2);
   k_grid_spread_adj<R><<<dim3(xcd_blocks(e.ntile), e.nseg), MDFF_BLOCK, 0, st>>>(
-      e, p->d_seg, q, mu, g, n, tab, tab2, p->d_ov, p->d_cnt, p->cap, static_cast<R*>(p->d_G));
+      e, p->d_seg, q, mu, g, n, tab, tab2, p->d_ov, p->d_cnt, static_cast<R*>(p->d_G));
   convolve<R>(p, nullptr, st, 1, nullptr);
   CombineArgs ca;
   std::memset(&ca, 0, sizeof(ca));

@@ -85,6 +85,26 @@ def test_grid_clustered_atoms(oracle_lib):
     compare_engforce(g, oracle_lib.Oracle(p, s.itype, A).engforce(s.r, itime=1))
 
 
+def test_grid_lists_of_a_droplet_take_the_memory_of_its_atoms():
+    """1,800 atoms in one corner of a cell of 13,500 tiles.  An atom is a
+    candidate of at most 4 x 5 x 5 tiles (support and skin over tiles of 16 x
+    8 x 8 points), 8 bytes each: 1.4 MB, and the neighbour list and pair tables
+    of at most 1,800 entries per row.  Room for the longest list in every
+    tile would be 190 MB."""
+    import torch
+    from mdff_amd.field import ForceField
+    s = C.silica(600, 1200, seed=8, rc=4.0, kmax=9, pim=False)
+    A = 6.0 * s.A
+    s.params.kES[:] = [60, 60, 60]
+    ff = ForceField(s.params, s.itype, A)
+    free0 = torch.cuda.mem_get_info()[0]
+    g = ff.engforce(s.r, itime=1)
+    used = free0 - torch.cuda.mem_get_info()[0]
+    ff.close()
+    assert np.isfinite(g["f"]).all()
+    assert used < 64 << 20, used
+
+
 def test_grid_batch_matches_oracle(oracle_lib):
     """FP64 batch with a common, unequal-axes kmax (one plan over uneven
     configurations) against the oracle, configuration by configuration, and

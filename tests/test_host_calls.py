@@ -64,7 +64,7 @@ for kmax in ((1, 1, 1), (1, 58, 58), (2, 58, 58), (1, 64, 64), (2, 80, 80), (5, 
 
 
 # A call that has to grow the grid's tile lists: the displacement test asks for
-# a rebuild and the longest list comes out as GROWN; with `fail` the allocation
+# a rebuild and the entries of the lists come out as GROWN; with `fail` the allocation
 # after it is refused.
 GROW = """
 import ctypes, host_hip as H
@@ -78,9 +78,9 @@ def launch(name, gx, gy, gz, args):
     if b"k_grid_cap" in name and "cap" in want:
         arm.add("cap")
 def d2h(dst, n):
-    if n == 4 and "cap" in arm:
+    if n == 8 and "cap" in arm:
         arm.discard("cap")
-        ctypes.c_int.from_address(dst).value = GROWN
+        ctypes.c_longlong.from_address(dst).value = GROWN
     elif n == 8 and "disp" in arm:
         arm.discard("disp")
         ctypes.memset(dst, 0x41, n)
