@@ -894,7 +894,8 @@ struct mdffgpu_batch {
   // reciprocal sums through the uniform grid (configurations with a common
   // kmax), its U, V sums per atom
   mdff::grid::Plan* gp = nullptr;
-  bool grid_calls = false;  // the Ewald calls go through it (grid_state)
+  bool grid_calls = false;    // the Ewald calls go through it (grid_state)
+  bool grid_refused = false;  // its memory was refused
   double *d_apart = nullptr, *d_adj = nullptr, *d_v = nullptr, *d_w = nullptr;
   long long epoch = 0;
   int pol_type[MDFF_NT];
@@ -1123,7 +1124,9 @@ bool common_kmax(const mdffgpu_batch* b) {
 // 1536 (4.9 M points) 19.4 against 22.6 ms.
 constexpr size_t GRID_POINTS = 2500000;
 void grid_state(mdffgpu_batch* b) {
-  if (!b->P.lcoulomb || !common_kmax(b)) return;
+  if (!b->P.lcoulomb || !common_kmax(b) || b->grid_refused) return;
+  const size_t N = b->N;
+  bool ok = true;
   if (!b->gp) {
     std::vector<grid::Seg> segs(b->bc_h.size());
     for (size_t c = 0; c < segs.size(); ++c) {
@@ -1133,19 +1136,30 @@ void grid_state(mdffgpu_batch* b) {
       segs[c].n = b->bc_h[c].n;
     }
     b->gp = grid::create(b->st, segs, b->bc_h[0].kmax, !b->mixed);
-    if (!b->gp) bfail(b, MDFFGPU_ERR_ALLOC, "reciprocal-space grid");
-    b->grid_calls = !b->mixed || grid::points(b->gp) * segs.size() <= GRID_POINTS;
+    ok = b->gp != nullptr;
+    auto take = [&](double** p, size_t count) {
+      ok = ok && hipMalloc((void**)p, count * sizeof(double)) == hipSuccess;
+      if (ok) b->allocs.push_back(*p);
+    };
+    take(&b->d_adj, 4 * N);
+    take(&b->d_v, 3 * N);
+    take(&b->d_w, N);
+    take(&b->d_apart, 9 * N);
+    if (ok) {
+      fill(b, b->d_apart, 9 * N, 0.0);
+      b->grid_calls = !b->mixed || grid::points(b->gp) * segs.size() <= GRID_POINTS;
+    }
   }
-  if (!b->d_apart) {
-    // also after a call that failed between these
-    if (!b->d_adj) balloc(b, &b->d_adj, 4 * (size_t)b->N);
-    if (!b->d_v) balloc(b, &b->d_v, 3 * (size_t)b->N);
-    if (!b->d_w) balloc(b, &b->d_w, (size_t)b->N);
-    balloc(b, &b->d_apart, 9 * (size_t)b->N);
-    fill(b, b->d_apart, 9 * (size_t)b->N, 0.0);
+  if (!ok || !grid::bin(b->gp, b->st, b->d_s4, b->d_typ, b->d_cfg, b->polmask, 0.0)) {
+    // without the memory for the grid the batch goes on with the direct sums
+    // and the tangent gradients
+    (void)hipGetLastError();
+    grid::destroy(b->gp);
+    b->gp = nullptr;
+    b->grid_calls = false;
+    b->grid_refused = true;
+    return;
   }
-  if (!grid::bin(b->gp, b->st, b->d_s4, b->d_typ, b->d_cfg, b->polmask, 0.0))
-    bfail(b, MDFFGPU_ERR_ALLOC, "bins of the reciprocal-space grid");
   grid::prepare(b->gp, nullptr, b->st, b->d_s4);
   launch_check(b, "batch grid bins");
 }

@@ -33,7 +33,7 @@ bool supported(const int kmax[3]);
 
 // Plan for configurations that share kmax; fp64: grid and kernel tables in
 // double (support 16), else in float (support 10; transforms in double).
-// Null when device memory runs out.
+// Null when device memory runs out (the caller has the direct sums).
 Plan* create(hipStream_t st, const std::vector<Seg>& segs, const int kmax[3], bool fp64);
 void destroy(Plan* p);
 
@@ -44,7 +44,7 @@ void set_cells(Plan* p, hipStream_t st, const std::vector<Seg>& segs);
 // Atoms of a species with its bit in `active` come first in their own bins:
 // the calls over the active atoms alone read those.  Until the next call no
 // atom may move by more than drift (a length).  Waits for the stream; false
-// when device memory runs out.
+// when device memory runs out: the plan is of no use then.
 bool bin(Plan* p, hipStream_t st, const double4* s4, const int* typ, const int* cfg,
          unsigned active, double drift);
 bool binned(const Plan* p);

@@ -1743,12 +1743,38 @@ void update_floor(mdffgpu_ctx* c) {
     c->mx_floor = std::min(c->mx_floor, c->scf_best);
 }
 
+// Fractional coordinates of the positions in d_pos and, where the direct
+// reciprocal sums of this call need them (phases), their phases.
+void prepare(mdffgpu_ctx* c, bool phases) {
+  {
+    ProfScope _ps(c, K_PREPARE);
+    k_prepare<<<nblk(c->n), MDFF_BLOCK, 0, c->st>>>(c->n, c->d_pos, c->cell,
+                                                    c->renum ? c->d_int2ext : nullptr, c->d_typ,
+                                                    c->d_s, c->d_s4, phases ? c->d_eph : nullptr);
+  }
+  check_launch(c, "k_prepare");
+}
+
+// Without the memory for the grid (plan or bins) the context goes on with the
+// direct sums.
+void direct_sums(mdffgpu_ctx* c) {
+  grid::destroy(c->gp);
+  c->gp = nullptr;
+  if (c->P.precision != MDFFGPU_PREC_MIXED || c->mx) return;
+  c->mx = mixed::create(c);
+  if (!c->mx) fail(c, MDFFGPU_ERR_UNSUPPORTED, "mixed-precision path unavailable");
+  mx_active(c);
+}
+
 // Bins of the grid at the current positions, good for displacements up to
 // drift.
 void grid_bin(mdffgpu_ctx* c, double drift) {
-  if (!grid::bin(c->gp, c->st, c->d_s4, c->d_typ, nullptr, c->polmask, drift))
-    fail(c, MDFFGPU_ERR_ALLOC, "bins of the reciprocal-space grid");
-  check_launch(c, "grid bins");
+  if (grid::bin(c->gp, c->st, c->d_s4, c->d_typ, nullptr, c->polmask, drift)) {
+    check_launch(c, "grid bins");
+    return;
+  }
+  direct_sums(c);
+  prepare(c, true);  // the phases that the grid does not need
 }
 
 // Verlet list of the current positions (s4), grown until it holds every row.
@@ -1911,13 +1937,8 @@ void run(mdffgpu_ctx* c, int itime, mdffgpu_energies* en) {
   const int gb = nblk(n);
   hipStream_t st = c->st;
   std::memset(en, 0, sizeof(*en));
-  {
-    ProfScope _ps(c, K_PREPARE);
-    k_prepare<<<gb, MDFF_BLOCK, 0, st>>>(n, c->d_pos, c->cell, c->renum ? c->d_int2ext : nullptr,
-                                         c->d_typ, c->d_s, c->d_s4,
-                                         P.lcoulomb && !c->gp ? c->d_eph : nullptr);
-  }
-  check_launch(c, "k_prepare");
+  if (!c->gp) direct_sums(c);
+  prepare(c, P.lcoulomb && !c->gp);
   update_list(c);
   if (c->gp) grid::prepare(c->gp, c, st, c->d_s4);
   if (P.lcoulomb && c->linduced) build_t2(c);
@@ -2086,13 +2107,8 @@ void efg_frame(mdffgpu_ctx* c, const mdffgpu_efg_opts& o, mdffgpu_energies* en) 
   hipStream_t st = c->st;
   const bool ewald = (o.longrange == 0);
   ++c->evals;
-  {
-    ProfScope _ps(c, K_PREPARE);
-    k_prepare<<<gb, MDFF_BLOCK, 0, st>>>(n, c->d_pos, c->cell, c->renum ? c->d_int2ext : nullptr,
-                                         c->d_typ, c->d_s, c->d_s4,
-                                         c->gp && grid_fp64(c) ? nullptr : c->d_eph);
-  }
-  check_launch(c, "k_prepare");
+  if (!c->gp) direct_sums(c);
+  prepare(c, !(c->gp && grid_fp64(c)));
   // get_moments (src/field.f90:3686-3765) with calc = 'efg': the SCF starts
   // from the static field, no extrapolation
   std::memset(en, 0, sizeof(*en));
@@ -2174,13 +2190,15 @@ void efg_frame(mdffgpu_ctx* c, const mdffgpu_efg_opts& o, mdffgpu_energies* en) 
     ca.ndir = js;
     // reciprocal space: charge_density_k (src/efg.f90:2888-2930) and the
     // EFG of every k (:1507-1556), on the FP64 structure-factor kernels
-    if (c->gp && grid_fp64(c)) {
-      if (!c->linduced) {
-        // no list of this frame: bins of its positions alone
-        grid_bin(c, 0.0);
+    if (c->gp && grid_fp64(c) && !c->linduced) {
+      // no list of this frame: bins of its positions alone
+      grid_bin(c, 0.0);
+      if (c->gp) {
         grid::prepare(c->gp, c, st, c->d_s4);
         grid::unbin(c->gp);
       }
+    }
+    if (c->gp && grid_fp64(c)) {
       grid::sums(c->gp, c, st, q, mu, true, dip, true, false, false, c->d_apart, nullptr);
       check_launch(c, "grid sums");
       ca.rec = c->d_apart;
@@ -2378,16 +2396,11 @@ void create_impl(const mdffgpu_params* params, const int32_t* itype, const doubl
     if (c->P.lcoulomb) build_kmesh(c);
     size_t need = 12 * (size_t)std::max(nblk(c->kpad), nblk(c->n * LPA)) + 4096;
     ensure_part(c, need);
-    if (grid_rule(c)) {
-      c->gp = grid::create(c->st, grid_segs(c), c->kmax, grid_fp64(c));
-      if (!c->gp) fail(c, MDFFGPU_ERR_ALLOC, "reciprocal-space grid");
+    if (grid_rule(c)) c->gp = grid::create(c->st, grid_segs(c), c->kmax, grid_fp64(c));
+    if (c->gp)
       ensure_part(c, grid::partials(c->gp));
-    }
-    if (c->P.precision == MDFFGPU_PREC_MIXED && !c->gp) {
-      c->mx = mixed::create(c);
-      if (!c->mx) fail(c, MDFFGPU_ERR_UNSUPPORTED, "mixed-precision path unavailable");
-      mx_active(c);
-    }
+    else
+      direct_sums(c);
     // the clears of alloc_atoms are done before the context is handed out
     HCK(c, hipStreamSynchronize(c->st));
     *out = c;

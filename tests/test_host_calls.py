@@ -93,31 +93,74 @@ L = H.lib()
 
 
 def test_context_after_a_refused_bin_allocation(host_hip):
-    """The evaluation reports the error; the next one bins again before any
-    kernel reads the lists."""
+    """The evaluation goes on with the direct sums, the phases of which it
+    makes, and so do the next ones; nothing reads the lists."""
     host_hip(GROW + """
-s = C.silica(20, 40, seed=8, rc=4.0, kmax=3, pim=False)
-st, h = H.create(L, s)
-assert st == 0
-assert H.engforce_device(L, h, s.r) == 0
-del names[:]
-want.update(("disp", "cap"))
-fail = True
-assert H.engforce_device(L, h, s.r) == 3
-assert any(b"k_grid_cap" in x for x in names)
-assert not any(b"k_grid_lists" in x for x in names)
-fail = False
-want.clear()
-del names[:]
-assert H.engforce_device(L, h, s.r) == 0
-order = [k for x in names for k in (b"k_grid_bin", b"k_grid_lists") if k in x]
-assert order == [b"k_grid_bin", b"k_grid_lists"], order
+for prec, direct in ((P.PREC_FP64, b"k_rho64"), (P.PREC_MIXED, b"mx_rho")):
+    s = C.silica(20, 40, seed=8, rc=4.0, kmax=3, pim=False)
+    s.params.precision = prec
+    st, h = H.create(L, s)
+    assert st == 0
+    assert H.engforce_device(L, h, s.r) == 0
+    assert any(b"k_grid_lists" in x for x in names)
+    del names[:]
+    want.update(("disp", "cap"))
+    fail = True
+    # the failure of everything after the bins reaches the mixed path's own
+    # allocations too: that call reports it and the next one makes them
+    assert H.engforce_device(L, h, s.r) == (0 if prec == P.PREC_FP64 else 6)
+    assert any(b"k_grid_cap" in x for x in names)
+    assert not any(b"k_grid_lists" in x for x in names)
+    fail = False
+    want.clear()
+    for again in range(2):
+        if prec == P.PREC_MIXED or again:
+            del names[:]
+            assert H.engforce_device(L, h, s.r) == 0
+        assert any(direct in x for x in names), names
+        if prec == P.PREC_FP64 and not again:
+            bins = max(k for k, x in enumerate(names) if b"k_grid_cap" in x)
+            assert any(b"k_prepare" in x for x in names[bins:])
+        else:
+            assert not any(b"k_grid" in x for x in names), names
+    L.mdffgpu_destroy(h)
+""")
+
+
+def test_context_without_memory_for_the_grid(host_hip):
+    """Every allocation of a creation refused in turn: those of the grid leave
+    a context that takes the direct sums, the others an error."""
+    host_hip(GROW + """
+left = [0]
+def refuse_nth(n, kind):
+    left[0] -= 1
+    return 1 if left[0] == 0 else 0
+H.hooks(launch=launch, refuse=refuse_nth)
+for prec, direct in ((P.PREC_FP64, b"k_rho64"), (P.PREC_MIXED, b"mx_rho")):
+    s = C.silica(20, 40, seed=8, rc=4.0, kmax=3, pim=True)
+    s.params.precision = prec
+    kept = 0
+    for nth in range(1, 200):
+        left[0] = nth
+        st, h = H.create(L, s)
+        if left[0] > 0:
+            break
+        if st:
+            continue
+        kept += 1
+        del names[:]
+        assert H.engforce_device(L, h, s.r) == 0
+        assert any(direct in x for x in names) and not any(b"k_grid" in x for x in names)
+        L.mdffgpu_destroy(h)
+    assert st == 0 and kept >= 10, kept
+    L.mdffgpu_destroy(h)
 """)
 
 
 def test_batch_after_a_refused_allocation(host_hip):
     """A batch whose set_positions failed refuses evaluations (its lists are
-    gone) until one succeeds."""
+    gone) until one succeeds; without the memory for the grid it takes the
+    direct sums."""
     host_hip(GROW + """
 from mdff_amd import _lib
 _lib._lib = L
@@ -134,32 +177,43 @@ for prec in (P.PREC_FP64, P.PREC_MIXED):
     def positions():
         del names[:]
         return L.mdffgpu_batch_set_positions(b._h, r.ctypes.data, None)
-    # every allocation of the first call in turn
+    # every allocation of the first calls in turn, a batch each
     left = [0]
     def refuse_nth(n, kind):
         left[0] -= 1
         return 1 if left[0] == 0 else 0
-    H.hooks(launch=launch, refuse=refuse_nth)
-    failed = 0
+    failed = direct = 0
     for nth in range(1, 64):
+        b = Batch.from_systems(systems, precision=prec)
+        H.hooks(launch=launch, refuse=refuse_nth)
         left[0] = nth
         st = positions()
         if left[0] > 0:
             break
-        left[0] = 0
         if st:
             failed += 1
             assert evaluate() == 1, (prec, nth)
-    assert st == 0 and failed > 0
-    assert evaluate() == 0
+            assert positions() == 0
+            assert evaluate() == 0
+        else:
+            del names[:]
+            assert evaluate() == 0
+            if not any(b"k_grid" in x for x in names):
+                direct += 1
+        b.close()
+    assert st == 0 and failed > 0 and direct >= 10, (failed, direct)
+    assert evaluate() == 0 and any(b"k_grid_spread" in x for x in names)
     # and the growth of the lists
     H.hooks(launch=launch, refuse=refuse, d2h=d2h)
     want.add("cap")
     fail = True
-    assert positions() == 3
-    assert evaluate() == 1
+    st = positions()
+    assert st == 0
     fail = False
     want.clear()
+    del names[:]
+    assert evaluate() == 0
+    assert not any(b"k_grid" in x for x in names)
     assert positions() == 0
     assert evaluate() == 0
     b.close()
