@@ -1147,7 +1147,7 @@ void grid_state(mdffgpu_batch* b) {
     take(&b->d_apart, 9 * N);
     if (ok) {
       fill(b, b->d_apart, 9 * N, 0.0);
-      b->grid_calls = !b->mixed || grid::points(b->gp) * segs.size() <= GRID_POINTS;
+      b->grid_calls = !b->mixed || grid::size(b->bc_h[0].kmax, false).points * segs.size() <= GRID_POINTS;
     }
   }
   if (!ok || !grid::bin(b->gp, b->st, b->d_s4, b->d_typ, b->d_cfg, b->polmask, 0.0)) {

@@ -75,8 +75,15 @@ int sums(Plan* p, mdffgpu_ctx* ctx, hipStream_t st, const double* q, const doubl
 void adjoint_sums(Plan* p, hipStream_t st, const double* q, const double* mu, const double* g,
                   double* out);
 
-// Points of one configuration's grid.
-size_t points(const Plan* p);
+// What one configuration's grid takes with these kmax, for the choice between
+// it and the direct sums: points, tiles of the spread, flops of the
+// transforms of one call (without padding).
+struct Size {
+  size_t points;
+  int tiles;
+  double flops;
+};
+Size size(const int kmax[3], bool fp64);
 
 // Doubles that pout and ind->rpart need at most.
 size_t partials(const Plan* p);

@@ -1324,6 +1324,25 @@ bool supported(const int kmax[3]) {
   return true;
 }
 
+static int extent(int axis, const int kmax[3], bool fp64) {
+  return extent(kmax[axis], axis == 0 ? TX : TY, fp64 ? W64 : W32);
+}
+
+Size size(const int kmax[3], bool fp64) {
+  double M[3], k[3];
+  for (int a = 0; a < 3; ++a) {
+    M[a] = extent(a, kmax, fp64);
+    k[a] = kmax[a] + 1;
+  }
+  Size z;
+  z.points = (size_t)(M[0] * M[1] * M[2]);
+  z.tiles = (int)(M[0] / TX * (M[1] / TY) * (M[2] / TZ));
+  // the six folded cosine / sine products of the three axes, forward and back
+  z.flops = 4.0 * (M[0] * M[1] * M[2] * k[2] + 2.0 * M[0] * M[1] * k[1] * k[2] +
+                   2.0 * M[0] * k[0] * (2.0 * k[1] - 1.0) * k[2]);
+  return z;
+}
+
 template <typename T>
 static bool take(Plan* p, T** d, size_t count) {
   void* v = nullptr;
@@ -1432,7 +1451,7 @@ Plan* create(hipStream_t st, const std::vector<Seg>& segs, const int kmax[3], bo
   e.ng = 1;
   for (int a = 0; a < 3; ++a) {
     e.k[a] = kmax[a];
-    e.M[a] = extent(kmax[a], a == 0 ? TX : TY, fp64 ? W64 : W32);
+    e.M[a] = extent(a, kmax, fp64);
     e.nt[a] = e.M[a] / (a == 0 ? TX : TY);
     e.np[a] = (kmax[a] + 1 + 15) / 16 * 16;
     e.xp[a] = (e.M[a] / 2 + 15) / 16 * 16;
@@ -1492,7 +1511,6 @@ void set_cells(Plan* p, hipStream_t st, const std::vector<Seg>& segs) {
                                            p->d_D);
 }
 
-size_t points(const Plan* p) { return p->e.ng; }
 
 size_t partials(const Plan* p) {
   // seven energy and stress rows of k_grid_mid, two rows of the SCF

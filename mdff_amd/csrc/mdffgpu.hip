@@ -431,13 +431,34 @@ std::vector<grid::Seg> grid_segs(const mdffgpu_ctx* c) {
 
 // Whether the reciprocal sums go through the grid.  The direct sums stay
 // where there are quadrupoles (their second-order terms are not spread), in
-// the allocation-free context (its scratch is fixed) and for kmax beyond the
-// plan's extents.  There is no lower limit of size: whole evaluations with 45
-// atoms at kmax 5 take 1.12 ms with either in FP64 (launches and
-// synchronisations; 20 SCF iterations) and 0.61 against 0.67 ms in mixed
-// precision, 300 atoms at kmax 10 1.21 against 3.00 and 0.69 against 0.89 ms.
+// the allocation-free context (its scratch is fixed), for kmax beyond the
+// plan's extents, and where they are faster.  Time of a whole evaluation with
+// them over one with the grid, polarizable (12 Ewald calls) / rigid:
+// - small meshes in FP64, whose launches are fewer: kmax 2 at 3, 72, 600
+//   atoms 0.78, 0.92, 0.88 / 0.88, 0.89, 0.86, kmax 3 at 12, 72, 300 0.88,
+//   1.03, 1.04 / 0.88, 0.91, 0.92, kmax 5 0.97, 1.23, 1.25 / 0.93, 1.00, 1.01.
+// - many atoms per tile: few workgroups (18 tiles at kmax 5) then add long
+//   lists in the spread.  FP64: kmax 5 at 768, 3072, 12288 atoms 1.14, 0.76,
+//   0.40 / 1.03, 0.79, 0.56, kmax 8 at 3072, 12288, 49152 1.36, 1.03, 0.64 /
+//   1.03, 0.93, 0.65, kmax 12 at 49152 1.27 / 1.08.  Mixed: kmax 4 at 3072,
+//   12288 1.14, 0.54 / 0.93, 0.63, kmax 8 at 12288, 49152 1.21, 0.71 / 0.92,
+//   0.65, kmax 12 at 49152 1.14 / 0.93, kmax 16 at 98304 1.28 / 1.22.
+// - few atoms with a large mesh in FP64: the transforms cost the same
+//   whatever the atoms.  3, 48, 192, 768 atoms at kmax 60 1.06, 1.20, 1.54,
+//   2.10, at kmax 70 0.65, 0.72, 0.92, 1.57, at kmax 100 0.30, 0.30, 0.46;
+//   (10, 100, 100) with 48 and 768 0.92 and 1.20.  A direct call takes about
+//   130 + 1.5e-4 K + 1e-6 K N us over its launches, the transforms 14 to 20
+//   Mflop per us.
 bool grid_rule(const mdffgpu_ctx* c) {
-  return c->P.lcoulomb && c->nchunk > 0 && !c->noalloc && !c->lquad && grid::supported(c->kmax);
+  if (!c->P.lcoulomb || c->nchunk == 0 || c->noalloc || c->lquad || !grid::supported(c->kmax))
+    return false;
+  const bool fp64 = grid_fp64(c);
+  if (!fp64 && !mixed::supported(c->kmax)) return true;  // nothing to choose
+  const grid::Size z = grid::size(c->kmax, fp64);
+  const double n = c->n, K = c->nk, per_tile = n / z.tiles;
+  if (!fp64) return per_tile <= (c->linduced ? std::max(250.0, K / 20) : std::max(110.0, K / 60));
+  if (K < (c->linduced ? 150 : 700)) return false;
+  return per_tile <= K / 20 && z.flops / 20e6 <= 130 + 1.5e-4 * K + 1e-6 * K * n;
 }
 
 void build_tables(mdffgpu_ctx* c) {

@@ -90,6 +90,8 @@ float* dipole_weights(MixedState* m, int* npad);
 // Batched path: configurations with a common kmax, one segment each (cell,
 // alpha, atom range of the batch arrays; the padding is laid out here).
 MixedState* create_batch(int N, const int kmax[3], const std::vector<MxSeg>& segs);
+// Whether these sums exist for kmax.
+bool supported(const int kmax[3]);
 // Launch shape: K slices of the apply GEMM (1, 2 or 4) and atoms per
 // structure-factor split (a multiple of 128); false if rejected.
 bool valid_tuning(int app_slices, int split_atoms);

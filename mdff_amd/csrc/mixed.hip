@@ -1700,10 +1700,14 @@ bool set_active(MixedState* m, int dip0, int dip1, int fld0, int fld1) {
   return make_ranges(m);
 }
 
+// 8 N1 rows (N1 = kmax + 1 of the first axis) fit the 13 row tiles of
+// mx_rho_gemm.
+bool supported(const int kmax[3]) { return kmax[0] + 1 <= 25; }
+
 static bool sizes(MixedState* m) {
   CtxView v = view(m->ctx);
   mesh(m, v.kmax);
-  if (m->N1 > 25) return false;  // 8 N1 rows fit the 13 row tiles of mx_rho_gemm
+  if (!supported(v.kmax)) return false;
   m->N = v.n;
   m->nseg = 1;
   // whole row blocks of the apply GEMM (tables are zero past n)
@@ -1736,7 +1740,7 @@ MixedState* create_batch(int N, const int kmax[3], const std::vector<MxSeg>& seg
   std::vector<int> kseg(m->npad / 32);
   for (int z = 0; z < m->nseg; ++z)
     for (int k = segs[z].poff / 32; k < (segs[z].poff + segs[z].np) / 32; ++k) kseg[k] = z;
-  bool ok = m->N1 <= 25 && allocate(m);
+  bool ok = supported(kmax) && allocate(m);
   mx_alloc(&m->d_seg, segs.size());
   mx_alloc(&m->d_kseg, kseg.size());
   mx_alloc(&m->apart, (size_t)9 * N);

@@ -1,6 +1,7 @@
 """Reciprocal sums through the uniform grid (grid.hip) against the oracle,
 which sums every k vector: kmax from 1 (a grid of one tile, as wide as the
-kernel) over odd and unequal values to a padded last tile, atoms on the cell
+kernel; in FP64 by a batch, a single configuration takes the direct sums up
+to about kmax 2) over odd and unequal values to a padded last tile, atoms on the cell
 faces and outside the cell, a cluster (every atom in a few bins), and atoms
 moved within the list's skin since their bins were made.
 
@@ -113,7 +114,8 @@ def test_grid_batch_matches_oracle(oracle_lib):
     from mdff_amd.batch import Batch
     systems = [C.silica(n, 2 * n, seed=30 + n, rc=4.5, kmax=4, pim=True, scf_tol=1e-12,
                         pot_seed=3) for n in (16, 21, 40)]
-    for kmaxes in ([(3, 5, 4)] * 3, [(3, 5, 4), (4, 4, 4), (3, 5, 4)]):
+    for kmaxes in ([(3, 5, 4)] * 3, [(1, 1, 1)] * 3, [(2, 5, 1)] * 3,
+                   [(3, 5, 4), (4, 4, 4), (3, 5, 4)]):
         for s, k in zip(systems, kmaxes):
             s.params.kES[:] = list(k)
         b = Batch.from_systems(systems, precision=P.PREC_FP64)

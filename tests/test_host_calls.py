@@ -39,7 +39,7 @@ def test_energy_partials_of_the_grid_fit_their_buffer(host_hip):
     host_hip("""
 import ctypes, host_hip as H
 from mdff_amd import configs as C, params as P
-seen = []
+seen, grids = [], 0
 def launch(name, gx, gy, gz, args):
     if b"k_grid_midILb1E" in name:
         # EnArgs: cell (19 doubles), alpha, pout
@@ -57,9 +57,11 @@ for kmax in ((1, 1, 1), (1, 58, 58), (2, 58, 58), (1, 64, 64), (2, 80, 80), (5, 
         assert st == 0, kmax
         del seen[:]
         assert H.engforce_device(L, h, s.r) == 0
-        assert seen and all(need <= room for need, room in seen), (kmax, prec, seen)
+        assert all(need <= room for need, room in seen), (kmax, prec, seen)
         L.mdffgpu_destroy(h)
+        grids += bool(seen)
         print(kmax, prec, seen, flush=True)
+assert grids >= 15, grids  # the others take the direct sums
 """)
 
 
@@ -97,7 +99,7 @@ def test_context_after_a_refused_bin_allocation(host_hip):
     makes, and so do the next ones; nothing reads the lists."""
     host_hip(GROW + """
 for prec, direct in ((P.PREC_FP64, b"k_rho64"), (P.PREC_MIXED, b"mx_rho")):
-    s = C.silica(20, 40, seed=8, rc=4.0, kmax=3, pim=False)
+    s = C.silica(20, 40, seed=8, rc=4.0, kmax=10, pim=False)
     s.params.precision = prec
     st, h = H.create(L, s)
     assert st == 0
@@ -137,7 +139,7 @@ def refuse_nth(n, kind):
     return 1 if left[0] == 0 else 0
 H.hooks(launch=launch, refuse=refuse_nth)
 for prec, direct in ((P.PREC_FP64, b"k_rho64"), (P.PREC_MIXED, b"mx_rho")):
-    s = C.silica(20, 40, seed=8, rc=4.0, kmax=3, pim=True)
+    s = C.silica(20, 40, seed=8, rc=4.0, kmax=10, pim=True)
     s.params.precision = prec
     kept = 0
     for nth in range(1, 200):
@@ -217,4 +219,54 @@ for prec in (P.PREC_FP64, P.PREC_MIXED):
     assert positions() == 0
     assert evaluate() == 0
     b.close()
+""")
+
+
+# (kmax, atoms, polarizable): the path of the reciprocal sums on either side of
+# the lines of the rule in FP64 and in mixed precision
+ROUTES = [
+    # small meshes
+    ((2, 2, 2), 60, True, "direct", "grid"),
+    ((3, 3, 3), 60, True, "grid", "grid"),
+    # many atoms per tile
+    ((5, 5, 5), 90, True, "grid", "grid"),
+    ((5, 5, 5), 90, False, "direct", "grid"),
+    ((5, 5, 5), 3000, True, "direct", "grid"),
+    ((5, 5, 5), 3000, False, "direct", "direct"),
+    ((3, 3, 3), 1500, True, "direct", "direct"),
+    ((10, 10, 10), 648, False, "grid", "grid"),
+    ((10, 10, 10), 3000, True, "grid", "grid"),
+    ((8, 8, 8), 12288, True, "direct", "grid"),
+    ((24, 24, 24), 3000, False, "grid", "grid"),
+    # few atoms with a large mesh; mixed has no direct sums past 24
+    ((60, 60, 60), 3, False, "direct", "grid"),
+    ((60, 60, 60), 192, True, "grid", "grid"),
+    ((80, 80, 80), 192, True, "direct", "grid"),
+    ((10, 100, 100), 48, True, "direct", "grid"),
+    ((5, 80, 80), 48, True, "grid", "grid"),
+    # past the grid's extents
+    ((3, 3, 115), 90, True, "direct", "direct"),
+]
+
+
+def test_route_of_the_reciprocal_sums(host_hip):
+    host_hip(f"""
+import host_hip as H
+from mdff_amd import configs as C, params as P
+names = []
+H.hooks(launch=lambda name, gx, gy, gz, args: names.append(name))
+L = H.lib()
+for kmax, n, pim, *want in {ROUTES!r}:
+    s = C.silica(n // 3, n - n // 3, seed=8, rc=2.0 if n < 30 else 4.0, kmax=3, pim=pim)
+    s.params.kES[:] = list(kmax)
+    for prec, path in zip((P.PREC_FP64, P.PREC_MIXED), want):
+        s.params.precision = prec
+        st, h = H.create(L, s)
+        assert st == 0
+        del names[:]
+        assert H.engforce_device(L, h, s.r) == 0
+        L.mdffgpu_destroy(h)
+        grid = any(b"k_grid_spread" in x for x in names)
+        direct = any(b"k_rho64" in x or b"mx_rho" in x for x in names)
+        assert (grid, direct) == (path == "grid", path == "direct"), (kmax, n, pim, prec, path)
 """)
