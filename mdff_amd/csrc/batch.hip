@@ -1112,17 +1112,33 @@ bool common_kmax(const mdffgpu_batch* b) {
   return true;
 }
 
+// Whether the Ewald calls of a batch with a common kmax go through the grid.
+// In FP64 always: loss and gradient, 10 iterations, per-k kernels and
+// tangents against the grid, 4 configurations of 96 atoms at kmax 2
+// 1.9 against 0.9 ms, of 1536 at kmax 12 71 against 1.8 ms, 64 of 96 at
+// kmax 2 (the closest) 2.15 against 1.99.  In mixed precision the matrix-core
+// sums over every k are the other side (both with the reverse solve); of 229
+// batches (kmax 2 to 12, 1 to 100 configurations of 60 to 6000 atoms) the
+// grid takes about 0.3 ms per million points and 0.25 per 100 atoms per tile
+// of its largest configuration (the longest lists of the spread) more, the
+// sums 0.5 and 0.4 per 1e8 (atom, k).  Times grid / sums in ms: kmax 8, 16
+// and 64 configurations of 96 atoms 1.26 / 1.22 and 2.60 / 1.54, of 399
+// 1.44 / 1.66 and 3.29 / 2.47; kmax 12, 16 of 1536 2.42 / 3.11; kmax 3, one
+// of 1536 and of 6000 1.57 / 1.65 and 4.18 / 2.39.  The faster is taken to
+// 1.3 % on average, 23 % at worst.
+bool grid_rule(const mdffgpu_batch* b) {
+  if (!b->mixed) return true;
+  const int* k = b->bc_h[0].kmax;
+  const grid::Size z = grid::size(k, false);
+  const double K = 0.5 * ((2 * k[0] + 1) * (2 * k[1] + 1) * (2 * k[2] + 1) - 1);
+  int nmax = 0;
+  for (const BatchCfg& x : b->bc_h) nmax = std::max(nmax, x.n);
+  return 0.3e-6 * z.points * b->bc_h.size() + 0.25e-2 * nmax / z.tiles <= 0.5 + 0.4e-8 * b->N * K;
+}
+
 // Grid plan of a batch whose configurations share kmax, binned at the current
 // positions (set_positions: never inside a graph capture).  The reverse pass
-// always uses it.  The Ewald calls do in FP64 (loss and gradient by tangents,
-// per-k kernels against the grid: 12 configurations, 5,400 atoms, kmax 8,
-// 51.2 -> 10.4 ms, 64, 58,000 atoms, 119 -> 55 ms, 2, 400 atoms, kmax 5,
-// 13.4 -> 4.8 ms) and in mixed precision up to GRID_POINTS grid points in all,
-// beyond which the matrix-core sums over every k are as fast (they grow with
-// the atoms, the grid with the k mesh): 12 configurations of up to 800 atoms
-// 9.5 -> 6.8 ms, 32 of up to 1000 (2.5 M points) 12.4 -> 11.8, 64 of up to
-// 1536 (4.9 M points) 19.4 against 22.6 ms.
-constexpr size_t GRID_POINTS = 2500000;
+// always uses it, the Ewald calls by grid_rule.
 void grid_state(mdffgpu_batch* b) {
   if (!b->P.lcoulomb || !common_kmax(b) || b->grid_refused) return;
   const size_t N = b->N;
@@ -1147,7 +1163,7 @@ void grid_state(mdffgpu_batch* b) {
     take(&b->d_apart, 9 * N);
     if (ok) {
       fill(b, b->d_apart, 9 * N, 0.0);
-      b->grid_calls = !b->mixed || grid::size(b->bc_h[0].kmax, false).points * segs.size() <= GRID_POINTS;
+      b->grid_calls = grid_rule(b);
     }
   }
   if (!ok || !grid::bin(b->gp, b->st, b->d_s4, b->d_typ, b->d_cfg, b->polmask, 0.0)) {
@@ -1427,7 +1443,7 @@ void backward(mdffgpu_batch* b, int n_scf) {
     fill(b, b->d_out + slot, b->ntype + b->npol + 2 * b->ndamp, 0.0);
     return;
   }
-  if (b->gp && (b->grid_calls || mx_state(b))) {
+  if (b->gp && (b->grid_calls || (b->mixed && mx_state(b)))) {
     reverse<R>(b, n_scf, slot);
     return;
   }

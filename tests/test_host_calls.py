@@ -270,3 +270,42 @@ for kmax, n, pim, *want in {ROUTES!r}:
         direct = any(b"k_rho64" in x or b"mx_rho" in x for x in names)
         assert (grid, direct) == (path == "grid", path == "direct"), (kmax, n, pim, prec, path)
 """)
+
+
+def test_route_of_a_mixed_batch(host_hip):
+    """Either side of the lines of the rule of a mixed batch (atoms and number
+    of the configurations, kmax); differing kmax take the per-k kernels."""
+    host_hip("""
+import copy, ctypes, host_hip as H
+import numpy as np
+from mdff_amd import configs as C, params as P, _lib
+names, made = [], {}
+H.hooks(launch=lambda name, gx, gy, gz, args: names.append(name))
+_lib._lib = L = H.lib()
+from mdff_amd.batch import Batch
+for natm, nconf, kmax, prec, want in (
+        (96, 4, 8, P.PREC_MIXED, "grid"), (96, 64, 8, P.PREC_MIXED, "direct"),
+        (399, 16, 8, P.PREC_MIXED, "grid"), (399, 64, 8, P.PREC_MIXED, "direct"),
+        (96, 10, 12, P.PREC_MIXED, "direct"), (399, 1, 3, P.PREC_MIXED, "grid"),
+        (1800, 2, 3, P.PREC_MIXED, "direct"), (96, 64, 8, P.PREC_FP64, "grid"),
+        (1800, 2, 3, P.PREC_FP64, "grid"), (96, 2, (5, 6), P.PREC_MIXED, "per k"),
+        (96, 2, (5, 6), P.PREC_FP64, "per k")):
+    ks = kmax if isinstance(kmax, tuple) else (kmax,) * nconf
+    s0 = made.setdefault(natm, C.silica(natm // 3, natm - natm // 3, seed=8, rc=4.0, kmax=3, pim=True))
+    systems = [copy.deepcopy(s0) for k in ks]
+    for s, k in zip(systems, ks):
+        s.params.kES[:] = [k] * 3
+    b = Batch.from_systems(systems, precision=prec)
+    r = np.ascontiguousarray(np.concatenate([s.r for s in systems]).T)
+    tgt, loss, grad = np.zeros_like(r), ctypes.c_double(), np.zeros(b.nparam)
+    assert L.mdffgpu_batch_set_positions(b._h, r.ctypes.data, None) == 0
+    del names[:]
+    assert L.mdffgpu_batch_loss_grad(b._h, tgt.ctypes.data, None, ctypes.byref(loss),
+                                     grad.ctypes.data_as(H.dp), 3, None, None, None) == 0
+    # the reverse pass spreads with k_grid_spread_adj
+    got = [w for w, key in (("grid", b"13k_grid_spreadI"), ("direct", b"mx_rho"),
+                            ("per k", b"k_b_rho")) if any(key in x for x in names)]
+    assert got == [want], (natm, nconf, kmax, prec, got)
+    assert any(b"k_b_rev_dir" in x for x in names) == (want != "per k")
+    b.close()
+""")
