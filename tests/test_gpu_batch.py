@@ -207,9 +207,10 @@ def test_mixed_launch_shapes_agree_and_autotune():
     """Every launch shape of the FP32 matrix-core reciprocal sums (K slices
     of the apply, atoms per structure-factor split) gives the same loss and
     gradient to FP32 summation-order noise; the autotuner keeps one of them;
-    an FP64 batch has no such shape."""
+    an FP64 batch has no such shape.  Twelve small configurations at kmax 12
+    take these sums, not the grid."""
     from mdff_amd.batch import MIXED_CANDIDATES, Batch, autotune
-    systems = _systems(3, nmax=300, kmax=4, tol=1e-10)
+    systems = _systems(12, nmax=300, kmax=12, tol=1e-10)
     b = Batch.from_systems(systems, precision=P.PREC_MIXED)
     b.set_positions(_positions(systems))
     target = _target(b, systems)

@@ -1,6 +1,8 @@
 """The reciprocal sums and the SCF pair table cover only the atoms that need
 them: the SCF calls' moments and fields sit on the polarizable atoms, which
-the context's species-major numbering keeps contiguous.  The silica
+the context's species-major numbering keeps contiguous.  In mixed precision
+both through the grid (kmax 8) and by the matrix-core sums over every k, which
+a context takes with this many atoms at kmax 3 and 5.  The silica
 workloads have the polarizable species last; here it is the first (Si
 polarizable, O not), so that the covered range starts at atom 0 and the
 other species follows it."""
@@ -46,10 +48,18 @@ def test_first_species_polarizable_fp64_vs_oracle(oracle_lib):
     ff.close()
 
 
+def _ran(ff):
+    """Which reciprocal sums the context launched."""
+    st = ff.profile_stats()
+    return {"grid": "grid_spread" in st, "direct": "mx_apply" in st}
+
+
+@pytest.mark.parametrize("n_si,kmax,path", [(500, 8, "grid"), (500, 3, "direct"),
+                                            (1600, 5, "direct")])
 @pytest.mark.parametrize("solver", [P.SCF_JACOBI, P.SCF_PCG])
-def test_first_species_polarizable_mixed_vs_fp64(solver):
+def test_first_species_polarizable_mixed_vs_fp64(solver, n_si, kmax, path):
     from mdff_amd.field import ForceField
-    s = _si_polar(500, 1000, seed=96, rc=8.0, kmax=8)
+    s = _si_polar(n_si, 2 * n_si, seed=96, rc=8.0, kmax=kmax)
     s.params.conv_tol_ind = 1e-8
     p64 = copy.deepcopy(s.params)
     p64.precision = P.PREC_FP64
@@ -58,25 +68,27 @@ def test_first_species_polarizable_mixed_vs_fp64(solver):
     pmx.scf_solver = solver
     f64 = ForceField(p64, s.itype, s.A)
     fmx = ForceField(pmx, s.itype, s.A)
+    fmx.profile(True)
     try:
         o = f64.engforce(s.r, itime=1)
         g = fmx.engforce(s.r, itime=1)
+        assert _ran(fmx) == {"grid": path == "grid", "direct": path == "direct"}
     finally:
         f64.close()
         fmx.close()
     ef, em, eg = rel_rms(g["f"], o["f"]), rel_rms(g["mu"], o["mu"]), rel_rms(g["efg"], o["efg"])
-    print(f"Si-polarizable 1500 solver {solver}: force {ef:.2e} dipole {em:.2e} efg {eg:.2e} "
+    print(f"Si-polarizable {s.natm} kmax {kmax} solver {solver}: force {ef:.2e} dipole {em:.2e} efg {eg:.2e} "
           f"n_scf {g['n_scf']} (fp64 {o['n_scf']})", flush=True)
     assert np.abs(o["mu"][s.itype == 2]).max() == 0.0  # O carries no dipole
     assert ef <= 1e-5 and em <= 1e-5 and eg <= 1e-5, (ef, em, eg)
 
 
-@pytest.mark.parametrize("slices", [1, 4])
+@pytest.mark.parametrize("slices", [1, 2, 4])
 def test_apply_slice_counts_vs_fp64(slices):
-    """The other apply K-slice counts on the polarizable-first melt (their
-    row blocks cover the polarizable rows only), against FP64."""
+    """The apply K-slice counts on the polarizable-first melt (their row
+    blocks cover the polarizable rows only), against FP64."""
     from mdff_amd.field import ForceField
-    s = _si_polar(500, 1000, seed=97, rc=8.0, kmax=8)
+    s = _si_polar(1600, 3200, seed=97, rc=8.0, kmax=5)
     s.params.conv_tol_ind = 1e-8
     p64 = copy.deepcopy(s.params)
     p64.precision = P.PREC_FP64
@@ -84,10 +96,12 @@ def test_apply_slice_counts_vs_fp64(slices):
     pmx.precision = P.PREC_MIXED
     f64 = ForceField(p64, s.itype, s.A)
     fmx = ForceField(pmx, s.itype, s.A)
+    fmx.profile(True)
     try:
         assert fmx.set_mixed_tuning(slices, 512)
         o = f64.engforce(s.r, itime=1)
         g = fmx.engforce(s.r, itime=1)
+        assert _ran(fmx) == {"grid": False, "direct": True}
     finally:
         f64.close()
         fmx.close()
