@@ -71,6 +71,7 @@ struct mdffgpu_ctx {
   int kmax[3] = {0, 0, 0};
   int KC = 1, nchunk = 0, kpad = 0, nk = 0;
   std::vector<KChunk> chunks_h;
+  bool kmesh_ready = false;  // kmesh_tables has run for the current cell
   int rho_split = 1, rho_atoms = 1, app_split = 1, app_chunks = 1;
   // neighbour list
   int maxnb = 0;
@@ -325,9 +326,9 @@ void set_lattice(mdffgpu_ctx* c, const double* A) {
   if (!make_cell(A, c->cell, c->W)) fail(c, MDFFGPU_ERR_ARG, "cell volume is not positive");
 }
 
-// Half-space k mesh of kpoint_sum_init (src/kspace.f90:142-207) arranged
-// in chunks of KC consecutive n3; padding slots carry A_k = 0.
-void build_kmesh(mdffgpu_ctx* c) {
+// Extents of the half-space k mesh of kpoint_sum_init
+// (src/kspace.f90:142-207), arranged in chunks of KC consecutive n3.
+void kmesh_shape(mdffgpu_ctx* c) {
   const mdffgpu_params& P = c->P;
   for (int a = 0; a < 3; ++a) {
     c->kmax[a] = P.kES[a];
@@ -337,6 +338,19 @@ void build_kmesh(mdffgpu_ctx* c) {
   const int L3 = 2 * kz + 1;
   const int nch3 = (L3 + KC_MAX - 1) / KC_MAX;
   c->KC = (L3 + nch3 - 1) / nch3;
+  // row n1 = n2 = 0 holds n3 >= 1, row n1 = 0 n2 >= 0
+  const int rows = ky + kx * (2 * ky + 1);
+  c->nk = kz + rows * L3;
+  c->nchunk = (kz + c->KC - 1) / c->KC + rows * ((L3 + c->KC - 1) / c->KC);
+  c->kpad = c->nchunk * c->KC;
+}
+
+// Its tables for the direct sums; padding slots carry A_k = 0.
+void kmesh_tables(mdffgpu_ctx* c) {
+  const mdffgpu_params& P = c->P;
+  c->kmesh_ready = false;
+  if (c->nchunk == 0) return;
+  const int kx = c->kmax[0], ky = c->kmax[1], kz = c->kmax[2];
   const int KC = c->KC;
   std::vector<KChunk>& ch = c->chunks_h;
   ch.clear();
@@ -344,7 +358,6 @@ void build_kmesh(mdffgpu_ctx* c) {
   const double tpi = 2.0 * MDFF_PI;
   const double alpha2 = P.alphaES * P.alphaES;
   const double* B = c->cell.B;
-  int nk = 0;
   for (int n1 = 0; n1 <= kx; ++n1) {
     int n2min = (n1 == 0) ? 0 : -ky;
     for (int n2 = n2min; n2 <= ky; ++n2) {
@@ -370,7 +383,6 @@ void build_kmesh(mdffgpu_ctx* c) {
             kv[0].push_back(vx);
             kv[1].push_back(vy);
             kv[2].push_back(vz);
-            ++nk;
           } else {
             Ak.push_back(0.0);
             kcoe.push_back(0.0);
@@ -382,10 +394,6 @@ void build_kmesh(mdffgpu_ctx* c) {
       }
     }
   }
-  c->nk = nk;
-  c->nchunk = (int)ch.size();
-  c->kpad = c->nchunk * KC;
-  if (c->nchunk == 0) return;
   std::vector<double> kvec(3 * (size_t)c->kpad);
   for (int a = 0; a < 3; ++a)
     std::memcpy(kvec.data() + (size_t)a * c->kpad, kv[a].data(), c->kpad * sizeof(double));
@@ -412,6 +420,7 @@ void build_kmesh(mdffgpu_ctx* c) {
   dalloc(c, &c->d_apart, (size_t)c->app_split * 9 * n);
   // rows a partial call leaves alone hold finite values
   HCK(c, hipMemsetAsync(c->d_apart, 0, (size_t)c->app_split * 9 * n * sizeof(double), c->st));
+  c->kmesh_ready = true;
 }
 
 // Grid plan of the reciprocal sums in the precision they run in.
@@ -1776,16 +1785,21 @@ void prepare(mdffgpu_ctx* c, bool phases) {
   check_launch(c, "k_prepare");
 }
 
-// Without the memory for the grid (plan or bins) the context goes on with the
-// direct sums.
+// The direct sums, by the rule or without the memory for the grid (plan or
+// bins): their k mesh and, in mixed precision, the matrix-core state.
 void direct_sums(mdffgpu_ctx* c) {
   grid::destroy(c->gp);
   c->gp = nullptr;
+  if (c->P.lcoulomb && !c->kmesh_ready) kmesh_tables(c);
   if (c->P.precision != MDFFGPU_PREC_MIXED || c->mx) return;
   c->mx = mixed::create(c);
   if (!c->mx) fail(c, MDFFGPU_ERR_UNSUPPORTED, "mixed-precision path unavailable");
   mx_active(c);
 }
+
+// Whether this context reads the k mesh: the direct sums, and mdffgpu_efg of
+// a mixed one (its reciprocal space is FP64, the grid FP32).
+bool kmesh_used(const mdffgpu_ctx* c) { return c->P.lcoulomb && !(c->gp && grid_fp64(c)); }
 
 // Bins of the grid at the current positions, good for displacements up to
 // drift.
@@ -1958,7 +1972,7 @@ void run(mdffgpu_ctx* c, int itime, mdffgpu_energies* en) {
   const int gb = nblk(n);
   hipStream_t st = c->st;
   std::memset(en, 0, sizeof(*en));
-  if (!c->gp) direct_sums(c);
+  if (!c->gp) direct_sums(c);  // as a refused allocation left it
   prepare(c, P.lcoulomb && !c->gp);
   update_list(c);
   if (c->gp) grid::prepare(c->gp, c, st, c->d_s4);
@@ -2414,14 +2428,19 @@ void create_impl(const mdffgpu_params* params, const int32_t* itype, const doubl
     k_ranges(c);
     update_cutoffs(c);
     if (c->list_cut > 0.0) set_list_capacity(c, initial_capacity(c));
-    if (c->P.lcoulomb) build_kmesh(c);
+    if (c->P.lcoulomb) kmesh_shape(c);
     size_t need = 12 * (size_t)std::max(nblk(c->kpad), nblk(c->n * LPA)) + 4096;
     ensure_part(c, need);
     if (grid_rule(c)) c->gp = grid::create(c->st, grid_segs(c), c->kmax, grid_fp64(c));
-    if (c->gp)
+    if (c->gp) {
       ensure_part(c, grid::partials(c->gp));
-    else
+      dalloc(c, &c->d_apart, 9 * (size_t)c->n);
+      // rows a partial call leaves alone hold finite values
+      HCK(c, hipMemsetAsync(c->d_apart, 0, 9 * (size_t)c->n * sizeof(double), c->st));
+      if (kmesh_used(c)) kmesh_tables(c);
+    } else {
       direct_sums(c);
+    }
     // the clears of alloc_atoms are done before the context is handed out
     HCK(c, hipStreamSynchronize(c->st));
     *out = c;
@@ -2711,7 +2730,8 @@ int mdffgpu_set_cell(mdffgpu_ctx* c, const double* A) {
     c->list_valid = false;
     c->mx_floor = 0.0;
     if (c->list_cut > 0.0) set_list_capacity(c, std::max(c->maxnb, initial_capacity(c)));
-    if (c->P.lcoulomb) build_kmesh(c);
+    c->kmesh_ready = false;
+    if (kmesh_used(c)) kmesh_tables(c);
     if (c->mx) mixed::on_cell(c->mx);
     if (c->gp) {
       grid::set_cells(c->gp, c->st, grid_segs(c));

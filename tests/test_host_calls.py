@@ -72,9 +72,12 @@ GROW = """
 import ctypes, host_hip as H
 import numpy as np
 from mdff_amd import configs as C, params as P
-names, arm, fail = [], set(), False
+names, arm, fail = [], set(), lambda n: False
+mesh = []
 def launch(name, gx, gy, gz, args):
     names.append(name)
+    if b"k_rho_reduce64" in name:
+        mesh.append(H.pointer(args, 0, 24))
     if b"k_disp" in name and "disp" in want:
         arm.add("disp")
     if b"k_grid_cap" in name and "cap" in want:
@@ -87,7 +90,7 @@ def d2h(dst, n):
         arm.discard("disp")
         ctypes.memset(dst, 0x41, n)
 def refuse(n, kind):
-    return 1 if fail and kind == 0 and any(b"k_grid_cap" in x for x in names) else 0
+    return 1 if fail(n) and kind == 0 and any(b"k_grid_cap" in x for x in names) else 0
 want, GROWN = set(), 100000
 H.hooks(launch=launch, refuse=refuse, d2h=d2h)
 L = H.lib()
@@ -98,7 +101,10 @@ def test_context_after_a_refused_bin_allocation(host_hip):
     """The evaluation goes on with the direct sums, the phases of which it
     makes, and so do the next ones; nothing reads the lists."""
     host_hip(GROW + """
-for prec, direct in ((P.PREC_FP64, b"k_rho64"), (P.PREC_MIXED, b"mx_rho")):
+# the lists alone are refused, or every allocation after the bins: then the
+# first call reports it and the next one makes what the direct sums need
+for all_of_them, prec, direct in ((f, *w) for f in (False, True) for w in (
+        (P.PREC_FP64, b"k_rho64"), (P.PREC_MIXED, b"mx_rho"))):
     s = C.silica(20, 40, seed=8, rc=4.0, kmax=10, pim=False)
     s.params.precision = prec
     st, h = H.create(L, s)
@@ -107,20 +113,22 @@ for prec, direct in ((P.PREC_FP64, b"k_rho64"), (P.PREC_MIXED, b"mx_rho")):
     assert any(b"k_grid_lists" in x for x in names)
     del names[:]
     want.update(("disp", "cap"))
-    fail = True
-    # the failure of everything after the bins reaches the mixed path's own
-    # allocations too: that call reports it and the next one makes them
-    assert H.engforce_device(L, h, s.r) == (0 if prec == P.PREC_FP64 else 6)
+    del mesh[:]
+    fail = lambda n: all_of_them or n == 8 * (GROWN + GROWN // 8 + 8)
+    st = H.engforce_device(L, h, s.r)
+    assert (st != 0) == all_of_them, (prec, st)
     assert any(b"k_grid_cap" in x for x in names)
     assert not any(b"k_grid_lists" in x for x in names)
-    fail = False
+    fail = lambda n: False
     want.clear()
     for again in range(2):
-        if prec == P.PREC_MIXED or again:
+        if all_of_them or again:
             del names[:]
             assert H.engforce_device(L, h, s.r) == 0
         assert any(direct in x for x in names), names
-        if prec == P.PREC_FP64 and not again:
+        if prec == P.PREC_FP64:
+            assert mesh and all(mesh), mesh  # A_k of k_rho_reduce64
+        if not all_of_them and not again:
             bins = max(k for k, x in enumerate(names) if b"k_grid_cap" in x)
             assert any(b"k_prepare" in x for x in names[bins:])
         else:
@@ -155,6 +163,42 @@ for prec, direct in ((P.PREC_FP64, b"k_rho64"), (P.PREC_MIXED, b"mx_rho")):
         assert any(direct in x for x in names) and not any(b"k_grid" in x for x in names)
         L.mdffgpu_destroy(h)
     assert st == 0 and kept >= 10, kept
+    L.mdffgpu_destroy(h)
+""")
+
+
+def test_fp64_grid_context_makes_no_k_mesh(host_hip):
+    """Creation and set_cell neither fill nor hold the tables of the direct
+    sums (3 kpad doubles of k vectors among them); a context that takes the
+    direct sums, or a mixed one (whose EFG is summed in FP64), does."""
+    host_hip("""
+import ctypes, host_hip as H
+import numpy as np
+from mdff_amd import configs as C, params as P
+sizes = []
+def record(n, kind):
+    sizes.append(n)
+    return 0
+H.hooks(refuse=record)
+L = H.lib()
+k = 20
+chunks = -(-(2 * k + 1) // 16)
+KC = -(-(2 * k + 1) // chunks)
+kpad = (-(-k // KC) + (k + k * (2 * k + 1)) * chunks) * KC
+for prec, quad, want in ((P.PREC_FP64, 0, False), (P.PREC_FP64, 1, True), (P.PREC_MIXED, 0, True)):
+    s = C.silica(20, 40, seed=8, rc=4.0, kmax=k, pim=True)
+    s.params.precision = prec
+    s.params.task_coul_quad[0] = quad
+    del sizes[:]
+    st, h = H.create(L, s)
+    assert st == 0
+    assert L.mdffgpu_num_kvectors(h) == ((2 * k + 1) ** 3 - 1) // 2
+    assert (24 * kpad in sizes) == want, (prec, quad)
+    del sizes[:]
+    A = np.ascontiguousarray(1.01 * np.asarray(s.A).reshape(-1, order="F"))
+    assert L.mdffgpu_set_cell(h, A.ctypes.data_as(H.dp)) == 0
+    assert (24 * kpad in sizes) == want, (prec, quad)
+    assert H.engforce_device(L, h, s.r) == 0
     L.mdffgpu_destroy(h)
 """)
 
@@ -208,10 +252,9 @@ for prec in (P.PREC_FP64, P.PREC_MIXED):
     # and the growth of the lists
     H.hooks(launch=launch, refuse=refuse, d2h=d2h)
     want.add("cap")
-    fail = True
-    st = positions()
-    assert st == 0
-    fail = False
+    fail = lambda n: True
+    assert positions() == 0
+    fail = lambda n: False
     want.clear()
     del names[:]
     assert evaluate() == 0
