@@ -1882,7 +1882,7 @@ void update_list(mdffgpu_ctx* c) {
   const int n = c->n;
   const int gb = nblk(n);
   hipStream_t st = c->st;
-  bool rebuild = !c->list_valid || (c->gp && !grid::binned(c->gp));
+  bool rebuild = !c->list_valid;
   if (c->list_cut > 0.0 && !rebuild) {
     // Verlet skin (vnlistcheck, src/tools.f90:446-535): the list holds every
     // pair within cutoff + skin at the last build, so it stays complete
@@ -1899,7 +1899,12 @@ void update_list(mdffgpu_ctx* c) {
     prof_collect(c);
     rebuild = 2.0 * std::sqrt(c->h_sc[SC_DISP]) > P.skindiff;
   }
-  if (c->list_cut > 0.0 && rebuild) rebuild_list(c);
+  if (c->list_cut > 0.0 && rebuild)
+    rebuild_list(c);
+  else if (c->gp && !grid::binned(c->gp))
+    // an EFG frame put its own bins there: these positions and the later ones
+    // that the list is good for are within skin/2 of its reference
+    grid_bin(c, P.skindiff);
 }
 
 bool has_shortrange(const mdffgpu_params& P) {

@@ -184,3 +184,31 @@ def test_refused_options():
     o.lefg_old = 1
     with pytest.raises(MdffError):
         _gpu_efg(s.params, s.itype, s.A, s.r, o)
+
+
+@pytest.mark.parametrize("precision", [P.PREC_FP64, P.PREC_MIXED])
+def test_efg_and_force_calls_in_turn(oracle_lib, precision):
+    """EFG frames of rigid ions between force evaluations: each call is right
+    for its positions, to either side of the list's reference within half the
+    skin, and the neighbour list is built once."""
+    from helpers import compare_engforce
+    from mdff_amd.field import ForceField
+    s = C.silica(40, 80, seed=12, rc=5.0, kmax=10, pim=False, efg=True)
+    p = s.params
+    p.precision = precision
+    o = P.efg_opts("ewald")
+    step = np.random.default_rng(2).standard_normal(s.r.shape)
+    step *= 0.49 * p.skindiff / np.linalg.norm(step, axis=1).max()
+    orc = oracle_lib.Oracle(p, s.itype, s.A)
+    ff = ForceField(p, s.itype, s.A)
+    for k, x in enumerate((0.0, 1.0, -1.0, 0.5)):
+        r = s.r + x * step
+        g, ref = ff.engforce(r, itime=k + 1), orc.engforce(r, itime=k + 1)
+        if precision == P.PREC_FP64:
+            compare_engforce(g, ref)
+        else:
+            assert np.linalg.norm(g["f"] - ref["f"]) <= 4e-6 * np.linalg.norm(ref["f"])
+        close(ff.efg(r - 0.3 * step, o)["efg"],
+              oracle_lib.efgcalc(p, o, s.itype, s.A, r - 0.3 * step)["efg"])
+    assert ff.list_info()["builds"] == 1
+    ff.close()
