@@ -32,6 +32,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <new>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -959,6 +960,21 @@ namespace {
   va_end(ap);
   if (b) b->err = buf;
   throw BFail{code};
+}
+
+// Status of the exception being handled: none leaves a C entry point.
+int caught(mdffgpu_batch* b) {
+  try {
+    throw;
+  } catch (BFail& f) {
+    return f.code;
+  } catch (std::bad_alloc&) {
+    b->err = "host memory";
+    return MDFFGPU_ERR_ALLOC;
+  } catch (...) {
+    b->err = "unexpected host exception";
+    return MDFFGPU_ERR_DEVICE;
+  }
 }
 
 thread_local std::string g_batch_create_error;
@@ -1907,8 +1923,8 @@ int mdffgpu_batch_set_model(mdffgpu_batch* b, const mdffgpu_params* model) {
   try {
     set_model(b, *model, false);
     return MDFFGPU_OK;
-  } catch (BFail& f) {
-    return f.code;
+  } catch (...) {
+    return caught(b);
   }
 }
 
@@ -1918,8 +1934,8 @@ int mdffgpu_batch_set_positions(mdffgpu_batch* b, const double* d_pos, void* str
     if (stream) BCK(b, hipStreamSynchronize((hipStream_t)stream));
     set_positions_impl(b, d_pos);
     return MDFFGPU_OK;
-  } catch (BFail& f) {
-    return f.code;
+  } catch (...) {
+    return caught(b);
   }
 }
 
@@ -1938,8 +1954,8 @@ int mdffgpu_batch_forces(mdffgpu_batch* b, double* d_force, int32_t scf_iters,
     if (n_scf) *n_scf = ns;
     if (rmsd) *rmsd = r;
     return MDFFGPU_OK;
-  } catch (BFail& f) {
-    return f.code;
+  } catch (...) {
+    return caught(b);
   }
 }
 
@@ -2001,8 +2017,8 @@ int mdffgpu_batch_loss_grad(mdffgpu_batch* b, const double* d_target, double* d_
     if (n_scf) *n_scf = ns;
     if (rmsd) *rmsd = r;
     return MDFFGPU_OK;
-  } catch (BFail& f) {
-    return f.code;
+  } catch (...) {
+    return caught(b);
   }
 }
 

@@ -13,6 +13,7 @@
 #include <initializer_list>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -260,6 +261,21 @@ void fail(mdffgpu_ctx* c, int code, const char* fmt, ...) {
   else
     g_create_error = buf;
   throw Fail{code};
+}
+
+// Status of the exception being handled: none leaves a C entry point.
+int caught(mdffgpu_ctx* c) {
+  try {
+    throw;
+  } catch (Fail& f) {
+    return f.code;
+  } catch (std::bad_alloc&) {
+    c->err = "host memory";
+    return MDFFGPU_ERR_ALLOC;
+  } catch (...) {
+    c->err = "unexpected host exception";
+    return MDFFGPU_ERR_DEVICE;
+  }
 }
 
 void hipck(mdffgpu_ctx* c, hipError_t e, const char* what) {
@@ -2449,7 +2465,7 @@ void create_impl(const mdffgpu_params* params, const int32_t* itype, const doubl
     // the clears of alloc_atoms are done before the context is handed out
     HCK(c, hipStreamSynchronize(c->st));
     *out = c;
-  } catch (Fail&) {
+  } catch (...) {
     g_create_error = c->err;
     mdffgpu_destroy(c);
     throw;
@@ -2744,8 +2760,8 @@ int mdffgpu_set_cell(mdffgpu_ctx* c, const double* A) {
       HCK(c, hipStreamSynchronize(c->st));
     }
     return MDFFGPU_OK;
-  } catch (Fail& f) {
-    return f.code;
+  } catch (...) {
+    return caught(c);
   }
 }
 
@@ -2794,10 +2810,11 @@ int mdffgpu_engforce(mdffgpu_ctx* c, const double* rx, const double* ry, const d
       }
     if (theta_t && !th) std::memset(theta_t, 0, 9 * b);
     return MDFFGPU_OK;
-  } catch (Fail& f) {
+  } catch (...) {
+    const int code = caught(c);
     c->io_want = 0;
     (void)hipStreamSynchronize(c->st);
-    return f.code;
+    return code;
   }
 }
 
@@ -2822,10 +2839,11 @@ int mdffgpu_engforce_device(mdffgpu_ctx* c, const double* d_pos, int32_t itime,
     c->out_force = c->out_mu = c->out_ef = c->out_efg = nullptr;
     c->st = c->own_stream;
     return MDFFGPU_OK;
-  } catch (Fail& f) {
+  } catch (...) {
+    const int code = caught(c);
     c->out_force = c->out_mu = c->out_ef = c->out_efg = nullptr;
     c->st = c->own_stream;
-    return f.code;
+    return code;
   }
 }
 
@@ -3109,9 +3127,10 @@ int mdffgpu_md_run(mdffgpu_ctx* c, const mdffgpu_md_params* mp, int32_t itime0, 
     HCK(c, hipStreamSynchronize(c->st));
     c->st = c->own_stream;
     return MDFFGPU_OK;
-  } catch (Fail& f) {
+  } catch (...) {
+    const int code = caught(c);
     c->st = c->own_stream;
-    return f.code;
+    return code;
   }
 }
 
@@ -3243,9 +3262,10 @@ int mdffgpu_efg(mdffgpu_ctx* c, const mdffgpu_efg_opts* o, const double* rx, con
     std::memcpy(efg_t, c->h_io, 9 * n * sizeof(double));
     if (mu_t) std::memcpy(mu_t, c->h_io + 9 * n, 3 * n * sizeof(double));
     return MDFFGPU_OK;
-  } catch (Fail& f) {
+  } catch (...) {
+    const int code = caught(c);
     (void)hipStreamSynchronize(c->st);
-    return f.code;
+    return code;
   }
 }
 
@@ -3298,8 +3318,8 @@ int mdffgpu_get_dipole_history(mdffgpu_ctx* c, double* hist) {
     HCK(c, hipMemcpyAsync(hist, src, cnt * sizeof(double), hipMemcpyDeviceToHost, c->st));
     HCK(c, hipStreamSynchronize(c->st));
     return MDFFGPU_OK;
-  } catch (Fail& f) {
-    return f.code;
+  } catch (...) {
+    return caught(c);
   }
 }
 
@@ -3313,8 +3333,8 @@ int mdffgpu_set_dipole_history(mdffgpu_ctx* c, const double* hist) {
     if (c->renum) gather_dev(c, c->d_hist, c->d_xbuf, 3, K);
     HCK(c, hipStreamSynchronize(c->st));
     return MDFFGPU_OK;
-  } catch (Fail& f) {
-    return f.code;
+  } catch (...) {
+    return caught(c);
   }
 }
 

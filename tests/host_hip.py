@@ -67,3 +67,13 @@ def engforce_device(L, h, r, itime=1):
     en = MdffEnergies()
     return L.mdffgpu_engforce_device(h, pos.ctypes.data, itime, f.ctypes.data, None, None, None,
                                      ctypes.byref(en), None)
+
+
+def engforce(L, h, r, itime=1):
+    from mdff_amd.params import MdffEnergies
+    x = [np.ascontiguousarray(r[:, a]) for a in range(3)]
+    f = [np.zeros(len(r)) for _ in range(3)]
+    en = MdffEnergies()
+    d = lambda a: a.ctypes.data_as(dp)
+    return L.mdffgpu_engforce(h, *map(d, x), itime, *map(d, f), None, None, None, None,
+                              ctypes.byref(en))

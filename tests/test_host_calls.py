@@ -167,6 +167,46 @@ for prec, direct in ((P.PREC_FP64, b"k_rho64"), (P.PREC_MIXED, b"mx_rho")):
 """)
 
 
+def test_host_memory_failure_is_a_status(host_hip):
+    """Without pinned memory the staging of a host call falls back to ordinary
+    memory; without that too the call returns MDFFGPU_ERR_ALLOC, as do a
+    context and a batch whose tables find none, and the next call works."""
+    host_hip(GROW + """
+from mdff_amd import _lib
+_lib._lib = L
+from mdff_amd.batch import Batch
+s = C.silica(200, 400, seed=8, rc=4.0, kmax=6, pim=True)
+st, h = H.create(L, s)
+assert st == 0
+assert H.engforce_device(L, h, s.r) == 0  # the numbering is decided
+H.hooks(launch=launch, refuse=lambda n, kind: 1 if kind == 1 else 0)
+H.hip.host_hip_new_limit(6 * 600 * 8)
+assert H.engforce(L, h, s.r) == 3
+assert b"host memory" in L.mdffgpu_last_error(h)
+H.hip.host_hip_new_limit(2 ** 62)
+assert H.engforce(L, h, s.r) == 0
+H.hooks(launch=launch)
+assert H.engforce(L, h, s.r) == 0
+L.mdffgpu_destroy(h)
+s.params.task_coul_quad[0] = 1  # direct sums
+st, h = H.create(L, s)
+A = np.ascontiguousarray(np.asarray(s.A).reshape(-1, order="F"))
+H.hip.host_hip_new_limit(1024)
+assert L.mdffgpu_set_cell(h, A.ctypes.data_as(H.dp)) == 3
+H.hip.host_hip_new_limit(2 ** 62)
+assert H.engforce_device(L, h, s.r) == 0
+L.mdffgpu_destroy(h)
+s.params.task_coul_quad[0] = 0
+b = Batch.from_systems([s, s], precision=P.PREC_FP64)
+r = np.ascontiguousarray(np.concatenate([s.r, s.r]).T)
+H.hip.host_hip_new_limit(64)
+assert L.mdffgpu_batch_set_positions(b._h, r.ctypes.data, None) == 3
+H.hip.host_hip_new_limit(2 ** 62)
+assert L.mdffgpu_batch_set_positions(b._h, r.ctypes.data, None) == 0
+b.close()
+""")
+
+
 def test_fp64_grid_context_makes_no_k_mesh(host_hip):
     """Creation and set_cell neither fill nor hold the tables of the direct
     sums (3 kpad doubles of k vectors among them); a context that takes the
