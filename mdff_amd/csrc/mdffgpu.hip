@@ -477,8 +477,9 @@ std::vector<grid::Seg> grid_segs(const mdffgpu_ctx* c) {
 bool grid_rule(const mdffgpu_ctx* c) {
   if (!c->P.lcoulomb || c->nchunk == 0 || c->noalloc || c->lquad || !grid::supported(c->kmax))
     return false;
+  // a mixed context has direct sums up to kmax 24 of the first axis only
+  if (c->P.precision == MDFFGPU_PREC_MIXED && !mixed::supported(c->kmax)) return true;
   const bool fp64 = grid_fp64(c);
-  if (!fp64 && !mixed::supported(c->kmax)) return true;  // nothing to choose
   const grid::Size z = grid::size(c->kmax, fp64);
   const double n = c->n, K = c->nk, per_tile = n / z.tiles;
   if (!fp64) return per_tile <= (c->linduced ? std::max(250.0, K / 20) : std::max(110.0, K / 60));

@@ -336,11 +336,14 @@ def test_route_of_the_reciprocal_sums(host_hip):
     host_hip(f"""
 import host_hip as H
 from mdff_amd import configs as C, params as P
-names = []
+names, made = [], {{}}
 H.hooks(launch=lambda name, gx, gy, gz, args: names.append(name))
 L = H.lib()
 for kmax, n, pim, *want in {ROUTES!r}:
-    s = C.silica(n // 3, n - n // 3, seed=8, rc=2.0 if n < 30 else 4.0, kmax=3, pim=pim)
+    if (n, pim) not in made:
+        made[n, pim] = C.silica(n // 3, n - n // 3, seed=8, rc=2.0 if n < 30 else 4.0, kmax=3,
+                                pim=pim)
+    s = made[n, pim]
     s.params.kES[:] = list(kmax)
     for prec, path in zip((P.PREC_FP64, P.PREC_MIXED), want):
         s.params.precision = prec
@@ -352,6 +355,16 @@ for kmax, n, pim, *want in {ROUTES!r}:
         grid = any(b"k_grid_spread" in x for x in names)
         direct = any(b"k_rho64" in x or b"mx_rho" in x for x in names)
         assert (grid, direct) == (path == "grid", path == "direct"), (kmax, n, pim, prec, path)
+# mixed with an FP64 reciprocal space: by the FP64 lines where it has both
+for k, path in ((5, b"k_rho64"), (60, b"k_grid_spread")):
+    s = C.silica(1, 2, seed=8, rc=2.0, kmax=k, pim=False)
+    s.params.precision, s.params.mixed_fp64_parts = P.PREC_MIXED, P.MIXED_FP64_KSPACE
+    st, h = H.create(L, s)
+    assert st == 0, k
+    del names[:]
+    assert H.engforce_device(L, h, s.r) == 0
+    L.mdffgpu_destroy(h)
+    assert any(path in x for x in names), k
 """)
 
 
