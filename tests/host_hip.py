@@ -77,3 +77,14 @@ def engforce(L, h, r, itime=1):
     d = lambda a: a.ctypes.data_as(dp)
     return L.mdffgpu_engforce(h, *map(d, x), itime, *map(d, f), None, None, None, None,
                               ctypes.byref(en))
+
+
+def melt(n, pim):
+    """A silica system of n atoms at random positions (no kernel runs)."""
+    from mdff_amd import configs as C
+    s = C.silica(20, 40, seed=8, rc=4.0, kmax=3, pim=pim)
+    L = max(8.1, (13.0 * n) ** (1.0 / 3.0))
+    s.params.natm = n
+    A = L * np.eye(3)
+    itype = np.repeat([1, 2], [n // 3, n - n // 3]).astype(np.int32)
+    return C.System(s.params, itype, A, L * np.random.default_rng(n).random((n, 3)), s.name, {})

@@ -175,7 +175,8 @@ def test_host_memory_failure_is_a_status(host_hip):
 from mdff_amd import _lib
 _lib._lib = L
 from mdff_amd.batch import Batch
-s = C.silica(200, 400, seed=8, rc=4.0, kmax=6, pim=True)
+s = H.melt(600, True)
+s.params.kES[:] = [6, 6, 6]
 st, h = H.create(L, s)
 assert st == 0
 assert H.engforce_device(L, h, s.r) == 0  # the numbering is decided
@@ -335,15 +336,12 @@ ROUTES = [
 def test_route_of_the_reciprocal_sums(host_hip):
     host_hip(f"""
 import host_hip as H
-from mdff_amd import configs as C, params as P
-names, made = [], {{}}
+from mdff_amd import params as P
+names = []
 H.hooks(launch=lambda name, gx, gy, gz, args: names.append(name))
 L = H.lib()
 for kmax, n, pim, *want in {ROUTES!r}:
-    if (n, pim) not in made:
-        made[n, pim] = C.silica(n // 3, n - n // 3, seed=8, rc=2.0 if n < 30 else 4.0, kmax=3,
-                                pim=pim)
-    s = made[n, pim]
+    s = H.melt(n, pim)
     s.params.kES[:] = list(kmax)
     for prec, path in zip((P.PREC_FP64, P.PREC_MIXED), want):
         s.params.precision = prec
@@ -357,7 +355,8 @@ for kmax, n, pim, *want in {ROUTES!r}:
         assert (grid, direct) == (path == "grid", path == "direct"), (kmax, n, pim, prec, path)
 # mixed with an FP64 reciprocal space: by the FP64 lines where it has both
 for k, path in ((5, b"k_rho64"), (60, b"k_grid_spread")):
-    s = C.silica(1, 2, seed=8, rc=2.0, kmax=k, pim=False)
+    s = H.melt(3, False)
+    s.params.kES[:] = [k] * 3
     s.params.precision, s.params.mixed_fp64_parts = P.PREC_MIXED, P.MIXED_FP64_KSPACE
     st, h = H.create(L, s)
     assert st == 0, k
@@ -374,8 +373,8 @@ def test_route_of_a_mixed_batch(host_hip):
     host_hip("""
 import copy, ctypes, host_hip as H
 import numpy as np
-from mdff_amd import configs as C, params as P, _lib
-names, made = [], {}
+from mdff_amd import params as P, _lib
+names = []
 H.hooks(launch=lambda name, gx, gy, gz, args: names.append(name))
 _lib._lib = L = H.lib()
 from mdff_amd.batch import Batch
@@ -387,7 +386,7 @@ for natm, nconf, kmax, prec, want in (
         (1800, 2, 3, P.PREC_FP64, "grid"), (96, 2, (5, 6), P.PREC_MIXED, "per k"),
         (96, 2, (5, 6), P.PREC_FP64, "per k")):
     ks = kmax if isinstance(kmax, tuple) else (kmax,) * nconf
-    s0 = made.setdefault(natm, C.silica(natm // 3, natm - natm // 3, seed=8, rc=4.0, kmax=3, pim=True))
+    s0 = H.melt(natm, True)
     systems = [copy.deepcopy(s0) for k in ks]
     for s, k in zip(systems, ks):
         s.params.kES[:] = [k] * 3
