@@ -113,8 +113,9 @@ def time_path(args, sys_, precision, frames_dev, scf=None, tuning=None, table=Tr
         sl, sp = (int(x) for x in args.tuning.split(","))
         tuning = {"apply_slices": sl, "split_atoms": sp}
     elif precision == P.PREC_MIXED:
-        # launch shape of the matrix-core reciprocal sums, picked on a
-        # separate context (its dipole history is not the timed one's)
+        # launch shape of the matrix-core reciprocal sums, if this workload
+        # takes them, picked on a separate context (its dipole history is not
+        # the timed one's)
         ft = ForceField(p, sys_.itype, sys_.A)
         tuning = ft.autotune(frames_dev[0], force, itime=1, reps=2)
         ft.close()
@@ -255,13 +256,14 @@ def batch_leg(args):
     b64.set_model(set_theta(b64.model, th0))
     noise = torch.tensor(0.05 * rng.standard_normal(tuple(f_hidden.shape)), device="cuda")
     target = (f_hidden + noise).contiguous()
-    # launch shapes by the autotuner: FP32 matrix-core K slices and split
-    # size, FP64 reciprocal-apply lanes per atom
+    # launch shapes by the autotuner where the sums have one: FP32 matrix-core
+    # K slices and split size (FP64 goes through the grid)
     tune32 = autotune(b32, target, BATCH_SCF, reps=2, use_cache=False)
     tune64 = autotune(b64, target, BATCH_SCF, reps=2, use_cache=False)
     out = {"nconf": len(systems), "natm": natm, "scf_iters": BATCH_SCF,
-           "evals": args.batch_evals, "tuning": {"mixed": tune32["best"],
-                                                 "fp64": tune64["best"]}}
+           "evals": args.batch_evals,
+           "tuning": {k: t["best"] if t["ms"] else None
+                      for k, t in (("mixed", tune32), ("fp64", tune64))}}
     ref = {}
     for key, b in (("fp64", b64), ("mixed", b32)):
         loss, grad, forces = b.loss_grad(target, BATCH_SCF, want_forces=True)
@@ -492,11 +494,14 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        # the mixed path: FP32 pair and real-space arithmetic, reciprocal
-        # sums on the fp16 matrix cores with every operand split in fp16
-        # hi + lo (22-bit significands, 3 products, FP32 accumulation),
-        # FP64 reductions and SCF residual
-        "dtype": "f16x2-split mfma + f32 + f64" if "mixed" in res else "f64",
+        # the mixed path: FP32 pair and real-space arithmetic, FP64 reductions
+        # and SCF residual; reciprocal sums through a grid (FP32 spread on
+        # the matrix cores and interpolation, FP64 transforms) or, where the
+        # direct sums are the faster, on the fp16 matrix cores with every
+        # operand split in fp16 hi + lo (22-bit significands, 3 products,
+        # FP32 accumulation)
+        "dtype": ("f64" if "mixed" not in res else "f32 + f64"
+                  if "grid_spread" in head["kernels"] else "f16x2-split mfma + f32 + f64"),
         "data": "synthetic",
         "config": {
             "workload": (f"{sys_.name}: polarizable silica-like melt, {sys_.natm} atoms, "

@@ -441,11 +441,13 @@ int mdffgpu_profile_only(mdffgpu_ctx* ctx, int32_t kernel);
  * the Python autotuner): K slices of the field apply (1, 2 or 4) and atoms
  * per structure-factor split of the sums with charges (a multiple of 128;
  * the dipole-only sums of the SCF and final calls size their splits to fill
- * the device in one round).  The grid sums, which every context takes whose
- * kmax they support, have no such shape: there the arguments are checked
- * only.  MDFFGPU_ERR_UNSUPPORTED on an FP64 context.
+ * the device in one round).  The grid sums, which most contexts take, have no
+ * such shape: there the arguments are checked only (see
+ * mdffgpu_launch_shapes).  MDFFGPU_ERR_UNSUPPORTED on an FP64 context.
  * No counterpart in the reference. */
 int mdffgpu_set_mixed_tuning(mdffgpu_ctx* ctx, int32_t apply_slices, int32_t split_atoms);
+/* Whether that launch shape has an effect on this context (1 or 0). */
+int32_t mdffgpu_launch_shapes(const mdffgpu_ctx* ctx);
 int mdffgpu_profile_read(const mdffgpu_ctx* ctx, int32_t kernel,
                          double* total_ms, int64_t* launches);
 const char* mdffgpu_kernel_name(int32_t kernel);
@@ -524,13 +526,18 @@ int mdffgpu_batch_set_tuning(mdffgpu_batch* b, int32_t apply_lanes);
 
 /* Launch shape of the FP32 batch's matrix-core reciprocal sums, chosen by
    the autotuner: K slices of the field apply (1, 2 or 4) and atoms per
-   structure-factor split (a multiple of 128).  A small batch takes the grid
-   sums, which have no such shape: there the arguments are checked only.
+   structure-factor split (a multiple of 128).  A batch on the grid sums,
+   which have no such shape, checks the arguments only.
    MDFFGPU_ERR_UNSUPPORTED when the batch has no such path (FP64, or
    configurations with different kmax).
    No counterpart in the reference. */
 int mdffgpu_batch_set_mixed_tuning(mdffgpu_batch* b, int32_t apply_slices,
                                    int32_t split_atoms);
+
+/* Which launch shape has an effect at the positions last set: 0 none (the
+   grid sums), 1 mdffgpu_batch_set_tuning (the per-k kernels), 2
+   mdffgpu_batch_set_mixed_tuning (the matrix-core sums). */
+int32_t mdffgpu_batch_launch_shapes(const mdffgpu_batch* b);
 
 const char* mdffgpu_batch_last_error(const mdffgpu_batch* b);
 

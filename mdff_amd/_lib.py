@@ -45,6 +45,7 @@ PROTOTYPES = {
     "mdffgpu_profile_enable": (ctypes.c_int, [_vp, ctypes.c_int32]),
     "mdffgpu_profile_only": (ctypes.c_int, [_vp, ctypes.c_int32]),
     "mdffgpu_set_mixed_tuning": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int32]),
+    "mdffgpu_launch_shapes": (ctypes.c_int32, [_vp]),
     "mdffgpu_profile_read": (ctypes.c_int, [_vp, ctypes.c_int32, _dp,
                                             ctypes.POINTER(ctypes.c_int64)]),
     "mdffgpu_kernel_name": (ctypes.c_char_p, [ctypes.c_int32]),
@@ -63,6 +64,7 @@ PROTOTYPES = {
     "mdffgpu_batch_graph": (ctypes.c_int, [_vp, ctypes.c_int32]),
     "mdffgpu_batch_set_tuning": (ctypes.c_int, [_vp, ctypes.c_int32]),
     "mdffgpu_batch_set_mixed_tuning": (ctypes.c_int, [_vp, ctypes.c_int32, ctypes.c_int32]),
+    "mdffgpu_batch_launch_shapes": (ctypes.c_int32, [_vp]),
     "mdffgpu_batch_last_error": (ctypes.c_char_p, [_vp]),
 }
 

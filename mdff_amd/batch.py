@@ -237,6 +237,12 @@ class Batch:
         self._check(st)
         return True
 
+    def launch_shapes(self) -> int:
+        """Which launch shape has an effect at the positions last set: 0 none
+        (reciprocal sums through the grid), 1 set_tuning, 2
+        set_mixed_tuning."""
+        return int(_lib.lib().mdffgpu_batch_launch_shapes(self._h))
+
     # -- evaluation ---------------------------------------------------------
     def forces(self, scf_iters: int = 0):
         """Forces (3, natm) float64 CUDA tensor, and (n_scf, rmsd)."""
@@ -316,15 +322,20 @@ def _cache_path() -> str:
                           os.path.join(os.path.expanduser("~"), ".cache", "mdff_amd", "tune.json"))
 
 
+_SHAPES = {0: "grid", 1: "per-k", 2: "matrix-core"}
+
+
 def _key(batch: Batch, scf_iters: int) -> str:
     import torch
-    kmax = max(max(g["kmax"]) for g in batch.configs)
+    kmax = sorted({tuple(g["kmax"]) for g in batch.configs})
     return (f"{torch.cuda.get_device_name(0)}|nconf={len(batch.configs)}|natm={batch.natm}|"
-            f"kmax={kmax}|prec={batch.model.precision}|scf={scf_iters}")
+            f"kmax={kmax}|prec={batch.model.precision}|scf={scf_iters}|"
+            f"sums={_SHAPES[batch.launch_shapes()]}")
 
 
 MIXED_CANDIDATES = tuple({"apply_slices": a, "split_atoms": b}
                          for a in (1, 2, 4) for b in (512, 1024, 2048))
+DEFAULTS = ({"apply_slices": 2, "split_atoms": 2048}, {"apply_lanes": 4})
 FP64_CANDIDATES = tuple({"apply_lanes": k} for k in (2, 4, 8, 16))
 
 
@@ -342,11 +353,17 @@ def autotune(batch: Batch, target, scf_iters: int, candidates=None, reps: int = 
     matrix-core field apply and the atoms per structure-factor split, for
     the FP64 batch the lanes per atom of the reciprocal-space kernel.
     Results are cached per device and batch shape in a JSON file
-    (MDFF_TUNE_CACHE)."""
+    (MDFF_TUNE_CACHE).  A batch on the grid sums, where no launch shape has
+    an effect, keeps the default; nothing is timed or cached."""
     import torch
+    shapes = batch.launch_shapes()
     if candidates is None:
         mixed = batch.set_mixed_tuning(2, 2048)
         candidates = MIXED_CANDIDATES if mixed else FP64_CANDIDATES
+    if shapes == 0:
+        best = next((c for c in candidates if c in DEFAULTS), candidates[0])
+        _apply(batch, best)
+        return {"best": dict(best), "ms": []}
     key = _key(batch, scf_iters)
     path = _cache_path()
     cache = {}

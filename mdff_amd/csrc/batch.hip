@@ -2062,6 +2062,11 @@ int mdffgpu_batch_set_mixed_tuning(mdffgpu_batch* b, int32_t apply_slices, int32
                                                                    : MDFFGPU_ERR_ARG;
 }
 
+int32_t mdffgpu_batch_launch_shapes(const mdffgpu_batch* b) {
+  if (!b || !b->positions_set || !b->P.lcoulomb || b->grid_calls) return 0;
+  return b->mixed && b->mx ? 2 : 1;
+}
+
 const char* mdffgpu_batch_last_error(const mdffgpu_batch* b) {
   if (!b) return g_batch_create_error.c_str();
   return b->err.c_str();

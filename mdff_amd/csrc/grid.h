@@ -32,7 +32,7 @@ struct Plan;
 bool supported(const int kmax[3]);
 
 // Plan for configurations that share kmax; fp64: grid and kernel tables in
-// double (support 16), else in float (support 10; transforms in double).
+// double (support 17), else in float (support 10; transforms in double).
 // Null when device memory runs out (the caller has the direct sums).
 Plan* create(hipStream_t st, const std::vector<Seg>& segs, const int kmax[3], bool fp64);
 void destroy(Plan* p);

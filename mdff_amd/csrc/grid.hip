@@ -27,9 +27,10 @@
 //
 // Work: 2 W^3 terms per atom and O(M^3 kmax) for the transforms, against
 // O(kmax^3) per atom for the direct sum: at 24,576 atoms and kmax 24
-// (58,824 k) 1e4 against 6e5 terms per atom.  An FP64 step (17 Ewald calls)
-// went from 20.15 to 5.37 ms, a mixed one (11 calls) from 2.31 to 1.56 ms;
-// at 3000 atoms and kmax 10, 2.31 -> 1.82 and 1.36 -> 0.87 ms.
+// (58,824 k) 1e4 against 6e5 terms per atom.  Evaluations of 12 Ewald calls
+// with the direct sums and with the grid in one build, ms: 24,576 atoms at
+// kmax 20 7.79 / 2.26 FP64, 1.90 / 1.17 mixed; 3000 at kmax 24 2.53 / 0.96,
+// 1.80 / 0.80; 3072 at kmax 10 1.25 / 0.84, 1.23 / 0.65.
 //
 // Every step is a gather (a workgroup owns its tile of the grid, a wave its
 // atom) with a fixed order of summation: results are bitwise reproducible.
@@ -454,9 +455,9 @@ __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_lists(
 }
 
 // Kernel values of every atom: tab[atom][axis][phi, phi'][W] and
-// tab2[atom][axis][phi''][W], and the first points l0[atom] of its support.  One thread per (atom, axis, point); the
-// coefficients in LDS with the piece fastest, so that the lanes of an atom
-// read consecutive words.
+// tab2[atom][axis][phi''][W], and the first points l0[atom] of its support.
+// One thread per (atom, axis, point); the coefficients in LDS with the piece
+// fastest, so that the lanes of an atom read consecutive words.
 template <typename R>
 __global__ __launch_bounds__(MDFF_BLOCK) void k_grid_tab(int n, Ext e, const double4* __restrict__ s4,
                                                          const R* __restrict__ poly,
@@ -511,8 +512,9 @@ static int xcd_blocks(int n) { return (n + 7) / 8 * 8; }
 //   G = sum_j (mx phi'_x) (phi_y phi_z) + phi_x ((q phi_y + my phi'_y) phi_z + phi_y mz phi'_z).
 // The factors of 32 atoms at a time are expanded to the tile's points in LDS
 // (zero outside an atom's support), the next 32 loaded while the current
-// ones multiply; no zeroed grid and no atomics.  The tile shape makes 2.6
-// (W = 10) to 3.5 (W = 16) products per term of the support.  Where the grid
+// ones multiply; no zeroed grid and no atomics.  The tile shape makes
+// (W + 15)(W + 7)^2 / W^3 products per term of the support: 3.7 at W = 17,
+// 7.2 at W = 10.  Where the grid
 // has few tiles, gridDim.z (one or two) blocks share a tile's atoms and write partial
 // grids, which the forward transform adds.
 constexpr int SCH = 32;  // atoms per LDS chunk
@@ -1114,11 +1116,11 @@ __device__ __forceinline__ R wave_total(R x) {
 // (their rows padded with their own beginning, so that a group never wraps):
 // consecutive waves take atoms in bin order, which share most of their
 // support in the caches.  16,384 atoms on 96^3 points: 13 us at W = 10, 59 us
-// at W = 17, the latter bound by the lines it takes through L2 (a support's
-// row of 136 bytes spans two or three; the same with one to five passes'
-// loads in flight).  With the region of a tile staged in LDS 15 and 52 us,
-// but 12 us instead of 5 for 2,000 atoms on 48^3 (few workgroups, each first
-// waiting for its region).
+// at W = 17, the latter bound by the lines it takes through L2 (9.5 M requests,
+// 2.0 per row of 136 bytes, 97 % hits; the same with one to five passes'
+// loads in flight).  With the region of a tile staged in LDS 15 and 52 us
+// (the FP64 SCF instance 61 against 62), but 12 us instead of 5 for 2,000
+// atoms on 48^3 (few workgroups, each first waiting for its region).
 //
 // IND (an SCF field of one configuration, no surface term): the field of
 // k_combine64<ES_IND> is formed here too, with the block partials of its

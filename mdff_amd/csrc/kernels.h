@@ -24,7 +24,7 @@ constexpr int TASK_QUAD_ANY = TASK_QQUAD | TASK_DQUAD | TASK_QUADQ;
 enum KernelId {
   K_PREPARE, K_NLIST, K_SR, K_DIR_STATIC, K_DIR_IND, K_DIR_FINAL, K_RHO_CHG, K_RHO_DIP,
   K_RHO_BOTH, K_RHO_RED, K_APPLY_F, K_APPLY_EFG, K_MOMENTS, K_COMBINE, K_INDUCED,
-  K_RESID, K_EXTRAP, K_REDUCE, K_ADD, K_PAIRS_T2, K_DD_FIELD, K_MX_SR, K_MX_DIR, K_MX_PHASE, K_MX_RHO,
+  K_RESID, K_EXTRAP, K_REDUCE, K_ADD, K_DD_TABLE, K_DD_TAB, K_MX_SR, K_MX_DIR, K_MX_PHASE, K_MX_RHO,
   K_MX_RHO_RED, K_MX_APPLY, K_MX_COMBINE, K_MX_WEIGHTS, K_MX_GPREP, K_BATCH, K_ADJ,
   K_EFG_DIR, K_EFG_DS, K_EFG_COMBINE, K_MD, K_QUAD, K_WFC, K_GRID_PREP, K_GRID_SPREAD, K_GRID_FT,
   K_GRID_GATHER, K_COUNT

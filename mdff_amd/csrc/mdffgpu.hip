@@ -215,7 +215,7 @@ const char* const kKernelNames[K_COUNT] = {
     "k_prepare", "k_nlist", "k_shortrange", "k_es_dir<static>", "k_es_dir<ind>",
     "k_es_dir<final>", "k_rho64<chg>", "k_rho64<dip>", "k_rho64<chg+dip>", "k_rho_reduce64",
     "k_apply64<field>", "k_apply64<efg>", "k_moments", "k_combine64", "k_induced",
-    "k_scf_resid", "k_extrap", "k_reduce_rows", "k_add", "k_pairs_t2", "k_dd_field",
+    "k_scf_resid", "k_extrap", "k_reduce_rows", "k_add", "k_dd_table", "k_dd_tab",
     "mx_shortrange", "mx_es_dir",
     "mx_phase", "mx_rho", "mx_rho_reduce", "mx_apply", "mx_combine", "mx_weights", "mx_gprep",
     "batch", "adjoint", "k_efg_es_dir", "k_efg_ds", "k_efg_combine", "md", "k_es_quad", "k_wfc",
@@ -722,7 +722,7 @@ void es_ind_dir(mdffgpu_ctx* c, const double* mu, bool packed = false) {
   const int n = c->n;
   hipStream_t st = c->st;
   const int gb = nblk(n);
-  ProfScope _ps(c, K_DD_FIELD);
+  ProfScope _ps(c, K_DD_TAB);
   if (scf_field_fp32(c)) {
     float4* m4 = reinterpret_cast<float4*>(c->d_mu4);
     const size_t cap = (size_t)c->maxnb * n;
@@ -744,7 +744,7 @@ void es_ind_dir(mdffgpu_ctx* c, const double* mu, bool packed = false) {
                     nullptr, nullptr, c->d_perm, all ? nullptr : c->d_polrows,
                     all ? n : c->npolrows, c->d_efdir);
   }
-  check_launch(c, "k_dd_field");
+  check_launch(c, "k_dd_tab");
 }
 
 // One Ewald call; with dir_done (ES_IND only) the real-space part has
@@ -1101,7 +1101,7 @@ void build_t2(mdffgpu_ctx* c) {
   }
   c->t2_in_static = mx && !(c->P.mixed_fp64_parts & MDFFGPU_MIXED_FP64_DIRECT);
   if (c->t2_in_static) return;
-  ProfScope _ps(c, K_PAIRS_T2);
+  ProfScope _ps(c, K_DD_TABLE);
   if (mx) {
     int* tj = dd_tj(c);
     k_dd_table<false, float><<<nblk(n * 64), MDFF_BLOCK, 0, c->st>>>(da, c->polmask, dd_tab(c), tj,
@@ -3354,6 +3354,8 @@ int mdffgpu_set_mixed_tuning(mdffgpu_ctx* c, int32_t apply_slices, int32_t split
   if (hipStreamSynchronize(c->st) != hipSuccess) return MDFFGPU_ERR_DEVICE;
   return mixed::set_tuning(c->mx, apply_slices, split_atoms) ? MDFFGPU_OK : MDFFGPU_ERR_ARG;
 }
+
+int32_t mdffgpu_launch_shapes(const mdffgpu_ctx* c) { return c && c->mx && c->P.lcoulomb ? 1 : 0; }
 
 int mdffgpu_profile_enable(mdffgpu_ctx* c, int32_t on) {
   if (!c) return MDFFGPU_ERR_ARG;

@@ -205,12 +205,14 @@ class ForceField:
         """Times engforce_device on one frame for every mixed-path launch
         shape (apply K slices x structure-factor split size) and keeps the
         fastest.  Each timed call is an evaluation of that frame (dipole
-        history included), so tune a context that is not mid-trajectory."""
+        history included), so tune a context that is not mid-trajectory.
+        {} where no launch shape has an effect (FP64, or reciprocal sums
+        through the grid): nothing is timed."""
         import torch
+        if not _lib.lib().mdffgpu_launch_shapes(self._h):
+            return {}
         if candidates is None:
             candidates = [(a, b) for a in (1, 2, 4) for b in (512, 1024, 2048)]
-        if not self.set_mixed_tuning(*candidates[0]):
-            return {}
         times = []
         for cand in candidates:
             self.set_mixed_tuning(*cand)

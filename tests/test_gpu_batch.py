@@ -203,6 +203,26 @@ def test_mixed_batch_against_fp64():
     b32.close()
 
 
+def test_autotune_only_where_a_shape_has_an_effect(tmp_path, monkeypatch):
+    """A grid batch is not timed and leaves no cache entry for the batch of
+    the same size whose kmax differ (per-k kernels), which is."""
+    import os
+    from mdff_amd.batch import Batch, autotune
+    monkeypatch.setenv("MDFF_TUNE_CACHE", str(tmp_path / "tune.json"))
+    systems = _systems(2, nmax=120, kmax=4, tol=1e-8)
+    for kmax, shapes in (((4, 4), 0), ((4, 3), 1)):
+        for s, k in zip(systems, kmax):
+            s.params.kES[:] = [k] * 3
+        b = Batch.from_systems(systems, precision=P.PREC_FP64)
+        b.set_positions(_positions(systems))
+        assert b.launch_shapes() == shapes
+        rec = autotune(b, _target(b, systems), 5, reps=1)
+        assert len(rec["ms"]) == (4 if shapes else 0)
+        assert os.path.exists(tmp_path / "tune.json") == bool(shapes)
+        assert autotune(b, _target(b, systems), 5, reps=1) == rec
+        b.close()
+
+
 def test_mixed_launch_shapes_agree_and_autotune():
     """Every launch shape of the FP32 matrix-core reciprocal sums (K slices
     of the apply, atoms per structure-factor split) gives the same loss and
@@ -223,7 +243,9 @@ def test_mixed_launch_shapes_agree_and_autotune():
             continue
         assert abs(loss - ref[0]) <= 1e-6 * abs(ref[0]), (slices, split)
         assert np.allclose(grad, ref[1], rtol=1e-4, atol=1e-6 * np.max(np.abs(ref[1])))
+    assert b.launch_shapes() == 2
     rec = autotune(b, target, 20, reps=1, use_cache=False)
+    assert len(rec["ms"]) == len(MIXED_CANDIDATES)
     assert rec["best"] in [dict(c) for c in MIXED_CANDIDATES]
     b.close()
     b64 = Batch.from_systems(systems, precision=P.PREC_FP64)
