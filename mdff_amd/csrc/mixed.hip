@@ -1042,11 +1042,12 @@ __global__ __launch_bounds__(MDFF_BLOCK) void mx_rho_reduce(
 // Scale of apply column (w, n1): values of w(n) g(n1, n) are at most
 // APPLY_SCALE after multiplying by APPLY_SCALE 2^-e; gmaxbits = max |g| over
 // the n1 plane, wmax = largest |w| (1, kmax2, kmax3, ...).  A power of two
-// keeps the scaling exact.
+// keeps the scaling exact.  Planes below 2^-112 (Gaussian factors of large k
+// that underflow) keep the scale of that value, which FP32 still holds.
 __device__ __forceinline__ float class_scale(unsigned int gmaxbits, float wmax) {
   const float gm = __uint_as_float(gmaxbits) * wmax;
   if (!(gm > 0.f)) return APPLY_SCALE;
-  return exp2f(-ceilf(log2f(gm))) * APPLY_SCALE;
+  return exp2f(fminf(-ceilf(log2f(gm)), 112.f)) * APPLY_SCALE;
 }
 
 // weights of the apply: 0 -> 1, 1 -> n2, 2 -> n3, 3 -> n2^2, 4 -> n2 n3,

@@ -108,3 +108,28 @@ def test_apply_slice_counts_vs_fp64(slices):
     ef, eg = rel_rms(g["f"], o["f"]), rel_rms(g["efg"], o["efg"])
     print(f"apply slices {slices}: force {ef:.2e} efg {eg:.2e}", flush=True)
     assert ef <= 1e-5 and eg <= 1e-5, (ef, eg)
+
+
+@pytest.mark.parametrize("falloff", [60.0, 72.0, 80.0, 88.0, 95.0, 102.0])
+def test_planes_whose_ewald_factors_underflow(falloff):
+    """Matrix-core sums with an alpha at which the factors exp(-k^2 / 4 alpha^2)
+    of the last n1 plane fall to exp(-falloff), through the smallest FP32
+    values and past them: the plane's FP32 scale stays finite, and the forces
+    are those of FP64."""
+    from mdff_amd.field import ForceField
+    s = _si_polar(500, 1000, seed=96, rc=8.0, kmax=3)
+    p = s.params
+    p.ldip_polar[0] = 0
+    for k in range(len(p.poldip)):
+        p.poldip[k] = 0.0
+    p.alphaES = 3 * 2.0 * np.pi / s.A[0, 0] / (2.0 * np.sqrt(falloff))
+    out = []
+    for prec in (P.PREC_FP64, P.PREC_MIXED):
+        p.precision = prec
+        ff = ForceField(p, s.itype, s.A)
+        ff.profile(True)
+        out.append(ff.engforce(s.r, itime=1))
+        assert not _ran(ff)["grid"]
+        ff.close()
+    e = rel_rms(out[1]["f"], out[0]["f"])
+    assert e <= 1e-5, e
