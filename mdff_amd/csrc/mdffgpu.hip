@@ -2165,6 +2165,7 @@ void efg_frame(mdffgpu_ctx* c, const mdffgpu_efg_opts& o, mdffgpu_energies* en) 
   const bool ewald = (o.longrange == 0);
   ++c->evals;
   if (!c->gp) direct_sums(c);
+  if (ewald && kmesh_used(c) && !c->kmesh_ready) kmesh_tables(c);
   prepare(c, !(c->gp && grid_fp64(c)));
   // get_moments (src/field.f90:3686-3765) with calc = 'efg': the SCF starts
   // from the static field, no extrapolation
@@ -2753,13 +2754,14 @@ int mdffgpu_set_cell(mdffgpu_ctx* c, const double* A) {
     c->mx_floor = 0.0;
     if (c->list_cut > 0.0) set_list_capacity(c, std::max(c->maxnb, initial_capacity(c)));
     c->kmesh_ready = false;
-    if (kmesh_used(c)) kmesh_tables(c);
-    if (c->mx) mixed::on_cell(c->mx);
     if (c->gp) {
       grid::set_cells(c->gp, c->st, grid_segs(c));
       // a later call may run on the caller's stream
       HCK(c, hipStreamSynchronize(c->st));
     }
+    // after the plan: if this is refused the next call that reads it retries
+    if (kmesh_used(c)) kmesh_tables(c);
+    if (c->mx) mixed::on_cell(c->mx);
     return MDFFGPU_OK;
   } catch (...) {
     return caught(c);

@@ -88,3 +88,13 @@ def melt(n, pim):
     A = L * np.eye(3)
     itype = np.repeat([1, 2], [n // 3, n - n // 3]).astype(np.int32)
     return C.System(s.params, itype, A, L * np.random.default_rng(n).random((n, 3)), s.name, {})
+
+
+def efg(L, h, r):
+    from mdff_amd import params as P
+    x = [np.ascontiguousarray(r[:, a]) for a in range(3)]
+    out = np.zeros(9 * len(r))
+    en = P.MdffEnergies()
+    d = lambda a: a.ctypes.data_as(dp)
+    return L.mdffgpu_efg(h, ctypes.byref(P.efg_opts("ewald")), *map(d, x), None, d(out),
+                         ctypes.byref(en))

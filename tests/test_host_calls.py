@@ -167,6 +167,36 @@ for prec, direct in ((P.PREC_FP64, b"k_rho64"), (P.PREC_MIXED, b"mx_rho")):
 """)
 
 
+def test_set_cell_without_memory_for_the_k_mesh(host_hip):
+    """set_cell of a mixed grid context whose k mesh is refused reports it; the
+    plan has the new cell, and the next EFG call makes the tables it reads."""
+    host_hip(GROW + """
+s = H.melt(60, False)
+s.params.kES[:] = [6, 6, 6]
+s.params.precision = P.PREC_MIXED
+st, h = H.create(L, s)
+assert st == 0
+A = np.ascontiguousarray(1.01 * np.asarray(s.A).reshape(-1, order="F"))
+for which in (1, 2, 3, 4):  # chunks, A_k and the rest in turn
+    left = [which]
+    def refuse_nth(n, kind):
+        if kind == 0 and names and b"k_grid_factors" in names[-1]:
+            left[0] -= 1
+            return 1 if left[0] == 0 else 0
+        return 0
+    H.hooks(launch=launch, refuse=refuse_nth)
+    del names[:], mesh[:]
+    assert L.mdffgpu_set_cell(h, A.ctypes.data_as(H.dp)) == 3
+    assert any(b"k_grid_factors" in x for x in names)
+    H.hooks(launch=launch)
+    assert H.engforce_device(L, h, s.r) == 0
+    assert any(b"k_grid_spread" in x for x in names) and not mesh
+    assert H.efg(L, h, s.r) == 0, L.mdffgpu_last_error(h)
+    assert mesh and all(mesh), mesh
+L.mdffgpu_destroy(h)
+""")
+
+
 def test_host_memory_failure_is_a_status(host_hip):
     """Without pinned memory the staging of a host call falls back to ordinary
     memory; without that too the call returns MDFFGPU_ERR_ALLOC, as do a
